@@ -684,7 +684,7 @@ def main():
         "step_mfma_frac": step_tflops / PEAK_BF16_TFLOPS,
         "grad_norm": norm,
         "roofline": {
-            "kernel": "eth_gemm (gemm256_m16/m32 and gemm_kernel instantiations: every GEMM launch of a step)",
+            "kernel": "eth_gemm (gemm256_m16/m32 and gemm_ring instantiations: every GEMM launch of a step)",
             "bound": "mfma",
             "achieved": gemm["achieved_tflops"],
             "peak": PEAK_BF16_TFLOPS,

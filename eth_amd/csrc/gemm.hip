@@ -1,5 +1,5 @@
 // bf16/fp16 GEMM on CDNA4 matrix cores (v_mfma_f32_32x32x16_{bf16,f16}),
-// fp32 accumulation, LDS-staged double-buffered tiles.
+// fp32 accumulation, operands staged through LDS by direct loads.
 //
 //   C[m, n] (+)= alpha * sum_k A(m, k) * B(k, n)  (+ bias[n])
 //
@@ -10,10 +10,6 @@
 //   dgrad    dX = dY W      : A K-contiguous, B N-contiguous
 //   wgrad    dW += dY^T X   : A M-contiguous, B N-contiguous, fp32 C += (the
 //                             Megatron main_grad accumulation, fused)
-// In the fallback kernel, M-contiguous / N-contiguous operands are
-// transposed in registers on their way into LDS (4 k-rows x 8 columns per
-// thread), so every LDS tile is stored K-contiguous and each MFMA operand is
-// one 16-byte LDS read.
 //
 // Kernels:
 //  * gemm256_m16_kernel / gemm256_m32_kernel, the main ones: 256x256x64
@@ -31,10 +27,11 @@
 //    the forward, data-gradient and weight-gradient products (for the last,
 //    both operands row-contiguous, through asm MFMAs); m32
 //    (v_mfma_f32_32x32x16) a row-contiguous A with a K-contiguous B.  Both
-//    need K % 128 == 0, 16-byte aligned C rows and enough tiles to fill
-//    the chip.
-//  * gemm_kernel, the general fallback: 256x256 (8 waves) or 128x128 (4
-//    waves) tiles, register-staged double buffering, any K % 8 == 0.
+//    need K % 128 == 0 and 16-byte aligned C rows.
+//  * gemm_ring_kernel: 128x128 or 64x64 tiles with four LDS stages, for the
+//    grids that 256x256 tiles leave mostly idle and for every shape and
+//    alignment (any K % 8 == 0).
+// plan_tile() chooses among them by the time each would take.
 // Tiles are assigned XCD-aware (consecutive workgroups land on different
 // XCDs, so the tile id is remapped to give each XCD a contiguous range) and
 // in GROUP_M-row groups so neighbouring workgroups share A and B tiles in L2.
@@ -42,6 +39,7 @@
 // Replaces the F.linear / cuBLAS calls of mpu/layers.py:357-370,452-470 and
 // the main_grad.add_ hook of model/distributed.py:116-123.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -65,14 +63,9 @@ __device__ __forceinline__ f32x16_t mfma32(const uint4& a, const uint4& b, const
   }
 }
 
-constexpr int kPad = 8;  // LDS row padding (elements): 16 B breaks bank aliasing
-
-// Workgroup barrier ordering LDS only.  __syncthreads also fences global
-// memory, which makes every wave wait for its outstanding stores.
-__device__ __forceinline__ void lds_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-// The same after this wave's direct global->LDS loads have landed.
+// Workgroup barrier after this wave's LDS accesses and direct global->LDS
+// loads have completed.  (__syncthreads also fences global memory, which
+// makes every wave wait for its outstanding stores.)
 __device__ __forceinline__ void dma_barrier() {
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
@@ -111,203 +104,6 @@ constexpr int32_t kOob = (int32_t)0x80000000u;
 __device__ __forceinline__ rsrc_t make_rsrc(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
-__device__ __forceinline__ uint4 buf_load16(rsrc_t r, int32_t voff, int32_t soff) {
-  auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-  return __builtin_bit_cast(uint4, v);
-}
-
-// ROWS x BK tile of a K-contiguous operand (row r at P[(r0+r)*ld + k]):
-// CPT 16-byte chunks per thread.
-template <int ROWS, int BK, int NT>
-struct KTile {
-  static constexpr int CPR = BK / 8;
-  static constexpr int CPT = ROWS * CPR / NT;
-  static_assert(CPT >= 1 && ROWS * CPR % NT == 0, "tile split");
-  uint4 v[CPT];
-  int32_t off[CPT];
-  __device__ __forceinline__ void init(int64_t ld, int r0, int rows) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = threadIdx.x + i * NT;
-      const int r = c / CPR, kc = (c % CPR) * 8;
-      off[i] = r0 + r < rows ? (int32_t)((((int64_t)(r0 + r)) * ld + kc) * 2) : kOob;
-    }
-  }
-  __device__ __forceinline__ void load(rsrc_t rs, int64_t ld, int k0, int K, bool kfull) {
-    const int32_t soff = k0 * 2;
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      int32_t o = off[i];
-      if (!kfull && k0 + ((threadIdx.x + i * NT) % CPR) * 8 >= K) o = kOob;
-      v[i] = buf_load16(rs, o, soff);
-    }
-  }
-  __device__ __forceinline__ void store(uint16_t* S) const {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = threadIdx.x + i * NT;
-      const int r = c / CPR, kc = (c % CPR) * 8;
-      *reinterpret_cast<uint4*>(S + r * (BK + kPad) + kc) = v[i];
-    }
-  }
-  // whole-tile load when K % BK == 0 (an empty resource reads zeros)
-  __device__ __forceinline__ void fetch(rsrc_t rs, int64_t, int k0) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) v[i] = buf_load16(rs, off[i], k0 * 2);
-  }
-  // part P of NP: store the staged chunks to LDS, then refill the same
-  // registers with k-tile k0
-  template <int P, int NP>
-  __device__ __forceinline__ void cycle(uint16_t* S, rsrc_t rs, int64_t, int k0) {
-#pragma unroll
-    for (int i = P * CPT / NP; i < (P + 1) * CPT / NP; ++i) {
-      const int c = threadIdx.x + i * NT;
-      const int r = c / CPR, kc = (c % CPR) * 8;
-      *reinterpret_cast<uint4*>(S + r * (BK + kPad) + kc) = v[i];
-      v[i] = buf_load16(rs, off[i], k0 * 2);
-    }
-  }
-};
-
-// BK x ROWS tile of an operand contiguous along the row index (element
-// (r, k) at P[k*ld + r0 + r]): each thread reads 4 k-rows of 8 consecutive
-// r and writes them transposed (8 rows of 4 k) into LDS.  The k-group index
-// varies fastest across lanes, so the 8-byte LDS writes of a wavefront
-// spread over all banks (rows 8 apart would alias otherwise).
-template <int ROWS, int BK, int NT>
-struct RTile {
-  static constexpr int RG = ROWS / 8, KG = BK / 4;
-  static constexpr int BPT = RG * KG / NT;
-  static_assert(BPT >= 1 && RG * KG % NT == 0, "tile split");
-  uint4 v[BPT][4];
-  int32_t off[BPT];
-  __device__ __forceinline__ void init(int64_t ld, int r0, int rows) {
-#pragma unroll
-    for (int b = 0; b < BPT; ++b) {
-      const int blk = threadIdx.x + b * NT;
-      const int kg = blk % KG, rg = blk / KG;
-      const int r = r0 + rg * 8;
-      off[b] = r < rows ? (int32_t)((((int64_t)kg * 4) * ld + r) * 2) : kOob;
-    }
-  }
-  __device__ __forceinline__ void load(rsrc_t rs, int64_t ld, int k0, int K, bool kfull) {
-    const int32_t soff = (int32_t)((int64_t)k0 * ld * 2);
-    const int32_t row_bytes = (int32_t)(ld * 2);
-#pragma unroll
-    for (int b = 0; b < BPT; ++b) {
-      const int kg = (threadIdx.x + b * NT) % KG;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        int32_t o = off[b] == kOob ? kOob : off[b] + j * row_bytes;
-        if (!kfull && k0 + kg * 4 + j >= K) o = kOob;
-        v[b][j] = buf_load16(rs, o, soff);
-      }
-    }
-  }
-  __device__ __forceinline__ void store(uint16_t* S) const {
-#pragma unroll
-    for (int b = 0; b < BPT; ++b) store_block(S, b);
-  }
-  __device__ __forceinline__ void fetch(rsrc_t rs, int64_t ld, int k0) {
-    const int32_t soff = (int32_t)((int64_t)k0 * ld * 2);
-    const int32_t row_bytes = (int32_t)(ld * 2);
-#pragma unroll
-    for (int b = 0; b < BPT; ++b)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[b][j] = buf_load16(rs, off[b] == kOob ? kOob : off[b] + j * row_bytes, soff);
-  }
-  template <int P, int NP>
-  __device__ __forceinline__ void cycle(uint16_t* S, rsrc_t rs, int64_t ld, int k0) {
-    const int32_t soff = (int32_t)((int64_t)k0 * ld * 2);
-    const int32_t row_bytes = (int32_t)(ld * 2);
-#pragma unroll
-    for (int b = P * BPT / NP; b < (P + 1) * BPT / NP; ++b) {
-      store_block(S, b);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[b][j] = buf_load16(rs, off[b] == kOob ? kOob : off[b] + j * row_bytes, soff);
-    }
-  }
-  __device__ __forceinline__ void store_block(uint16_t* S, int b) const {
-    const int blk = threadIdx.x + b * NT;
-    const int kg = blk % KG, rg = blk / KG;
-    const uint32_t* w0 = reinterpret_cast<const uint32_t*>(&v[b][0]);
-    const uint32_t* w1 = reinterpret_cast<const uint32_t*>(&v[b][1]);
-    const uint32_t* w2 = reinterpret_cast<const uint32_t*>(&v[b][2]);
-    const uint32_t* w3 = reinterpret_cast<const uint32_t*>(&v[b][3]);
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      // rows 2p and 2p+1 of the 8-row group
-      const uint32_t a0 = w0[p], a1 = w1[p], a2 = w2[p], a3 = w3[p];
-      uint2 lo, hi;
-      lo.x = (a0 & 0xffffu) | (a1 << 16);
-      lo.y = (a2 & 0xffffu) | (a3 << 16);
-      hi.x = (a0 >> 16) | (a1 & 0xffff0000u);
-      hi.y = (a2 >> 16) | (a3 & 0xffff0000u);
-      uint16_t* row = S + (rg * 8 + 2 * p) * (BK + kPad) + kg * 4;
-      *reinterpret_cast<uint2*>(row) = lo;
-      *reinterpret_cast<uint2*>(row + (BK + kPad)) = hi;
-    }
-  }
-};
-
-template <int ROWS, int BK, int NT, bool KCONTIG>
-struct TileLoader;
-template <int ROWS, int BK, int NT>
-struct TileLoader<ROWS, BK, NT, true> : KTile<ROWS, BK, NT> {};
-template <int ROWS, int BK, int NT>
-struct TileLoader<ROWS, BK, NT, false> : RTile<ROWS, BK, NT> {};
-
-// BK x ROWS tile of an operand contiguous along the row index (element
-// (r, k) at P[k*ld + r0 + r]), copied as it is into LDS [BK][ROWS + 32]:
-// whole 512-byte k-rows per 32 lanes from global memory, 16-byte LDS
-// writes, and ds_read_b64_tr_b16 transposes on the way out (tr_frag).  The
-// 32-element pad puts the four k-rows one transposing read touches in
-// disjoint bank ranges.
-template <int ROWS, int BK, int NT>
-struct MTile {
-  static constexpr int CPR = ROWS / 8;  // 16-byte chunks per k-row
-  static constexpr int CPT = BK * CPR / NT;
-  static constexpr int LROW = ROWS + 32;
-  static_assert(CPT >= 1 && BK * CPR % NT == 0, "tile split");
-  u32x4_t v[CPT];
-  int32_t off[CPT];
-  __device__ __forceinline__ void init(int64_t ld, int r0, int rows) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = threadIdx.x + i * NT;
-      const int k = c / CPR, r = (c % CPR) * 8;
-      off[i] = r0 + r < rows ? (int32_t)(((int64_t)k * ld + r0 + r) * 2) : kOob;
-    }
-  }
-  __device__ __forceinline__ void fetch(rsrc_t rs, int64_t ld, int k0) {
-    const int32_t soff = (int32_t)((int64_t)k0 * ld * 2);
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) v[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, off[i], soff, 0);
-  }
-  __device__ __forceinline__ void store(uint16_t* S) const {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = threadIdx.x + i * NT;
-      *reinterpret_cast<u32x4_t*>(S + (c / CPR) * LROW + (c % CPR) * 8) = v[i];
-    }
-  }
-  template <int P, int NP>
-  __device__ __forceinline__ void cycle(uint16_t* S, rsrc_t rs, int64_t ld, int k0) {
-    const int32_t soff = (int32_t)((int64_t)k0 * ld * 2);
-#pragma unroll
-    for (int i = P * CPT / NP; i < (P + 1) * CPT / NP; ++i) {
-      const int c = threadIdx.x + i * NT;
-      *reinterpret_cast<u32x4_t*>(S + (c / CPR) * LROW + (c % CPR) * 8) = v[i];
-      v[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, off[i], soff, 0);
-    }
-  }
-};
-template <int ROWS, int BK, int NT, bool KCONTIG>
-struct Tile256;
-template <int ROWS, int BK, int NT>
-struct Tile256<ROWS, BK, NT, true> : KTile<ROWS, BK, NT> {};
-template <int ROWS, int BK, int NT>
-struct Tile256<ROWS, BK, NT, false> : MTile<ROWS, BK, NT> {};
 
 // Tile moved by direct global->LDS loads (buffer_load_dwordx4 ... lds):
 // lane i of an instruction writes its 16 bytes at the wave's LDS base +
@@ -392,119 +188,10 @@ struct GemmArgs {
   int flags;
   float alpha;
   uint32_t c_bytes;  // extent of C (the gemm256 kernels' store range)
+  bool c_vec;        // C rows take 4-column vector accesses
   int k_split;              // split-K: k extent per split (0: one split of K)
   int64_t c_split_stride;   // split-K: elements between the splits' C slices
 };
-
-template <int BM, int BN, int BK, int WAVES_M, int WAVES_N, bool A_K, bool B_K, bool FP16>
-__global__ void __launch_bounds__(64 * WAVES_M * WAVES_N) gemm_kernel(GemmArgs g) {
-  constexpr int NT = 64 * WAVES_M * WAVES_N;
-  constexpr int WM = BM / WAVES_M, WN = BN / WAVES_N;
-  constexpr int TM = WM / 32, TN = WN / 32;
-  constexpr int LDS_ROW = BK + kPad;
-  __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * LDS_ROW];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BN * LDS_ROW];
-
-  const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
-  int tm, tn;
-  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int wm = wid / WAVES_N, wn = wid % WAVES_N;
-  const int lr = lane & 31, lk = (lane >> 5) * 8;
-
-  f32x16_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  const int nk = (g.K + BK - 1) / BK;
-  // MFMA over one LDS stage; operand fragments of k-step ks+1 are read from
-  // LDS while the MFMAs of k-step ks run
-  auto compute = [&](int st) {
-    const uint16_t* as = As[st] + (wm * WM + lr) * LDS_ROW + lk;
-    const uint16_t* bs = Bs[st] + (wn * WN + lr) * LDS_ROW + lk;
-    uint4 af[2][TM], bfr[2][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) af[0][i] = *reinterpret_cast<const uint4*>(as + i * 32 * LDS_ROW);
-#pragma unroll
-    for (int j = 0; j < TN; ++j) bfr[0][j] = *reinterpret_cast<const uint4*>(bs + j * 32 * LDS_ROW);
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-      const int cur = ks & 1, nxt = cur ^ 1;
-      if (ks + 1 < BK / 16) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-          af[nxt][i] = *reinterpret_cast<const uint4*>(as + i * 32 * LDS_ROW + (ks + 1) * 16);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          bfr[nxt][j] = *reinterpret_cast<const uint4*>(bs + j * 32 * LDS_ROW + (ks + 1) * 16);
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = mfma32<FP16>(af[cur][i], bfr[cur][j], acc[i][j]);
-    }
-  };
-
-  const rsrc_t ra = make_rsrc(g.A, g.a_bytes), rb = make_rsrc(g.B, g.b_bytes);
-  const bool kfull = g.K % BK == 0;
-  TileLoader<BM, BK, NT, A_K> la;
-  TileLoader<BN, BK, NT, B_K> lb;
-  la.init(g.lda, m0, g.M);
-  lb.init(g.ldb, n0, g.N);
-  la.load(ra, g.lda, 0, g.K, kfull);
-  lb.load(rb, g.ldb, 0, g.K, kfull);
-  la.store(As[0]);
-  lb.store(Bs[0]);
-  __syncthreads();
-  for (int kt = 0; kt < nk; ++kt) {
-    const int st = kt & 1;
-    const bool more = kt + 1 < nk;
-    if (more) {
-      la.load(ra, g.lda, (kt + 1) * BK, g.K, kfull);
-      lb.load(rb, g.ldb, (kt + 1) * BK, g.K, kfull);
-    }
-    compute(st);
-    if (more) {
-      la.store(As[st ^ 1]);
-      lb.store(Bs[st ^ 1]);
-    }
-    __syncthreads();
-  }
-
-  // epilogue: lane holds column n = lane%32 and rows (r/4)*8 + (lane/32)*4 + r%4
-  const bool accumulate = g.flags & ETH_GEMM_ACCUMULATE;
-  const bool has_bias = (g.flags & ETH_GEMM_BIAS) && g.bias;
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = n0 + wn * WN + j * 32 + lr;
-    if (n >= g.N) continue;
-    float bn = 0.f;
-    if (has_bias) bn = FP16 ? h2f_bits(g.bias[n]) : bf2f(g.bias[n]);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int m = m0 + wm * WM + i * 32 + (r >> 2) * 8 + (lane >> 5) * 4 + (r & 3);
-        if (m >= g.M) continue;
-        const float v = acc[i][j][r] * g.alpha + bn;
-        const int64_t off = (int64_t)m * g.ldc + n;
-        if (g.c_dtype == ETH_F32) {
-          float* c = reinterpret_cast<float*>(g.C) + off;
-          *c = accumulate ? *c + v : v;
-        } else if (g.c_dtype == ETH_BF16) {
-          reinterpret_cast<uint16_t*>(g.C)[off] = f2bf(v);
-        } else {
-          reinterpret_cast<uint16_t*>(g.C)[off] = f2h_bits(v);
-        }
-      }
-    }
-  }
-}
 
 // 256x256x64 tiles, 4 waves of 128x128 (one per SIMD), K % 128 == 0.
 //
@@ -542,6 +229,21 @@ __device__ __forceinline__ void mfma16_asm(f32x4_t& c, const uint4& a, const uin
   else
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
                  : "+a"(c)
+                 : "v"(__builtin_bit_cast(u32x4_t, a)), "v"(__builtin_bit_cast(u32x4_t, b)));
+}
+
+// The same with the accumulator tied to its VGPRs: for the kernels whose
+// accumulators fit there (through the builtin, the allocator rotates them
+// through copies around the loop's back edge).
+template <bool FP16>
+__device__ __forceinline__ void mfma16_tied(f32x4_t& c, const uint4& a, const uint4& b) {
+  if constexpr (FP16)
+    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0"
+                 : "+v"(c)
+                 : "v"(__builtin_bit_cast(u32x4_t, a)), "v"(__builtin_bit_cast(u32x4_t, b)));
+  else
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0"
+                 : "+v"(c)
                  : "v"(__builtin_bit_cast(u32x4_t, a)), "v"(__builtin_bit_cast(u32x4_t, b)));
 }
 
@@ -1080,6 +782,290 @@ __global__ void __launch_bounds__(256, 1) gemm256_m32_kernel(GemmArgs g) {
 #undef STAGE_SLAB
 }
 
+// TILE x TILE x 64 tiles (128 or 64) on 4 waves in a 2 x 2 grid, four LDS
+// stages filled by direct loads up to four k-tiles ahead.  With one or two
+// small tiles per CU no other workgroup hides the load latency, so the ring
+// does; per k-tile one barrier, set between the two k-steps:
+//   k-step 0: the MFMAs of the fragments already in registers run while the
+//             fragments of k-step 1 are read;
+//   barrier:  this k-tile's LDS reads are done in every wave (its stage is
+//             free) and the next k-tile has landed;
+//   k-step 1: its MFMAs run while the first fragments of the next k-tile are
+//             read, and k-tile t + 4 streams into the freed stage.
+// LDS images carry no padding: K-contiguous operands as in DTile,
+// row-contiguous ones [64][ROWS] with 16-byte chunk c of k-row k at
+// c ^ rc_swizzle(k), so the four k-rows (eight, for two 16-lane groups) that a
+// transposing read touches lie in distinct banks.  Any K % 8 == 0 (the last
+// k-tile's missing chunks read zeros through an out-of-range offset), any M, N
+// and C alignment.  Bound by LDS and L2: a 128x128 k-tile writes 32 KB to LDS
+// and reads 64 KB (768 cycles at 128 B/clk) for 512 MFMA cycles, and takes
+// about 1000; a 64x64 one has half the work per byte.  The register-staged
+// double-buffered tiles it replaced took 57 us for [1024, 1024] x 4096 deep
+// (now 17), 33 us for [2048, 2048] x 2048 (24), 139 us for the 8192-deep data
+// gradient of the same output (80).
+template <int ROWS>
+__device__ __forceinline__ int rc_swizzle(int k) {
+  return ROWS == 128 ? ((k & 3) << 1) | (((k >> 3) & 1) << 3) : (((k >> 1) & 1) << 1) | (((k >> 3) & 1) << 2);
+}
+template <int ROWS, bool KC>
+struct RingTile {
+  static constexpr int UPR = KC ? 8 : ROWS / 8;  // 16-byte units per LDS row
+  static constexpr int PER_WAVE = ROWS * 8 / 256;
+  static constexpr int IMG = ROWS * 64;
+  int32_t off[PER_WAVE];
+  int kof[PER_WAVE];  // k of the lane's unit within the k-tile
+  int wave;
+  __device__ __forceinline__ void init(int64_t ld, int r0, int rows) {
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < PER_WAVE; ++j) {
+      const int u = (wave * PER_WAVE + j) * 64 + lane;
+      const int line = u / UPR, c = u % UPR;
+      const int r = KC ? line : (c ^ rc_swizzle<ROWS>(line)) * 8;
+      kof[j] = KC ? (c ^ kc_swizzle(line)) * 8 : line;
+      off[j] = r0 + r < rows ? (int32_t)((KC ? (int64_t)(r0 + r) * ld + kof[j] : (int64_t)kof[j] * ld + r0 + r) * 2)
+                             : kOob;
+    }
+  }
+  // k-tile [k0, k0 + 64) into the image at S; k at or past kend reads zeros
+  // (one compare and select per load, and no second path)
+  __device__ __forceinline__ void issue(uint16_t* S, rsrc_t rs, int64_t ld, int k0, int kend) {
+    const int32_t soff = k0 < kend ? (KC ? k0 * 2 : (int32_t)((int64_t)k0 * ld * 2)) : 0;
+    const int left = kend - k0;
+#pragma unroll
+    for (int j = 0; j < PER_WAVE; ++j)
+      dma16(rs, S + (wave * PER_WAVE + j) * 512, kof[j] < left ? off[j] : kOob, soff);
+  }
+};
+
+template <int TILE, bool A_K, bool B_K, bool FP16>
+__global__ void __launch_bounds__(256, 1) gemm_ring_kernel(GemmArgs g) {
+  constexpr int BM = TILE, BN = TILE;
+  constexpr int WM = BM / 2, WN = BN / 2;    // a wave's block
+  constexpr int TI = WM / 16, TJ = WN / 16;  // of 16 x 16 MFMA blocks
+  typedef RingTile<BM, A_K> ATile;
+  typedef RingTile<BN, B_K> BTile;
+  constexpr int A_IMG = ATile::IMG, STAGE = A_IMG + BTile::IMG;
+  constexpr int PPW = ATile::PER_WAVE + BTile::PER_WAVE;  // direct loads of a wave per k-tile
+  constexpr int ER = WN + 4;                              // epilogue staging row (fp32, padded)
+  static_assert(4 * 16 * ER * 4 <= 2 * STAGE, "the epilogue's staging fits a stage");
+  // separate arrays, so the compiler can tell the direct loads into one
+  // stage from the fragment reads of another
+  __shared__ __attribute__((aligned(16))) uint16_t st0[STAGE];
+  __shared__ __attribute__((aligned(16))) uint16_t st1[STAGE];
+  __shared__ __attribute__((aligned(16))) uint16_t st2[STAGE];
+  __shared__ __attribute__((aligned(16))) uint16_t st3[STAGE];
+
+  const int tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
+  int tm, tn;
+  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int wm = wid >> 1, wn = wid & 1;
+  const int l16 = lane & 15, lg = lane >> 4;
+  const int nk = (g.K + 63) / 64;
+
+  const rsrc_t ra = make_rsrc(g.A, g.a_bytes), rb = make_rsrc(g.B, g.b_bytes);
+  ATile la;
+  BTile lb;
+  la.init(g.lda, m0, g.M);
+  lb.init(g.ldb, n0, g.N);
+#define RING_ISSUE(S, KT)                              \
+  {                                                    \
+    la.issue(S, ra, g.lda, (KT) * 64, g.K);            \
+    lb.issue((S) + A_IMG, rb, g.ldb, (KT) * 64, g.K);  \
+  }
+  RING_ISSUE(st0, 0)
+  RING_ISSUE(st1, 1)
+  RING_ISSUE(st2, 2)
+  RING_ISSUE(st3, 3)
+
+  f32x4_t acc[TI][TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+#pragma unroll
+    for (int j = 0; j < TJ; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // lane offsets of the fragments of k-step 0 (k-step 1: see frag): lane l
+  // holds row l%16 of the block, k 8*(l/16) .. +7
+  int aof[TI], bof[TJ];
+#pragma unroll
+  for (int i = 0; i < TI; ++i)
+    aof[i] = A_K ? (wm * WM + i * 16 + l16) * 64 + ((lg ^ kc_swizzle(l16)) * 8)
+                 : (8 * lg + (l16 >> 2)) * BM +
+                       ((((wm * WM + i * 16) >> 3) + ((l16 & 3) >> 1)) ^ rc_swizzle<BM>(8 * lg + (l16 >> 2))) * 8 +
+                       (l16 & 1) * 4;
+#pragma unroll
+  for (int j = 0; j < TJ; ++j)
+    bof[j] = A_IMG + (B_K ? (wn * WN + j * 16 + l16) * 64 + ((lg ^ kc_swizzle(l16)) * 8)
+                          : (8 * lg + (l16 >> 2)) * BN +
+                                ((((wn * WN + j * 16) >> 3) + ((l16 & 3) >> 1)) ^
+                                 rc_swizzle<BN>(8 * lg + (l16 >> 2))) * 8 +
+                                (l16 & 1) * 4);
+  uint4 fa[2][TI], fb[2][TJ];
+  // k-step 1: chunk 4 + lg is chunk lg with bit 2 flipped (K-contiguous);
+  // 32 k-rows further, where rc_swizzle repeats (row-contiguous)
+  auto read = [&](auto ks_c, const uint16_t* S) __attribute__((always_inline)) {
+    constexpr int ks = decltype(ks_c)::value;
+#pragma unroll
+    for (int i = 0; i < TI; ++i)
+      fa[ks][i] = A_K ? *reinterpret_cast<const uint4*>(S + (aof[i] ^ (ks * 32)))
+                      : tr_frag(S + aof[i] + ks * 32 * BM, BM);
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+      fb[ks][j] = B_K ? *reinterpret_cast<const uint4*>(S + (bof[j] ^ (ks * 32)))
+                      : tr_frag(S + bof[j] + ks * 32 * BN, BN);
+  };
+  // column blocks [J0, J1) of k-step ks
+  auto products = [&](auto ks_c, const int J0, const int J1) __attribute__((always_inline)) {
+    constexpr int ks = decltype(ks_c)::value;
+#pragma unroll
+    for (int j = J0; j < J1; ++j)
+#pragma unroll
+      for (int i = 0; i < TI; ++i) mfma16_tied<FP16>(acc[i][j], fb[ks][j], fa[ks][i]);
+  };
+  typedef std::integral_constant<int, 0> K0;
+  typedef std::integral_constant<int, 1> K1;
+  dma_barrier_but<3 * PPW>();
+  read(K0{}, st0);
+  __builtin_amdgcn_sched_barrier(0);
+#define RING_STEP(S, SN, KT)                \
+  {                                         \
+    products(K0{}, 0, 1);                   \
+    __builtin_amdgcn_sched_barrier(0);      \
+    read(K1{}, S);                          \
+    products(K0{}, 1, TJ);                  \
+    __builtin_amdgcn_sched_barrier(0);      \
+    dma_barrier_but<2 * PPW>();             \
+    RING_ISSUE(S, (KT) + 4)                 \
+    __builtin_amdgcn_sched_barrier(0);      \
+    read(K0{}, SN);                         \
+    products(K1{}, 0, TJ);                  \
+    __builtin_amdgcn_sched_barrier(0);      \
+  }
+  int kt = 0;
+  for (; kt + 4 <= nk; kt += 4) {
+    RING_STEP(st0, st1, kt)
+    RING_STEP(st1, st2, kt + 1)
+    RING_STEP(st2, st3, kt + 2)
+    RING_STEP(st3, st0, kt + 3)
+  }
+  if (kt < nk) RING_STEP(st0, st1, kt)
+  if (kt + 1 < nk) RING_STEP(st1, st2, kt + 1)
+  if (kt + 2 < nk) RING_STEP(st2, st3, kt + 2)
+  // asm MFMAs: wait states before any instruction reads their accumulators
+  asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+#undef RING_STEP
+#undef RING_ISSUE
+  dma_barrier();  // every load landed, every wave done with the stages
+
+  // Epilogue: 16-row slabs of the wave's block through its own LDS region,
+  // out in whole rows of WN columns
+  float* stage = reinterpret_cast<float*>(st0) + wid * 16 * ER;
+  constexpr int LPR = WN / 4, RPI = 64 / LPR;  // lanes per row (4 columns each), rows per pass
+  const int col = (lane % LPR) * 4, n = n0 + wn * WN + col;
+  const bool has_bias = (g.flags & ETH_GEMM_BIAS) && g.bias;
+  const bool add = g.flags & ETH_GEMM_ACCUMULATE;
+  float bn[4] = {0.f, 0.f, 0.f, 0.f};
+  if (has_bias) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < g.N) bn[e] = FP16 ? h2f_bits(g.bias[n + e]) : bf2f(g.bias[n + e]);
+  }
+#pragma unroll
+  for (int i = 0; i < TI; ++i) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the last slab's reads
+#pragma unroll
+    for (int j = 0; j < TJ; ++j)
+      *reinterpret_cast<f32x4_t*>(stage + l16 * ER + j * 16 + lg * 4) = acc[i][j];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // private to this wave
+#pragma unroll
+    for (int p = 0; p < 16 / RPI; ++p) {
+      const int r = p * RPI + lane / LPR, m = m0 + wm * WM + i * 16 + r;
+      f32x4_t v = *reinterpret_cast<const f32x4_t*>(stage + r * ER + col);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = v[e] * g.alpha + bn[e];
+      if (m >= g.M || n >= g.N) continue;
+      const int64_t o = (int64_t)m * g.ldc + n;
+      if (g.c_vec) {
+        if (g.c_dtype == ETH_F32) {
+          f32x4_t* c = reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(g.C) + o);
+          *c = add ? *c + v : v;
+        } else {
+          u32x2_t w;
+          if (g.c_dtype == ETH_BF16) {
+            w.x = f2bf_pair(v[0], v[1]);
+            w.y = f2bf_pair(v[2], v[3]);
+          } else {
+            w.x = f2h_bits(v[0]) | ((uint32_t)f2h_bits(v[1]) << 16);
+            w.y = f2h_bits(v[2]) | ((uint32_t)f2h_bits(v[3]) << 16);
+          }
+          *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(g.C) + o) = w;
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if (n + e >= g.N) break;
+          if (g.c_dtype == ETH_F32) {
+            float* c = reinterpret_cast<float*>(g.C) + o + e;
+            *c = add ? *c + v[e] : v[e];
+          } else {
+            reinterpret_cast<uint16_t*>(g.C)[o + e] = g.c_dtype == ETH_BF16 ? f2bf(v[e]) : f2h_bits(v[e]);
+          }
+        }
+      }
+    }
+  }
+}
+
+template <int TILE, bool FP16>
+static int launch_ring(const GemmArgs& a, int a_k, int b_k, hipStream_t s) {
+  const int tiles = ((a.M + TILE - 1) / TILE) * ((a.N + TILE - 1) / TILE);
+  if (a_k && b_k)
+    gemm_ring_kernel<TILE, true, true, FP16><<<tiles, 256, 0, s>>>(a);
+  else if (a_k && !b_k)
+    gemm_ring_kernel<TILE, true, false, FP16><<<tiles, 256, 0, s>>>(a);
+  else if (!a_k && !b_k)
+    gemm_ring_kernel<TILE, false, false, FP16><<<tiles, 256, 0, s>>>(a);
+  else
+    gemm_ring_kernel<TILE, false, true, FP16><<<tiles, 256, 0, s>>>(a);
+  ETH_CHECK_LAUNCH("eth_gemm");
+  return ETH_OK;
+}
+
+// Microseconds one launch of TILE x TILE tiles takes, fitted to sweeps of
+// transformer-layer products from 256^3 to [3000, 2560] x [10240, 2560] (bf16,
+// all three layouts; within about 15 %): rounds of one workgroup per CU (two
+// for 64x64, whose 64 KB of LDS leaves room for a second) times the k-tiles of
+// 64 at the measured pace plus the prologue and epilogue.  A 256x256 k-tile
+// runs faster when half the CUs idle (more clock and bandwidth for the rest).
+static double tile_time(int tile, int64_t M, int64_t N, int64_t K, int splits) {
+  const double tiles = (double)((M + tile - 1) / tile) * (double)((N + tile - 1) / tile) * splits;
+  const double nk = (double)(((K + splits - 1) / splits + 63) / 64);
+  if (tile == 256) return 3.0 + ceil(tiles / 256) * (nk * (tiles > 128 ? 1.20 : 0.93) + 9.0);
+  if (tile == 128) return 2.0 + ceil(tiles / 256) * (nk * 0.52 + 6.0);
+  return tiles <= 256 ? 2.0 + nk * 0.24 + 1.0 : 1.0 + ceil(tiles / 512) * (nk * 0.36 + 2.7);
+}
+
+// The tile that finishes first.  Measured on both sides of the lines (us, 256
+// / 128 / 64): [2048, 2048] x 2048 deep 39 / 24 / 29, [2048, 6144] x 2048 45 /
+// 66 / 76, [1024, 1024] x 4096 69 / 37 / 17, [1024, 4096] x 1024 24 / 16 / 18,
+// [3000, 2560] x 2560 48 / 53 / 66.
+static int plan_tile(int64_t M, int64_t N, int64_t K, bool wide) {
+  int best = 64;
+  double t = tile_time(64, M, N, K, 1);
+  for (int tile : {128, 256}) {
+    if (tile == 256 && !wide) continue;
+    const double u = tile_time(tile, M, N, K, 1);
+    if (u <= t) {
+      t = u;
+      best = tile;
+    }
+  }
+  return best;
+}
+
 template <bool FP16>
 static int launch_256(const GemmArgs& a, int a_k, int b_k, hipStream_t s, int splits = 1) {
   const int tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256) * splits;
@@ -1091,22 +1077,6 @@ static int launch_256(const GemmArgs& a, int a_k, int b_k, hipStream_t s, int sp
     gemm256_m16_kernel<false, false, FP16><<<tiles, 256, 0, s>>>(a);
   else
     gemm256_m32_kernel<false, true, FP16><<<tiles, 256, 0, s>>>(a);
-  ETH_CHECK_LAUNCH("eth_gemm");
-  return ETH_OK;
-}
-
-template <int BM, int BN, int BK, int WMW, int WNW, bool FP16>
-static int launch_layout(const GemmArgs& a, int a_k, int b_k, hipStream_t s) {
-  const int tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
-  constexpr int NT = 64 * WMW * WNW;
-  if (a_k && b_k)
-    gemm_kernel<BM, BN, BK, WMW, WNW, true, true, FP16><<<tiles, NT, 0, s>>>(a);
-  else if (a_k && !b_k)
-    gemm_kernel<BM, BN, BK, WMW, WNW, true, false, FP16><<<tiles, NT, 0, s>>>(a);
-  else if (!a_k && !b_k)
-    gemm_kernel<BM, BN, BK, WMW, WNW, false, false, FP16><<<tiles, NT, 0, s>>>(a);
-  else
-    gemm_kernel<BM, BN, BK, WMW, WNW, false, true, FP16><<<tiles, NT, 0, s>>>(a);
   ETH_CHECK_LAUNCH("eth_gemm");
   return ETH_OK;
 }
@@ -1154,29 +1124,27 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
   a.flags = flags;
   a.alpha = alpha;
   hipStream_t s = (hipStream_t)stream;
-  const int64_t big_tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  // the pipelined 256x256 kernel: K in whole k-tile pairs, C rows 16-byte
-  // aligned (vector stores), C extent plus one tile of rows below 2 GiB (its
-  // buffer offsets), and at least half a wave of tiles per chip
+  // the 256x256 kernels: K in whole k-tile pairs, C rows 16-byte aligned
+  // (vector stores), C extent plus one tile of rows below 2 GiB (its buffer
+  // offsets)
   const int esz = c_dtype == ETH_F32 ? 4 : 2;
   const int64_t c_extent = ((M - 1) * ldc + N) * esz;
-  const bool c_vec = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C % (4 * esz)) == 0;
+  a.c_vec = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C % (4 * esz)) == 0;
   a.k_split = 0;
   a.c_split_stride = 0;
-  if (K % 128 == 0 && c_vec && big_tiles >= 128 && c_extent + 256 * ldc * esz < (1LL << 31)) {
-    a.c_bytes = (uint32_t)c_extent;
-    return in_dtype == ETH_BF16 ? launch_256<false>(a, a_kcontig, b_kcontig, s)
-                                : launch_256<true>(a, a_kcontig, b_kcontig, s);
+  const bool wide = K % 128 == 0 && a.c_vec && c_extent + 256 * ldc * esz < (1LL << 31);
+  a.c_bytes = wide ? (uint32_t)c_extent : 0;
+  const bool fp16 = in_dtype == ETH_F16;
+  switch (plan_tile(M, N, K, wide)) {
+    case 256:
+      return fp16 ? launch_256<true>(a, a_kcontig, b_kcontig, s) : launch_256<false>(a, a_kcontig, b_kcontig, s);
+    case 128:
+      return fp16 ? launch_ring<128, true>(a, a_kcontig, b_kcontig, s)
+                  : launch_ring<128, false>(a, a_kcontig, b_kcontig, s);
+    default:
+      return fp16 ? launch_ring<64, true>(a, a_kcontig, b_kcontig, s)
+                  : launch_ring<64, false>(a, a_kcontig, b_kcontig, s);
   }
-  a.c_bytes = 0;
-  // otherwise 256x256 tiles (8 waves of 128x64) when the grid still fills
-  // the chip, 128x128 (4 waves of 64x64) below that
-  const bool big = big_tiles >= 192;
-  if (in_dtype == ETH_BF16)
-    return big ? launch_layout<256, 256, 64, 2, 4, false>(a, a_kcontig, b_kcontig, s)
-               : launch_layout<128, 128, 64, 2, 2, false>(a, a_kcontig, b_kcontig, s);
-  return big ? launch_layout<256, 256, 64, 2, 4, true>(a, a_kcontig, b_kcontig, s)
-             : launch_layout<128, 128, 64, 2, 2, true>(a, a_kcontig, b_kcontig, s);
 }
 
 namespace eth {
@@ -1210,6 +1178,14 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ W, int splits, in
 
 extern "C" int64_t eth_gemm_splitk_workspace(int64_t M, int64_t N, int splits) {
   return splits > 0 && M > 0 && N > 0 ? (int64_t)splits * M * N * 4 : 0;
+}
+
+extern "C" int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits) {
+  if (M <= 0 || N <= 0 || K <= 0 || splits < 2) return 0;
+  // the second kernel: a launch, and the partials and C at about 4.5 TB/s
+  const double sum = 5.0 + 4.0 * (double)M * (double)N * (splits + 1) / 4.5e6;
+  const double one = tile_time(plan_tile(M, N, K, K % 128 == 0), M, N, K, 1);
+  return tile_time(256, M, N, K, splits) + sum < one;
 }
 
 extern "C" int eth_gemm_splitk(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,

@@ -6,6 +6,7 @@ the current stream.  There is no CPU fallback: CPU tensors raise.
 """
 
 import ctypes
+import functools
 
 import numpy as np
 
@@ -82,6 +83,14 @@ def _splitk_splits(M, N, K, out):
     return splits
 
 
+@functools.lru_cache(maxsize=4096)
+def _splitk_pays(M, N, K, splits):
+    """Whether the split-K form finishes before the plain product (sizes
+    only; the smaller tiles fill the chip without a second pass unless K is
+    deep)."""
+    return splits > 1 and bool(nat.value("eth_gemm_splitk_pays", M, N, K, splits))
+
+
 _scratch = {}
 
 
@@ -146,7 +155,7 @@ def gemm(a, b, out=None, bias=None, accumulate=False, out_dtype=None, alpha=1.0)
     _observe("gemm", "begin", 2.0 * M * N * K)
     fp32_product = out.dtype == torch.float32 and alpha == 1.0 and bias is None
     splits = _splitk_splits(M, N, K, out) if fp32_product else 1
-    if splits > 1:
+    if _splitk_pays(M, N, K, splits):
         ws = _scratch_f32(nat.value("eth_gemm_splitk_workspace", M, N, splits) // 4, a.device)
         nat.call(
             "eth_gemm_splitk",

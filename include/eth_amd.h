@@ -248,6 +248,9 @@ int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t l
  * Same reference seam as eth_gemm's ETH_GEMM_ACCUMULATE form
  * (model/distributed.py:116-123 over mpu/layers.py:452-470). */
 int64_t eth_gemm_splitk_workspace(int64_t M, int64_t N, int splits);
+/* 1 where eth_gemm_splitk with `splits` is expected to finish before
+ * eth_gemm on the same [M, N] x K product, else 0. */
+int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits);
 int eth_gemm_splitk(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,
                     float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int in_dtype, int splits,
                     int accumulate, float* workspace, void* stream);

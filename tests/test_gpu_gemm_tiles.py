@@ -1,0 +1,73 @@
+"""GPU: the products of every tile size at the edges of tiles, k-tiles and
+ring trips, against fp64.
+
+The bound is elementwise: products of 16-bit operands are exact in fp32, each
+of the K fp32 additions rounds by at most 2^-24 of a partial sum no larger
+than sum |a||b| (doubled for the order inside an MFMA), and the result rounds
+once to its dtype (2^-9 of a bf16 value, 2^-12 of an fp16 one, with fp16's
+subnormal spacing as a floor)."""
+
+import pytest
+import torch
+
+from eth_amd import kernels as K
+from tests.conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+LAYOUTS = [(True, True), (True, False), (False, False), (False, True)]
+
+
+def _operands(M, N, Kd, a_k, b_k, dtype, cuda, seed):
+    gen = torch.Generator().manual_seed(seed)
+    a = torch.randn(M, Kd, generator=gen).to(dtype)
+    b = (torch.randn(Kd, N, generator=gen) * 0.1).to(dtype)
+    ad = a.to(cuda) if a_k else a.t().contiguous().to(cuda).t()
+    bd = b.t().contiguous().to(cuda).t() if b_k else b.to(cuda)
+    return a.double(), b.double(), ad, bd
+
+
+def _check(got, ref, mag, Kd, out_dtype, what):
+    unit = {torch.float32: 2.0**-23, torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11}[out_dtype]
+    bound = 2 * Kd * 2.0**-24 * mag + unit * ref.abs() + 2.0**-24
+    err = (got.cpu().double() - ref).abs()
+    assert bool((err <= bound).all()), f"{what}: worst {(err / bound).max().item():.3g} of the bound"
+
+
+@pytest.mark.parametrize("a_k,b_k", LAYOUTS)
+@pytest.mark.parametrize("M,N,Kd", [
+    (8, 8, 8),          # less than a tile in every direction
+    (64, 64, 64),       # one 64x64 tile, one k-tile
+    (72, 136, 72),      # one past a tile, k-tail of one chunk
+    (128, 128, 192),    # three k-tiles: the remainder steps alone
+    (120, 248, 264),    # four k-tiles and a tail
+    (200, 328, 1000),   # ragged everywhere
+    (2048, 1024, 328),  # 128x128 tiles, k-tail of one chunk
+    (1928, 2056, 520),  # 128x128 tiles, ragged edges
+])
+def test_products_at_tile_edges(cuda, M, N, Kd, a_k, b_k):
+    announce(f"gemm {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
+    for dtype in (torch.bfloat16, torch.float16):
+        a, b, ad, bd = _operands(M, N, Kd, a_k, b_k, dtype, cuda, M + 3 * N + 7 * Kd)
+        ref, mag = a @ b, a.abs() @ b.abs()
+        bias = torch.linspace(-1, 1, N).to(dtype)
+        _check(K.gemm(ad, bd, bias=bias.to(cuda)), ref + bias.double(), mag + bias.double().abs(), Kd, dtype,
+               f"{dtype} with bias")
+        acc = torch.full((M, N), 0.5, device=cuda)
+        K.gemm(ad, bd, out=acc, accumulate=True)
+        _check(acc, ref + 0.5, mag + 0.5, Kd, torch.float32, f"{dtype} accumulated")
+        once = acc.clone().fill_(0.5)
+        K.gemm(ad, bd, out=once, accumulate=True)
+        assert torch.equal(acc, once)
+
+
+@pytest.mark.parametrize("N", [3, 7, 66, 131])
+def test_products_with_unaligned_output_rows(cuda, N):
+    """Output widths and row strides that take no vector stores."""
+    M, Kd = 70, 136
+    announce(f"gemm {M}x{N}x{Kd} unaligned C")
+    a, b, ad, bd = _operands(M, N, Kd, True, True, torch.bfloat16, cuda, N)
+    wide = torch.full((M, N + 3), 9.0, dtype=torch.bfloat16, device=cuda)
+    K.gemm(ad, bd, out=wide[:, 1 : N + 1])
+    _check(wide[:, 1 : N + 1], a @ b, a.abs() @ b.abs(), Kd, torch.bfloat16, "strided output")
+    assert bool((wide[:, 0] == 9).all()) and bool((wide[:, N + 1 :] == 9).all())
