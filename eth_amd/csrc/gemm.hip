@@ -27,7 +27,8 @@
 //    the forward, data-gradient and weight-gradient products (for the last,
 //    both operands row-contiguous, through asm MFMAs); m32
 //    (v_mfma_f32_32x32x16) a row-contiguous A with a K-contiguous B.  Both
-//    need K % 128 == 0 and 16-byte aligned C rows.
+//    need 16-byte aligned C rows; m16 takes any K % 64 == 0, and any K for
+//    weight gradients, m32 K % 128 == 0.
 //  * gemm_ring_kernel: 128x128 or 64x64 tiles with four LDS stages, for the
 //    grids that 256x256 tiles leave mostly idle and for every shape and
 //    alignment (any K % 8 == 0).
@@ -149,6 +150,17 @@ struct DTile {
         off[j] = r0 + c * 8 < rows ? (int32_t)(((int64_t)row * ld + r0 + c * 8) * 2) : kOob;
     }
   }
+  // from here on the pieces' units at k >= left of a k-tile read zeros: set
+  // for the last k-tile when K is no multiple of 64, once its turn comes
+  __device__ __forceinline__ void limit(int left) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int j = 0; j < PER_WAVE; ++j) {
+      const int u = (wave * PER_WAVE + j) * 64 + lane;
+      const int row = u / UPR, c = u % UPR;
+      if ((KC ? (c ^ kc_swizzle(row)) * 8 : row) >= left) off[j] = kOob;
+    }
+  }
   // pieces [J0, J1) of k-tile k0 into the LDS image at S
   template <int J0, int J1>
   __device__ __forceinline__ void issue(uint16_t* S, rsrc_t rs, int64_t ld, int k0) {
@@ -193,7 +205,7 @@ struct GemmArgs {
   int64_t c_split_stride;   // split-K: elements between the splits' C slices
 };
 
-// 256x256x64 tiles, 4 waves of 128x128 (one per SIMD), K % 128 == 0.
+// 256x256x64 tiles, 4 waves of 128x128 (one per SIMD).
 //
 // MFMA v_mfma_f32_16x16x32: a 128x128 wave tile is 8 x 8 blocks of 16x16,
 // 4 fp32 accumulators per lane each (256 in all, AGPRs).  A k-tile of 64 is
@@ -247,7 +259,7 @@ __device__ __forceinline__ void mfma16_tied(f32x4_t& c, const uint4& a, const ui
                  : "v"(__builtin_bit_cast(u32x4_t, a)), "v"(__builtin_bit_cast(u32x4_t, b)));
 }
 
-template <bool A_K, bool B_K, bool FP16>
+template <bool A_K, bool B_K, bool FP16, bool TAIL = false>
 __global__ void __launch_bounds__(256, 1) gemm256_m16_kernel(GemmArgs g) {
   constexpr int BM = 256, BN = 256, BK = 64;
   typedef DTile<BM, BK, A_K> ATile;
@@ -300,7 +312,16 @@ __global__ void __launch_bounds__(256, 1) gemm256_m16_kernel(GemmArgs g) {
     for (int j = 0; j < 8; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   PIN_ACC
 
-  const int nk = (g.k_split ? g.k_split : g.K) / BK;
+  const int span = (g.k_split ? min(g.K, kb + g.k_split) : g.K) - kb;
+  const int nk = (span + BK - 1) / BK;
+  // TAIL: the last k-tile lacks rows of k (left of them are there; with
+  // left == 0 tail stays past it).  Weight gradients only, where K is the
+  // number of tokens, and an instantiation of their own (the branch in the
+  // loop costs 0.5 % of a layer's time): the other layouts' builtin MFMAs
+  // get their accumulators copied around with it (77 vs 51 us for
+  // [2048, 8192] x 2048), so they take K % 64 == 0 (model widths) here and
+  // leave other K to the ring kernel.
+  const int left = span % BK, tail = left ? nk - 1 : nk + 2;
   const rsrc_t ra = make_rsrc(g.A, g.a_bytes), rb = make_rsrc(g.B, g.b_bytes);
   // empty ranges: the loads issued past the last k-tile read zeros
   const rsrc_t ra0 = make_rsrc(g.A, 0), rb0 = make_rsrc(g.B, 0);
@@ -311,8 +332,17 @@ __global__ void __launch_bounds__(256, 1) gemm256_m16_kernel(GemmArgs g) {
   static_assert((NA == 8 || NA == 9) && (NB == 8 || NB == 9), "the k loop's load slots");
   la.init(g.lda, m0, g.M);
   lb.init(g.ldb, n0, g.N);
+#define LIMIT_IF(T)                      \
+  if constexpr (TAIL) {                  \
+    if ((T) == tail) {                   \
+      la.limit(left);                    \
+      lb.limit(left);                    \
+    }                                    \
+  }
+  LIMIT_IF(0)
   la.template issue<0, NA>(smem, ra, g.lda, kb);
   lb.template issue<0, NB>(smem + A_IMG, rb, g.ldb, kb);
+  LIMIT_IF(1)
 
   // queue item Q of a k-tile (the A pieces, then the B pieces) into stage S
 #define LOAD_Q(Q, S, RSA, RSB, KK)                                      \
@@ -417,13 +447,15 @@ __global__ void __launch_bounds__(256, 1) gemm256_m16_kernel(GemmArgs g) {
     const rsrc_t rsa2 = (KT) + 2 < nk ? ra : ra0;         \
     const rsrc_t rsb2 = (KT) + 2 < nk ? rb : rb0;         \
     KSTEP_A(cur, 0, cur, 1)                               \
+    LIMIT_IF((KT) + 2)                                    \
     KSTEP_B(cur, 1, nxt, 0)                               \
   }
   SB RD_A(smem, 0, 0) SB RD_A(smem, 0, 1) SB RD_A(smem, 0, 2) SB RD_A(smem, 0, 3) SB
 #pragma unroll
   for (int j = 0; j < 8; ++j) { RD_B(smem, 0, j) }
   SB
-  // two k-tiles per trip, so both LDS stages have fixed addresses
+  // two k-tiles per trip, so both LDS stages have fixed addresses (with an
+  // odd count the last one is all zeros)
   for (int kt = 0; kt < nk; kt += 2) {
     ITER(smem, smem1, kt)
     ITER(smem1, smem, kt + 1)
@@ -431,6 +463,7 @@ __global__ void __launch_bounds__(256, 1) gemm256_m16_kernel(GemmArgs g) {
   // asm MFMAs: wait states before any instruction reads their accumulators
   if constexpr (!A_K) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 #undef PIN_ACC
+#undef LIMIT_IF
 #undef ITER
 #undef KSTEP_A
 #undef KSTEP_B
@@ -1073,6 +1106,8 @@ static int launch_256(const GemmArgs& a, int a_k, int b_k, hipStream_t s, int sp
     gemm256_m16_kernel<true, true, FP16><<<tiles, 256, 0, s>>>(a);
   else if (a_k && !b_k)
     gemm256_m16_kernel<true, false, FP16><<<tiles, 256, 0, s>>>(a);
+  else if (!a_k && !b_k && a.K % 64)
+    gemm256_m16_kernel<false, false, FP16, true><<<tiles, 256, 0, s>>>(a);
   else if (!a_k && !b_k)
     gemm256_m16_kernel<false, false, FP16><<<tiles, 256, 0, s>>>(a);
   else
@@ -1124,15 +1159,15 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
   a.flags = flags;
   a.alpha = alpha;
   hipStream_t s = (hipStream_t)stream;
-  // the 256x256 kernels: K in whole k-tile pairs, C rows 16-byte aligned
-  // (vector stores), C extent plus one tile of rows below 2 GiB (its buffer
-  // offsets)
+  // the 256x256 kernels: C rows 16-byte aligned (vector stores), C extent
+  // plus one tile of rows below 2 GiB (its buffer offsets), and the K each
+  // layout takes
   const int esz = c_dtype == ETH_F32 ? 4 : 2;
   const int64_t c_extent = ((M - 1) * ldc + N) * esz;
   a.c_vec = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C % (4 * esz)) == 0;
   a.k_split = 0;
   a.c_split_stride = 0;
-  const bool wide = K % 128 == 0 && a.c_vec && c_extent + 256 * ldc * esz < (1LL << 31);
+  const bool wide = K % (a_kcontig ? 64 : b_kcontig ? 128 : 8) == 0 && a.c_vec && c_extent + 256 * ldc * esz < (1LL << 31);
   a.c_bytes = wide ? (uint32_t)c_extent : 0;
   const bool fp16 = in_dtype == ETH_F16;
   switch (plan_tile(M, N, K, wide)) {
@@ -1184,7 +1219,7 @@ extern "C" int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int spl
   if (M <= 0 || N <= 0 || K <= 0 || splits < 2) return 0;
   // the second kernel: a launch, and the partials and C at about 4.5 TB/s
   const double sum = 5.0 + 4.0 * (double)M * (double)N * (splits + 1) / 4.5e6;
-  const double one = tile_time(plan_tile(M, N, K, K % 128 == 0), M, N, K, 1);
+  const double one = tile_time(plan_tile(M, N, K, true), M, N, K, 1);
   return tile_time(256, M, N, K, splits) + sum < one;
 }
 

@@ -61,6 +61,26 @@ def test_products_at_tile_edges(cuda, M, N, Kd, a_k, b_k):
         assert torch.equal(acc, once)
 
 
+@pytest.mark.parametrize("a_k,b_k,Kd", [
+    # weight gradients: any number of tokens, the last k-tile short (one,
+    # two, three, four and six k-tiles)
+    (False, False, 8), (False, False, 72), (False, False, 184), (False, False, 200), (False, False, 328),
+    # forward and data gradients: an odd number of whole k-tiles
+    (True, True, 64), (True, True, 192), (True, False, 64), (True, False, 192),
+])
+def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd):
+    """128 tiles of 256x256 with ragged edges, every k-tile count the loop
+    and its prologue treat apart."""
+    M, N = 4088, 2040
+    announce(f"gemm wide {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
+    a, b, ad, bd = _operands(M, N, Kd, a_k, b_k, torch.bfloat16, cuda, Kd)
+    ref, mag = a @ b, a.abs() @ b.abs()
+    acc = torch.full((M, N), 0.5, device=cuda)
+    K.gemm(ad, bd, out=acc, accumulate=True)
+    _check(acc, ref + 0.5, mag + 0.5, Kd, torch.float32, "accumulated")
+    _check(K.gemm(ad, bd), ref, mag, Kd, torch.bfloat16, "16-bit")
+
+
 @pytest.mark.parametrize("N", [3, 7, 66, 131])
 def test_products_with_unaligned_output_rows(cuda, N):
     """Output widths and row strides that take no vector stores."""
