@@ -1183,30 +1183,59 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
 }
 
 namespace eth {
-// C[m, n] += sum_s W[s][m*N + n], splits added in order (deterministic)
-__global__ void splitk_reduce_kernel(const float* __restrict__ W, int splits, int64_t stride, float* __restrict__ C,
-                                     int64_t ldc, int M, int N, int accumulate) {
-  const int nq = N / 4;
-  const int64_t total = (int64_t)M * nq;
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < total; q += (int64_t)gridDim.x * blockDim.x) {
-    const int m = (int)(q / nq), n = (int)(q % nq) * 4;
-    float4 acc = *reinterpret_cast<const float4*>(W + (int64_t)m * N + n);
-    for (int sp = 1; sp < splits; ++sp) {
-      const float4 w = *reinterpret_cast<const float4*>(W + sp * stride + (int64_t)m * N + n);
-      acc.x += w.x;
-      acc.y += w.y;
-      acc.z += w.z;
-      acc.w += w.w;
+struct SplitSum {
+  const float* W;   // [splits][M][N] partial products
+  int splits;
+  int64_t stride;   // elements between splits
+  void* C;
+  int64_t ldc;
+  const uint16_t* bias;
+  int M, N;
+  int c_dtype, flags;
+  float alpha;
+};
+// C[m, n] (+)= alpha * sum_s W[s][m*N + n] (+ bias[n]), splits added in order
+// (deterministic) and rounded once.  Four columns a thread; the splits' loads
+// go out four at a time.
+template <bool FP16>
+__global__ void __launch_bounds__(256) splitk_sum_kernel(SplitSum g) {
+  const int nq = g.N / 4;
+  const int64_t total = (int64_t)g.M * nq;
+  for (int64_t q = blockIdx.x * 256LL + threadIdx.x; q < total; q += gridDim.x * 256LL) {
+    const int m = (int)(q / nq), n = (int)(q - (int64_t)m * nq) * 4;
+    const float* w = g.W + (int64_t)m * g.N + n;
+    f32x4_t v = *reinterpret_cast<const f32x4_t*>(w);
+    int s = 1;
+    for (; s + 3 < g.splits; s += 4) {
+      f32x4_t u[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) u[e] = *reinterpret_cast<const f32x4_t*>(w + (s + e) * g.stride);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v += u[e];
     }
-    float4* c = reinterpret_cast<float4*>(C + (int64_t)m * ldc + n);
-    if (accumulate) {
-      const float4 o = *c;
-      acc.x = o.x + acc.x;
-      acc.y = o.y + acc.y;
-      acc.z = o.z + acc.z;
-      acc.w = o.w + acc.w;
+    for (; s < g.splits; ++s) v += *reinterpret_cast<const f32x4_t*>(w + s * g.stride);
+    float bn[4] = {0.f, 0.f, 0.f, 0.f};
+    if (g.bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bn[e] = FP16 ? h2f_bits(g.bias[n + e]) : bf2f(g.bias[n + e]);
     }
-    *c = acc;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = v[e] * g.alpha + bn[e];
+    const int64_t o = (int64_t)m * g.ldc + n;
+    if (g.c_dtype == ETH_F32) {
+      f32x4_t* c = reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(g.C) + o);
+      *c = (g.flags & ETH_GEMM_ACCUMULATE) ? *c + v : v;
+    } else {
+      u32x2_t r;
+      if (g.c_dtype == ETH_BF16) {
+        r.x = f2bf_pair(v[0], v[1]);
+        r.y = f2bf_pair(v[2], v[3]);
+      } else {
+        r.x = f2h_bits(v[0]) | ((uint32_t)f2h_bits(v[1]) << 16);
+        r.y = f2h_bits(v[2]) | ((uint32_t)f2h_bits(v[3]) << 16);
+      }
+      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(g.C) + o) = r;
+    }
   }
 }
 }  // namespace eth
@@ -1223,22 +1252,29 @@ extern "C" int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int spl
   return tile_time(256, M, N, K, splits) + sum < one;
 }
 
-extern "C" int eth_gemm_splitk(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,
-                               float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int in_dtype, int splits,
-                               int accumulate, float* workspace, void* stream) {
+extern "C" int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb,
+                                   int b_kcontig, void* C, int64_t ldc, int c_dtype, const void* bias, int64_t M,
+                                   int64_t N, int64_t K, int in_dtype, int flags, float alpha, int splits,
+                                   float* workspace, void* stream) {
   ETH_CHECK_ARG(in_dtype == ETH_BF16 || in_dtype == ETH_F16, "eth_gemm_splitk: inputs must be bf16 or fp16");
+  ETH_CHECK_ARG(valid_dtype(c_dtype), "eth_gemm_splitk: bad output dtype %d", c_dtype);
   ETH_CHECK_ARG(A && B && C && workspace, "eth_gemm_splitk: null operand");
   ETH_CHECK_ARG(splits >= 1 && splits <= 16, "eth_gemm_splitk: splits must be in [1, 16] (got %d)", splits);
   ETH_CHECK_ARG(M > 0 && N > 0 && K > 0 && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31),
                 "eth_gemm_splitk: bad shape %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
-  ETH_CHECK_ARG(K % (128LL * splits) == 0, "eth_gemm_splitk: K (%lld) must be a multiple of 128 * splits",
-                (long long)K);
-  ETH_CHECK_ARG(N % 4 == 0 && ldc % 4 == 0 && ldc >= N && ((uintptr_t)C & 15) == 0 && ((uintptr_t)workspace & 15) == 0,
-                "eth_gemm_splitk: C and the workspace need 16-byte aligned rows (N %% 4 == 0)");
+  ETH_CHECK_ARG(K % (a_kcontig ? 64 : b_kcontig ? 128LL * splits : 8) == 0,
+                "eth_gemm_splitk: K (%lld) must be a multiple of 64 (K-contiguous A), 8 (both operands "
+                "row-contiguous) or 128 * splits", (long long)K);
+  const int esz = c_dtype == ETH_F32 ? 4 : 2;
+  ETH_CHECK_ARG(N % 4 == 0 && ldc % 4 == 0 && ldc >= N && ((uintptr_t)C % (4 * esz)) == 0 &&
+                    ((uintptr_t)workspace & 15) == 0,
+                "eth_gemm_splitk: C and the workspace need aligned rows of four columns (N %% 4 == 0)");
   ETH_CHECK_ARG(lda % 8 == 0 && ldb % 8 == 0, "eth_gemm_splitk: lda/ldb must be multiples of 8");
   ETH_CHECK_ARG(((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0, "eth_gemm_splitk: A/B must be 16-byte aligned");
   ETH_CHECK_ARG(a_kcontig ? lda >= K : (M % 8 == 0 && lda >= M), "eth_gemm_splitk: bad A layout");
   ETH_CHECK_ARG(b_kcontig ? ldb >= K : (N % 8 == 0 && ldb >= N), "eth_gemm_splitk: bad B layout");
+  ETH_CHECK_ARG(!(flags & ETH_GEMM_ACCUMULATE) || c_dtype == ETH_F32, "eth_gemm_splitk: accumulate needs fp32 C");
+  ETH_CHECK_ARG(!(flags & ETH_GEMM_BIAS) || bias, "eth_gemm_splitk: bias flag without bias");
   const int64_t a_elems = a_kcontig ? (M - 1) * lda + K : (K - 1) * lda + M;
   const int64_t b_elems = b_kcontig ? (N - 1) * ldb + K : (K - 1) * ldb + N;
   const int64_t slice = M * N;
@@ -1261,15 +1297,35 @@ extern "C" int eth_gemm_splitk(const void* A, int64_t lda, int a_kcontig, const 
   a.flags = 0;
   a.alpha = 1.0f;
   a.c_bytes = (uint32_t)(slice * 4);
-  a.k_split = (int)(K / splits);
+  // whole k-tiles per split (pairs for m32), the last split shorter; few
+  // k-tiles may leave fewer splits than asked for
+  const int unit = !a_kcontig && b_kcontig ? 128 : 64;
+  a.k_split = (int)(((K + splits - 1) / splits + unit - 1) / unit * unit);
+  splits = (int)((K + a.k_split - 1) / a.k_split);
   a.c_split_stride = slice;
   hipStream_t s = (hipStream_t)stream;
-  const int rc = in_dtype == ETH_BF16 ? launch_256<false>(a, a_kcontig, b_kcontig, s, splits)
-                                      : launch_256<true>(a, a_kcontig, b_kcontig, s, splits);
+  const bool fp16 = in_dtype == ETH_F16;
+  const int rc = fp16 ? launch_256<true>(a, a_kcontig, b_kcontig, s, splits)
+                      : launch_256<false>(a, a_kcontig, b_kcontig, s, splits);
   if (rc != ETH_OK) return rc;
+  const SplitSum sum{workspace, splits, slice, C, ldc, (flags & ETH_GEMM_BIAS) ? (const uint16_t*)bias : nullptr,
+                     (int)M, (int)N, c_dtype, flags, alpha};
   const int64_t quads = M * (N / 4);
   const int grid = (int)std::min<int64_t>((quads + 255) / 256, 2048);
-  splitk_reduce_kernel<<<grid, 256, 0, s>>>(workspace, splits, slice, C, ldc, (int)M, (int)N, accumulate);
+  if (fp16)
+    splitk_sum_kernel<true><<<grid, 256, 0, s>>>(sum);
+  else
+    splitk_sum_kernel<false><<<grid, 256, 0, s>>>(sum);
   ETH_CHECK_LAUNCH("eth_gemm_splitk");
   return ETH_OK;
+}
+
+extern "C" int eth_gemm_splitk(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,
+                               float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int in_dtype, int splits,
+                               int accumulate, float* workspace, void* stream) {
+  ETH_CHECK_ARG(splits >= 1 && splits <= 16, "eth_gemm_splitk: splits must be in [1, 16] (got %d)", splits);
+  ETH_CHECK_ARG(K % (128LL * splits) == 0, "eth_gemm_splitk: K (%lld) must be a multiple of 128 * splits",
+                (long long)K);
+  return eth_gemm_splitk_out(A, lda, a_kcontig, B, ldb, b_kcontig, C, ldc, ETH_F32, nullptr, M, N, K, in_dtype,
+                             accumulate ? ETH_GEMM_ACCUMULATE : 0, 1.0f, splits, workspace, stream);
 }

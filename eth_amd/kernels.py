@@ -71,24 +71,26 @@ def _observe(kind, phase, flops):
 
 
 def _splitk_splits(M, N, K, out):
-    """Split-K factor for an fp32 product whose 256x256 tile grid is too
-    small to fill the chip (fewer than 128 tiles): enough k-splits for about
-    one workgroup per CU, each split a multiple of 128 deep."""
+    """Split-K factor for a product whose 256x256 tile grid is too small to
+    fill the chip (fewer than 128 tiles): enough k-splits for about one
+    workgroup per CU, each at least 1024 deep."""
     tiles = -(-M // 256) * -(-N // 256)
-    if tiles >= 128 or N % 4 or out.stride(0) % 4 or out.data_ptr() % 16:
+    if tiles >= 128 or N % 4 or out.stride(0) % 4 or out.data_ptr() % (4 * out.element_size()):
         return 1
     splits = 1
-    while splits < 16 and tiles * splits * 2 <= 256 and K % (128 * splits * 2) == 0 and K // (splits * 2) >= 1024:
+    while splits < 16 and tiles * splits * 2 <= 256 and K // (splits * 2) >= 1024:
         splits *= 2
     return splits
 
 
 @functools.lru_cache(maxsize=4096)
-def _splitk_pays(M, N, K, splits):
-    """Whether the split-K form finishes before the plain product (sizes
-    only; the smaller tiles fill the chip without a second pass unless K is
-    deep)."""
-    return splits > 1 and bool(nat.value("eth_gemm_splitk_pays", M, N, K, splits))
+def _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig):
+    """Whether the split-K form takes this product and finishes before the
+    plain one (sizes and layout only; the smaller tiles fill the chip
+    without a second pass unless K is deep)."""
+    if splits < 2 or K % (64 if a_kcontig else 128 * splits if b_kcontig else 8) or 4 * (M + 256) * N >= 2**31:
+        return False
+    return bool(nat.value("eth_gemm_splitk_pays", M, N, K, splits))
 
 
 _scratch = {}
@@ -153,15 +155,16 @@ def gemm(a, b, out=None, bias=None, accumulate=False, out_dtype=None, alpha=1.0)
             raise ValueError("bias must be a contiguous [N] tensor of the input dtype")
         flags |= nat.GEMM_BIAS
     _observe("gemm", "begin", 2.0 * M * N * K)
-    fp32_product = out.dtype == torch.float32 and alpha == 1.0 and bias is None
-    splits = _splitk_splits(M, N, K, out) if fp32_product else 1
-    if _splitk_pays(M, N, K, splits):
-        ws = _scratch_f32(nat.value("eth_gemm_splitk_workspace", M, N, splits) // 4, a.device)
+    splits = _splitk_splits(M, N, K, out)
+    if _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig):
+        # (a fresh buffer per call: two threads may share the stream)
+        ws = torch.empty(splits * M * N, dtype=torch.float32, device=a.device)
         nat.call(
-            "eth_gemm_splitk",
+            "eth_gemm_splitk_out",
             nat.ptr(a), lda, a_kcontig,
             nat.ptr(b), ldb, b_kcontig,
-            nat.ptr(out), out.stride(0), M, N, K, code, splits, 1 if accumulate else 0, nat.ptr(ws),
+            nat.ptr(out), out.stride(0), nat.dtype_code(out.dtype),
+            nat.ptr(bias), M, N, K, code, flags, float(alpha), splits, nat.ptr(ws),
             nat.stream_ptr(a.device),
         )
         _observe("gemm", "end", 2.0 * M * N * K)

@@ -248,6 +248,14 @@ int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t l
  * Same reference seam as eth_gemm's ETH_GEMM_ACCUMULATE form
  * (model/distributed.py:116-123 over mpu/layers.py:452-470). */
 int64_t eth_gemm_splitk_workspace(int64_t M, int64_t N, int splits);
+/* The same for every output eth_gemm writes: C of c_dtype, alpha and bias
+ * applied to the sum of the partials, which is rounded once.  K % 64 == 0
+ * with a K-contiguous A, any K % 8 == 0 with both operands row-contiguous,
+ * K % (128 * splits) == 0 otherwise; N % 4 == 0 and C rows aligned to four
+ * columns.  Deterministic; the partials stay fp32. */
+int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,
+                        void* C, int64_t ldc, int c_dtype, const void* bias, int64_t M, int64_t N, int64_t K,
+                        int in_dtype, int flags, float alpha, int splits, float* workspace, void* stream);
 /* 1 where eth_gemm_splitk with `splits` is expected to finish before
  * eth_gemm on the same [M, N] x K product, else 0. */
 int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits);

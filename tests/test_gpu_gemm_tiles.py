@@ -10,6 +10,7 @@ subnormal spacing as a floor)."""
 import pytest
 import torch
 
+from eth_amd import _native as nat
 from eth_amd import kernels as K
 from tests.conftest import announce
 
@@ -79,6 +80,49 @@ def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd):
     K.gemm(ad, bd, out=acc, accumulate=True)
     _check(acc, ref + 0.5, mag + 0.5, Kd, torch.float32, "accumulated")
     _check(K.gemm(ad, bd), ref, mag, Kd, torch.bfloat16, "16-bit")
+
+
+@pytest.mark.parametrize("a_k,b_k,Kd,splits", [
+    (True, True, 320, 3),     # two whole splits and a short one
+    (True, False, 1984, 16),  # 31 k-tiles: two each, the last split one
+    (False, False, 200, 16),  # fewer k-tiles than splits, the last one short
+    (False, True, 512, 2),
+])
+def test_splitk_every_output(cuda, a_k, b_k, Kd, splits):
+    M, N = 264, 136
+    announce(f"gemm split-K {M}x{N}x{Kd}/{splits} a_k={a_k} b_k={b_k}")
+    for dtype in (torch.bfloat16, torch.float16):
+        a, b, ad, bd = _operands(M, N, Kd, a_k, b_k, dtype, cuda, Kd + splits)
+        ref, mag = a @ b, a.abs() @ b.abs()
+        bias = torch.linspace(-1, 1, N).to(dtype)
+        lda, ldb = ad.stride(0 if a_k else 1), bd.stride(1 if b_k else 0)
+        ws = torch.full((splits * M * N,), float("nan"), device=cuda)
+        for out_dtype in (dtype, torch.float32):
+            out = torch.full((M, N + 4), 0.5, dtype=out_dtype, device=cuda)
+            accumulate = out_dtype == torch.float32
+            flags = nat.GEMM_BIAS | (nat.GEMM_ACCUMULATE if accumulate else 0)
+            nat.call("eth_gemm_splitk_out", nat.ptr(ad), lda, int(a_k), nat.ptr(bd), ldb, int(b_k), nat.ptr(out),
+                     out.stride(0), nat.dtype_code(out_dtype), nat.ptr(bias.to(cuda)), M, N, Kd, nat.dtype_code(dtype),
+                     flags, 2.0, splits, nat.ptr(ws), nat.stream_ptr(cuda))
+            extra = bias.double() + (0.5 if accumulate else 0.0)
+            _check(out[:, :N], 2 * ref + extra, 2 * mag + extra.abs(), Kd, out_dtype, f"{dtype} -> {out_dtype}")
+            assert bool((out[:, N:] == 0.5).all())
+
+
+def test_deep_product_takes_splits(cuda):
+    """A 16-bit output of two wide tiles, 16448 deep: split-K, the same bits
+    every time, and refused where the layout's K does not allow it."""
+    M, N, Kd = 256, 512, 16448
+    announce(f"gemm deep {M}x{N}x{Kd}")
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=cuda)
+    splits = K._splitk_splits(M, N, Kd, out)
+    assert splits == 16 and K._splitk_pays(M, N, Kd, splits, 1, 0)
+    assert not K._splitk_pays(M, N, Kd + 8, splits, 1, 0) and not K._splitk_pays(M, N, Kd, splits, 0, 1)
+    assert not K._splitk_pays(2048, 2048, 2048, 2, 1, 1)
+    a, b, ad, bd = _operands(M, N, Kd, True, False, torch.bfloat16, cuda, 5)
+    got = K.gemm(ad, bd)
+    _check(got, a @ b, a.abs() @ b.abs(), Kd, torch.bfloat16, "deep")
+    assert torch.equal(got, K.gemm(ad, bd))
 
 
 @pytest.mark.parametrize("N", [3, 7, 66, 131])
