@@ -11,6 +11,8 @@ from pathlib import Path
 
 import numpy as np
 
+import torch
+
 LIB_PATH = Path(__file__).resolve().parent / "libeth_amd.so"
 
 ETH_OK, ETH_ERR_INVALID, ETH_ERR_HIP = 0, 1, 2
@@ -171,37 +173,47 @@ def exported_symbols():
     return ["eth_abi_version", "eth_last_error", *SIGNATURES, *VALUE_SIGNATURES]
 
 
+_bound = {}  # name -> the library's function, bound once
+
+
+def _bind(name):
+    fn = _bound[name] = getattr(load(), name)
+    return fn
+
+
 def value(name, *args):
-    return getattr(load(), name)(*args)
+    return (_bound.get(name) or _bind(name))(*args)
 
 
 def call(name, *args):
-    lib = load()
-    status = getattr(lib, name)(*args)
+    status = (_bound.get(name) or _bind(name))(*args)
     if status != ETH_OK:
-        msg = lib.eth_last_error().decode(errors="replace")
+        msg = load().eth_last_error().decode(errors="replace")
         if status == ETH_ERR_INVALID:
             raise ValueError(f"{name}: {msg}")
         raise EthError(f"{name}: {msg}")
 
 
-def dtype_code(torch_dtype):
-    import torch
+_DTYPE_CODES = {torch.float32: ETH_F32, torch.float16: ETH_F16, torch.bfloat16: ETH_BF16}
 
-    codes = {torch.float32: ETH_F32, torch.float16: ETH_F16, torch.bfloat16: ETH_BF16}
-    if torch_dtype not in codes:
+
+def dtype_code(torch_dtype):
+    code = _DTYPE_CODES.get(torch_dtype)
+    if code is None:
         raise ValueError(f"unsupported dtype {torch_dtype}")
-    return codes[torch_dtype]
+    return code
 
 
 def stream_ptr(device=None):
-    import torch
-
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream's handle (an address; the argument converters take
+    it as the void pointer).  Asked of the runtime by device index: wrapping
+    it in a torch.cuda.Stream first took longer than the launch's checks."""
+    index = torch.device(device).index if device is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(tensor):
-    return ctypes.c_void_p(tensor.data_ptr()) if tensor is not None else ctypes.c_void_p(0)
+    return tensor.data_ptr() if tensor is not None else None
 
 
 def require_cuda(*tensors):
@@ -212,7 +224,5 @@ def require_cuda(*tensors):
 
 def table_to_device(array, device):
     """Copy a numpy structured table to device memory (uint8 tensor)."""
-    import torch
-
     host = torch.from_numpy(np.ascontiguousarray(array).view(np.uint8).copy())
     return host.to(device=device, non_blocking=False)

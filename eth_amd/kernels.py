@@ -7,6 +7,7 @@ the current stream.  There is no CPU fallback: CPU tensors raise.
 
 import ctypes
 import functools
+import itertools
 
 import numpy as np
 
@@ -14,19 +15,20 @@ import torch
 
 from . import _native as nat
 
-_HALF = (torch.bfloat16, torch.float16)
+_HALF_CODES = {torch.bfloat16: nat.ETH_BF16, torch.float16: nat.ETH_F16}
 
 
 def _check_half(*ts):
     dt = ts[0].dtype
-    if dt not in _HALF:
+    code = _HALF_CODES.get(dt)
+    if code is None:
         raise ValueError(f"expected bf16/fp16 tensors, got {dt}")
     for t in ts:
         if t.dtype != dt:
             raise ValueError(f"dtype mismatch {t.dtype} vs {dt}")
         if not t.is_cuda:
             raise ValueError("eth_amd kernels run on the GPU only (no CPU fallback)")
-    return nat.dtype_code(dt)
+    return code
 
 
 def _rows_cols(x):
@@ -44,9 +46,10 @@ def _matrix_layout(t):
     if t.dim() != 2:
         raise ValueError("expected a 2-D operand")
     s0, s1 = t.stride()
-    if s1 == 1 and s0 >= t.shape[1]:
+    rows, cols = t.shape
+    if s1 == 1 and s0 >= cols:
         return s0, True
-    if s0 == 1 and s1 >= t.shape[0]:
+    if s0 == 1 and s1 >= rows:
         return s1, False
     raise ValueError(f"operand with strides {t.stride()} is neither row- nor column-major")
 
@@ -108,6 +111,8 @@ def _scratch_f32(numel, device):
 
 
 _side = {}
+_side_launches = itertools.count(1)
+_side_last = 0  # a value no earlier launch had, set at every side-stream launch
 
 
 def side_stream(device):
@@ -120,9 +125,23 @@ def side_stream(device):
     return st
 
 
-def join_side_streams():
+def mark_side_launch():
+    """Note work about to be issued on a side stream."""
+    global _side_last
+    _side_last = next(_side_launches)
+
+
+def side_mark():
+    """Changes whenever side-stream work was issued (by any thread)."""
+    return _side_last
+
+
+def join_side_streams(since=None):
     """Make the current stream wait for all side-stream work (before main
-    grads are read)."""
+    grads are read); with `since`, an earlier side_mark(), only if any was
+    issued after it."""
+    if since is not None and since == _side_last:
+        return
     for dev, st in _side.items():
         torch.cuda.current_stream(dev).wait_stream(st)
 

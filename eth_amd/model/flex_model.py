@@ -36,10 +36,22 @@ _SEGMENT_BREAK = "enc-1st-layernorm"
 _UPDATE_LEAD = 5
 
 
+def _parameters(module):
+    """module's parameters in no particular order, a shared one perhaps more
+    than once (module.parameters() names and deduplicates them, which for an
+    op's few parameters takes the host longer than the op's launch)."""
+    for p in module._parameters.values():
+        if p is not None:
+            yield p
+    for child in module._modules.values():
+        if child is not None:
+            yield from _parameters(child)
+
+
 def launch_updates(op):
     """Issue the not yet launched parts of an overlapped update that write
     op's parameters (an optimizer step leaves `_eth_update_launch` on them)."""
-    for p in op.parameters():
+    for p in _parameters(op):
         launch = getattr(p, "_eth_update_launch", None)
         if launch is not None:
             launch()
@@ -53,7 +65,7 @@ def await_parameters(op):
     forward's) do not queue it again (each queued wait costs the stream a
     few microseconds).  A part not launched yet is launched first, since a
     wait on an event not yet recorded waits for nothing."""
-    for p in op.parameters():
+    for p in _parameters(op):
         launch = getattr(p, "_eth_update_launch", None)
         if launch is not None:
             launch()

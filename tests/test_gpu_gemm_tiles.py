@@ -95,6 +95,7 @@ def test_splitk_every_output(cuda, a_k, b_k, Kd, splits):
         a, b, ad, bd = _operands(M, N, Kd, a_k, b_k, dtype, cuda, Kd + splits)
         ref, mag = a @ b, a.abs() @ b.abs()
         bias = torch.linspace(-1, 1, N).to(dtype)
+        bd1 = bias.to(cuda)
         lda, ldb = ad.stride(0 if a_k else 1), bd.stride(1 if b_k else 0)
         ws = torch.full((splits * M * N,), float("nan"), device=cuda)
         for out_dtype in (dtype, torch.float32):
@@ -102,7 +103,7 @@ def test_splitk_every_output(cuda, a_k, b_k, Kd, splits):
             accumulate = out_dtype == torch.float32
             flags = nat.GEMM_BIAS | (nat.GEMM_ACCUMULATE if accumulate else 0)
             nat.call("eth_gemm_splitk_out", nat.ptr(ad), lda, int(a_k), nat.ptr(bd), ldb, int(b_k), nat.ptr(out),
-                     out.stride(0), nat.dtype_code(out_dtype), nat.ptr(bias.to(cuda)), M, N, Kd, nat.dtype_code(dtype),
+                     out.stride(0), nat.dtype_code(out_dtype), nat.ptr(bd1), M, N, Kd, nat.dtype_code(dtype),
                      flags, 2.0, splits, nat.ptr(ws), nat.stream_ptr(cuda))
             extra = bias.double() + (0.5 if accumulate else 0.0)
             _check(out[:, :N], 2 * ref + extra, 2 * mag + extra.abs(), Kd, out_dtype, f"{dtype} -> {out_dtype}")
