@@ -1072,11 +1072,16 @@ static int launch_ring(const GemmArgs& a, int a_k, int b_k, hipStream_t s) {
 // all three layouts; within about 15 %): rounds of one workgroup per CU (two
 // for 64x64, whose 64 KB of LDS leaves room for a second) times the k-tiles of
 // 64 at the measured pace plus the prologue and epilogue.  A 256x256 k-tile
-// runs faster when half the CUs idle (more clock and bandwidth for the rest).
+// runs faster when half the CUs idle (more clock and bandwidth for the rest),
+// in a last round too.
 static double tile_time(int tile, int64_t M, int64_t N, int64_t K, int splits) {
   const double tiles = (double)((M + tile - 1) / tile) * (double)((N + tile - 1) / tile) * splits;
   const double nk = (double)(((K + splits - 1) / splits + 63) / 64);
-  if (tile == 256) return 3.0 + ceil(tiles / 256) * (nk * (tiles > 128 ? 1.20 : 0.93) + 9.0);
+  if (tile == 256) {
+    const double rounds = floor(tiles / 256), last = tiles - 256 * rounds;
+    const double full = nk * 1.20 + 9.0;
+    return 3.0 + rounds * full + (last > 128 ? full : last > 0 ? nk * 0.93 + 9.0 : 0.0);
+  }
   if (tile == 128) return 2.0 + ceil(tiles / 256) * (nk * 0.52 + 6.0);
   return tiles <= 256 ? 2.0 + nk * 0.24 + 1.0 : 1.0 + ceil(tiles / 512) * (nk * 0.36 + 2.7);
 }
@@ -1114,6 +1119,50 @@ static int launch_256(const GemmArgs& a, int a_k, int b_k, hipStream_t s, int sp
     gemm256_m32_kernel<false, true, FP16><<<tiles, 256, 0, s>>>(a);
   ETH_CHECK_LAUNCH("eth_gemm");
   return ETH_OK;
+}
+
+// The rows and columns of C to give whole rounds of 256x256 tiles, the rest
+// going to a second launch in its own best tile: a grid a little over a whole
+// number of rounds otherwise spends a full round on it ([7680, 2560] x 3000:
+// 300 tiles, 136 us in two rounds, 125 us as 250 tiles and 200 of 128x128).
+// Taken where the model promises 7 %; all of C where not.  Also measured
+// (us): [6144, 2816] x 2816 113 -> 80, [4400, 4608] x 1536 70 -> 63,
+// [2500, 8192] x 2048 87 -> 77, [1024, 50304] x 1024 107 -> 97.
+struct GemmCut {
+  int64_t m, n;
+};
+static GemmCut plan_cut(int64_t M, int64_t N, int64_t K, bool wide) {
+  GemmCut best{M, N};
+  if (!wide) return best;
+  const int tile = plan_tile(M, N, K, wide);
+  const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256, rounds = tm * tn / 256;
+  if (tile != 256 || rounds < 1 || tm * tn % 256 == 0) return best;
+  double t = 0.93 * tile_time(256, M, N, K, 1);
+  auto rest = [&](int64_t m, int64_t n) { return tile_time(plan_tile(m, n, K, wide), m, n, K, 1); };
+  const int64_t m1 = rounds * 256 / tn * 256, n1 = rounds * 256 / tm * 256;
+  if (m1 > 0 && m1 < M) {
+    const double u = tile_time(256, m1, N, K, 1) + rest(M - m1, N);
+    if (u < t) {
+      t = u;
+      best = GemmCut{m1, N};
+    }
+  }
+  if (n1 > 0 && n1 < N) {
+    const double u = tile_time(256, M, n1, K, 1) + rest(M, N - n1);
+    if (u < t) best = GemmCut{M, n1};
+  }
+  return best;
+}
+
+static int launch_planned(const GemmArgs& a, int a_k, int b_k, bool fp16, bool wide, hipStream_t s) {
+  switch (plan_tile(a.M, a.N, a.K, wide)) {
+    case 256:
+      return fp16 ? launch_256<true>(a, a_k, b_k, s) : launch_256<false>(a, a_k, b_k, s);
+    case 128:
+      return fp16 ? launch_ring<128, true>(a, a_k, b_k, s) : launch_ring<128, false>(a, a_k, b_k, s);
+    default:
+      return fp16 ? launch_ring<64, true>(a, a_k, b_k, s) : launch_ring<64, false>(a, a_k, b_k, s);
+  }
 }
 
 }  // namespace eth
@@ -1170,16 +1219,33 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
   const bool wide = K % (a_kcontig ? 64 : b_kcontig ? 128 : 8) == 0 && a.c_vec && c_extent + 256 * ldc * esz < (1LL << 31);
   a.c_bytes = wide ? (uint32_t)c_extent : 0;
   const bool fp16 = in_dtype == ETH_F16;
-  switch (plan_tile(M, N, K, wide)) {
-    case 256:
-      return fp16 ? launch_256<true>(a, a_kcontig, b_kcontig, s) : launch_256<false>(a, a_kcontig, b_kcontig, s);
-    case 128:
-      return fp16 ? launch_ring<128, true>(a, a_kcontig, b_kcontig, s)
-                  : launch_ring<128, false>(a, a_kcontig, b_kcontig, s);
-    default:
-      return fp16 ? launch_ring<64, true>(a, a_kcontig, b_kcontig, s)
-                  : launch_ring<64, false>(a, a_kcontig, b_kcontig, s);
+  const GemmCut cut = plan_cut(M, N, K, wide);
+  if (cut.m == M && cut.n == N) return launch_planned(a, a_kcontig, b_kcontig, fp16, wide, s);
+  // the part of whole rounds, then the rest (rows or columns of C)
+  const int64_t M2 = M - cut.m, N2 = N - cut.n;
+  GemmArgs r = a;
+  if (M2) {
+    a.M = (int)cut.m;
+    a.a_bytes = (uint32_t)((a_kcontig ? (cut.m - 1) * lda + K : (K - 1) * lda + cut.m) * 2);
+    a.c_bytes = (uint32_t)(((cut.m - 1) * ldc + N) * esz);
+    r.M = (int)M2;
+    r.A += a_kcontig ? cut.m * lda : cut.m;
+    r.a_bytes = (uint32_t)((a_kcontig ? (M2 - 1) * lda + K : (K - 1) * lda + M2) * 2);
+    r.C = (char*)C + cut.m * ldc * esz;
+    r.c_bytes = (uint32_t)(((M2 - 1) * ldc + N) * esz);
+  } else {
+    a.N = (int)cut.n;
+    a.b_bytes = (uint32_t)((b_kcontig ? (cut.n - 1) * ldb + K : (K - 1) * ldb + cut.n) * 2);
+    a.c_bytes = (uint32_t)(((M - 1) * ldc + cut.n) * esz);
+    r.N = (int)N2;
+    r.B += b_kcontig ? cut.n * ldb : cut.n;
+    r.b_bytes = (uint32_t)((b_kcontig ? (N2 - 1) * ldb + K : (K - 1) * ldb + N2) * 2);
+    r.C = (char*)C + cut.n * esz;
+    if (r.bias) r.bias += cut.n;
+    r.c_bytes = (uint32_t)(((M - 1) * ldc + N2) * esz);
   }
+  const int rc = launch_planned(a, a_kcontig, b_kcontig, fp16, wide, s);
+  return rc != ETH_OK ? rc : launch_planned(r, a_kcontig, b_kcontig, fp16, wide, s);
 }
 
 namespace eth {

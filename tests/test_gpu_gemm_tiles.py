@@ -82,6 +82,31 @@ def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd):
     _check(K.gemm(ad, bd), ref, mag, Kd, torch.bfloat16, "16-bit")
 
 
+@pytest.mark.parametrize("a_k,b_k,M,N,Kd", [
+    (False, False, 7680, 2552, 520),  # 300 wide tiles: 250 and a rest of rows
+    (True, True, 2304, 8192, 512),    # 288: a rest of columns, with bias
+    (True, False, 8200, 2048, 512),   # 264: eight rows past a whole round
+])
+def test_products_past_whole_rounds(cuda, a_k, b_k, M, N, Kd):
+    """Grids a little over a whole number of rounds run in two launches."""
+    announce(f"gemm rounds {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
+    gen = torch.Generator(device=cuda).manual_seed(M + N)
+    a = torch.randn(*((M, Kd) if a_k else (Kd, M)), device=cuda, generator=gen).bfloat16()
+    b = torch.randn(*((N, Kd) if b_k else (Kd, N)), device=cuda, generator=gen).bfloat16()
+    ad, bd = a if a_k else a.t(), b.t() if b_k else b
+    bias = torch.linspace(-1, 1, N, device=cuda).bfloat16()
+    ref = (ad.double() @ bd.double()).cpu()
+    mag = (ad.double().abs() @ bd.double().abs()).cpu()
+    extra = bias.double().cpu()
+    wide = torch.full((M, N + 8), 9.0, dtype=torch.bfloat16, device=cuda)
+    K.gemm(ad, bd, out=wide[:, :N], bias=bias)
+    _check(wide[:, :N], ref + extra, mag + extra.abs(), Kd, torch.bfloat16, "strided output with bias")
+    assert bool((wide[:, N:] == 9).all())
+    acc = torch.full((M, N), 0.5, device=cuda)
+    K.gemm(ad, bd, out=acc, accumulate=True)
+    _check(acc, ref + 0.5, mag + 0.5, Kd, torch.float32, "accumulated")
+
+
 @pytest.mark.parametrize("a_k,b_k,Kd,splits", [
     (True, True, 320, 3),     # two whole splits and a short one
     (True, False, 1984, 16),  # 31 k-tiles: two each, the last split one
