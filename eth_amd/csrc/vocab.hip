@@ -68,62 +68,75 @@ __global__ void __launch_bounds__(256) embedding_fwd_kernel(const int64_t* __res
 // ---------------------------------------------------------------------------
 // Deterministic embedding backward: sort, then one owner per table row.
 //
-// For each table (word ids, position ids) a single workgroup sorts the keys
+// For each table (word ids, position ids) the keys
 //   key = (clamped id << row_bits) | dout row        (row = s * B + b)
-// in LDS with a bitonic network, so equal ids become one contiguous run
-// ordered by dout row.  The accumulate kernel then gives every run to the
-// workgroup of its first sorted slot, which sums the run's dout rows in fp32
-// in that order and adds the sum into the fp32 main grad once: no atomics,
-// and the same bits on every run.  The keys fit 32 bits when
-// bits(V - 1) + bits(T - 1) <= 32; T <= kEmbSortMax keeps the LDS image at
-// 128 KB (static; gfx950 gives a workgroup up to 160 KB).  Longer inputs
-// run as consecutive chunks of whole sequence positions (at most
-// kEmbSortMax dout rows each), one sort + accumulate per chunk in sequence
-// order: each table row then receives one ordered sum per chunk.
-constexpr int kEmbSortThreads = 1024;
+// are put in ascending order, so equal ids become one contiguous run ordered
+// by dout row.  The keys are distinct, so the place of a key is the number of
+// smaller ones, counted by brute force: T^2 compares over the whole chip take
+// less time than a sorting network's chain of barriers in one workgroup (the
+// whole backward with uniform ids, against a bitonic sort in LDS: 128 rows of
+// 1024 9.5 -> 6.1 us, 2048 of 2048 41 -> 23 us, 8192 of 2048 133 -> 76 us,
+// 32768 of 1024 488 -> 313 us).  The accumulate kernel then gives every run to the workgroup of its
+// first sorted slot, which sums the run's dout rows in fp32 in that order and
+// adds the sum into the fp32 main grad once: no atomics, and the same bits on
+// every run.  The keys fit 32 bits when bits(V - 1) + bits(T - 1) <= 32.
+// Inputs above kEmbSortMax rows run as consecutive chunks of whole sequence
+// positions (at most kEmbSortMax dout rows each), one sort + accumulate per
+// chunk in sequence order: each table row then receives one ordered sum per
+// chunk.
 constexpr int kEmbSortMax = 32768;
+constexpr int kRankThreads = 256, kRankSegs = 8, kRankKeys = kRankThreads / kRankSegs;
+constexpr int kRankTile = 4096;  // keys staged in LDS at a time
 
 __device__ __forceinline__ int64_t clamp_id(int64_t v, int64_t n) { return v < 0 ? 0 : (v >= n ? n - 1 : v); }
 
-// blockIdx.x = 0 sorts the token ids into keys[0, T), 1 the position ids
-// into keys[T, 2T); sample b's ids start at ids + b * ld
-__global__ void __launch_bounds__(kEmbSortThreads) embedding_sort_kernel(const int64_t* __restrict__ tok,
-                                                                        const int64_t* __restrict__ pid,
-                                                                        uint32_t* __restrict__ keys, int B, int S,
-                                                                        int64_t ld, int64_t V, int64_t P,
-                                                                        int row_bits, int n2) {
-  __shared__ uint32_t sk[kEmbSortMax];
+// blockIdx.y = 0 sorts the token ids into keys[0, T), 1 the position ids
+// into keys[T, 2T); sample b's ids start at ids + b * ld.  A workgroup places
+// kRankKeys keys: kRankSegs lanes share a key, each comparing it with every
+// kRankSegs-th group of four staged keys (the lanes of one segment read the
+// same 16 bytes, the eight segments 128 consecutive ones).  Bound by the
+// compares, two VALU operations each.
+__global__ void __launch_bounds__(kRankThreads) embedding_sort_kernel(const int64_t* __restrict__ tok,
+                                                                      const int64_t* __restrict__ pid,
+                                                                      uint32_t* __restrict__ keys, int B, int S,
+                                                                      int64_t ld, int64_t V, int64_t P,
+                                                                      int row_bits) {
+  __shared__ __attribute__((aligned(16))) uint32_t sk[kRankTile];
   const int T = B * S;
-  const int64_t* ids = blockIdx.x == 0 ? tok : pid;
-  const int64_t lim = blockIdx.x == 0 ? V : P;
-  for (int i = threadIdx.x; i < n2; i += kEmbSortThreads) {
-    uint32_t k = 0xFFFFFFFFu;
-    if (i < T) {
-      const int si = i / B, bi = i - si * B;  // dout row i holds (s, b)
-      k = ((uint32_t)clamp_id(ids[(int64_t)bi * ld + si], lim) << row_bits) | (uint32_t)i;
+  const int64_t* ids = blockIdx.y == 0 ? tok : pid;
+  const int64_t lim = blockIdx.y == 0 ? V : P;
+  auto key_of = [&](int i) __attribute__((always_inline)) {  // dout row i holds (s, b)
+    const int si = i / B, bi = i - si * B;
+    return ((uint32_t)clamp_id(ids[(int64_t)bi * ld + si], lim) << row_bits) | (uint32_t)i;
+  };
+  const int seg = threadIdx.x % kRankSegs;
+  const int own = blockIdx.x * kRankKeys + threadIdx.x / kRankSegs;
+  const uint32_t mine = own < T ? key_of(own) : 0u;
+  int place = 0;
+  for (int t0 = 0; t0 < T; t0 += kRankTile) {
+    const int n = min(kRankTile, T - t0);
+    const int groups = (n + 3) / 4;  // of four keys, the last filled up with keys no smaller than any
+    __syncthreads();
+    for (int i = threadIdx.x; i < groups * 4; i += kRankThreads) sk[i] = i < n ? key_of(t0 + i) : 0xFFFFFFFFu;
+    __syncthreads();
+    const uint4* s4 = reinterpret_cast<const uint4*>(sk);
+#pragma unroll 4
+    for (int g = seg; g < groups; g += kRankSegs) {
+      const uint4 k = s4[g];
+      place += (k.x < mine) + (k.y < mine) + (k.z < mine) + (k.w < mine);
     }
-    sk[i] = k;
   }
-  __syncthreads();
-  for (int k = 2; k <= n2; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      for (int i = threadIdx.x; i < (n2 >> 1); i += kEmbSortThreads) {
-        const int lo = 2 * j * (i / j) + (i % j), hi = lo + j;
-        const uint32_t a = sk[lo], b = sk[hi];
-        if ((a > b) == ((lo & k) == 0)) {
-          sk[lo] = b;
-          sk[hi] = a;
-        }
-      }
-      __syncthreads();
-    }
-  }
-  uint32_t* out = keys + (int64_t)blockIdx.x * T;
-  for (int i = threadIdx.x; i < T; i += kEmbSortThreads) out[i] = sk[i];
+#pragma unroll
+  for (int off = 1; off < kRankSegs; off <<= 1) place += __shfl_xor(place, off, 64);
+  if (seg == 0 && own < T) keys[(int64_t)blockIdx.y * T + place] = mine;
 }
 
 // grid (T, column chunks of 2048, tables): the workgroup at the first
-// sorted slot of a run owns that table row
+// sorted slot of a run owns that table row.  A frequent token's run is a
+// chain of fp32 adds in row order, so its rows are loaded kAccumBatch at a
+// time: with one load at a time, 2048 tokens in text's proportions (the most
+// frequent 55 times) took 14 us longer than uniform ones, now no longer.
+constexpr int kAccumBatch = 16;
 template <bool FP16>
 __global__ void __launch_bounds__(256) embedding_accum_kernel(const uint32_t* __restrict__ keys,
                                                               const uint16_t* __restrict__ dout,
@@ -137,17 +150,37 @@ __global__ void __launch_bounds__(256) embedding_accum_kernel(const uint32_t* __
   const int c = blockIdx.y * 2048 + threadIdx.x * 8;
   if (c >= H) return;
   const uint32_t mask = (1u << row_bits) - 1u;
+  float4* d = reinterpret_cast<float4*>(dst + (int64_t)id * H + c);
+  float4 x0 = d[0], x1 = d[1];
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  int end = j + 1;
-  while (end < T && (ks[end] >> row_bits) == id) ++end;
-  for (int r = j; r < end; ++r) {
-    const uint4 a = *reinterpret_cast<const uint4*>(dout + (int64_t)(ks[r] & mask) * H + c);
+  auto add = [&](const uint4& a) __attribute__((always_inline)) {
     const uint16_t* e = reinterpret_cast<const uint16_t*>(&a);
 #pragma unroll
     for (int q = 0; q < 8; ++q) acc[q] += vin<FP16>(e[q]);
+  };
+  auto row_at = [&](int r) __attribute__((always_inline)) {
+    return *reinterpret_cast<const uint4*>(dout + (int64_t)(ks[r] & mask) * H + c);
+  };
+  int r = j;
+  // whole batches: the slot that ends one still belongs to the run
+  for (; r + kAccumBatch <= T && (ks[r + kAccumBatch - 1] >> row_bits) == id; r += kAccumBatch) {
+    uint4 a[kAccumBatch];
+#pragma unroll
+    for (int u = 0; u < kAccumBatch; ++u) a[u] = row_at(r + u);
+#pragma unroll
+    for (int u = 0; u < kAccumBatch; ++u) add(a[u]);
   }
-  float4* d = reinterpret_cast<float4*>(dst + (int64_t)id * H + c);
-  float4 x0 = d[0], x1 = d[1];
+  // the rest, fewer than a batch: loads that run past it read its last row
+  int left = 0;
+  while (r + left < T && left < kAccumBatch && (ks[r + left] >> row_bits) == id) ++left;
+  for (int u0 = 0; u0 < left; u0 += 4) {
+    uint4 a[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) a[u] = row_at(r + min(u0 + u, left - 1));
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (u0 + u < left) add(a[u]);
+  }
   x0.x += acc[0]; x0.y += acc[1]; x0.z += acc[2]; x0.w += acc[3];
   x1.x += acc[4]; x1.y += acc[5]; x1.z += acc[6]; x1.w += acc[7];
   d[0] = x0;
@@ -446,11 +479,9 @@ extern "C" int eth_embedding_bwd(const int64_t* tokens, const int64_t* positions
   for (int64_t s0 = 0; s0 < seq; s0 += sc) {
     const int64_t len = seq - s0 < sc ? seq - s0 : sc;
     const int64_t T = batch * len;
-    int n2 = 1;
-    while (n2 < T) n2 <<= 1;
-    if (n2 < 2) n2 = 2;
-    embedding_sort_kernel<<<2, kEmbSortThreads, 0, s>>>(tokens + s0, positions + s0, keys, (int)batch, (int)len,
-                                                          seq, vocab, max_pos, row_bits, n2);
+    const dim3 places((unsigned)((T + kRankKeys - 1) / kRankKeys), 2);
+    embedding_sort_kernel<<<places, kRankThreads, 0, s>>>(tokens + s0, positions + s0, keys, (int)batch, (int)len,
+                                                          seq, vocab, max_pos, row_bits);
     ETH_CHECK_LAUNCH("eth_embedding_bwd (sort)");
     dim3 grid((unsigned)T, (unsigned)((hidden + 2047) / 2048), 2);
     const uint16_t* dc = d + s0 * batch * hidden;  // dout rows [s0 * B, (s0 + len) * B)
