@@ -22,8 +22,8 @@
 // MFMA result layout of S^T equal to the operand layout of P^T in
 // O^T = V^T P^T, so P never leaves registers.  The dK/dV kernel uses the
 // mirror image (S = Q K^T, lane = key, query rows swizzled) and computes S
-// and P once for both gradients, in pairs of waves that hand P over through
-// LDS; dQ has its own kernel (recomputing P), so no atomics are needed and
+// and P once for both gradients (head dim 128 in pairs of waves that hand P
+// over through LDS); dQ has its own kernel (recomputing P), so no atomics are needed and
 // results are deterministic.  The dQ kernel runs first and also writes
 // delta = rowsum(dO * O), which the dK/dV kernel reads.
 //
@@ -116,9 +116,6 @@ constexpr int kBKV = 64;   // forward / dQ: keys per step
 constexpr int kBKV2 = 128; // dK/dV: keys per workgroup (4 waves x 32)
 constexpr int kBQ2 = 64;   // dK/dV: queries per step
 constexpr int32_t kAttnOob = (int32_t)0x80000000u;  // buffer offset past any tensor: loads read zeros
-// row length (elements) of an LDS tile read with ds_read_b64_tr_b16: four
-// consecutive rows then start 64 bytes apart in the bank space
-constexpr int tr_row(int d) { return d % 64 == 0 ? d + 32 : d + 64; }
 // 16 bytes of a row at column `col` of a strided tensor; with PAD, zeros
 // past the sequence or the head dim (without, every row and column is real)
 template <bool PAD>
@@ -136,95 +133,100 @@ __device__ __forceinline__ uint16_t* row_ptr(const AttnOut& t, int s, int b, int
   return t.p + (int64_t)s * t.ss + (int64_t)b * t.sb + (int64_t)h * t.sh;
 }
 
-// ROWS x D tile of a strided tensor through buffer loads: each thread's
-// offsets within the (batch, head) slice are fixed, the row advance is a
-// scalar offset, so a load costs no address arithmetic.  Stored into LDS
-// rows of LROW elements, row index optionally swizzled (SWZ).
 typedef __amdgpu_buffer_rsrc_t a_rsrc_t;
-template <int ROWS, int D, int LROW, bool SWZ, bool PAD>
-struct BufTile {
-  static constexpr int CPR = D / 8;
-  static constexpr int CPT = ROWS * CPR / kAttnThreads;
-  static_assert(ROWS * CPR % kAttnThreads == 0 && CPT >= 1, "tile split");
-  a_u32x4 v[CPT];
-  int32_t voff[CPT];
-  a_rsrc_t rs;
-  int32_t row_bytes;
-  int rows_left;  // tensor rows (sequence length); rows past it load zeros
-  int tid;        // this thread's index among the kAttnThreads that move the tile
-  // columns at or past hd load zeros (an out-of-range offset)
-  __device__ __forceinline__ void init(const AttnTensor& t, int b, int h, int seq, int hd) {
-    init(t, b, h, seq, hd, threadIdx.x);
-  }
-  __device__ __forceinline__ void init(const AttnTensor& t, int b, int h, int seq, int hd, int thread) {
-    tid = thread;
-    rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(t.p), (short)0, (int)t.bytes, 0x00020000);
-    row_bytes = (int32_t)(t.ss * 2);
-    rows_left = seq;
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = tid + i * kAttnThreads;
-      voff[i] = !PAD || (c % CPR) * 8 < hd
-                    ? (int32_t)(((int64_t)b * t.sb + (int64_t)h * t.sh + (int64_t)(c / CPR) * t.ss + (c % CPR) * 8) * 2)
-                    : kAttnOob;
-    }
-  }
-  __device__ __forceinline__ void load(int r0) {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = tid + i * kAttnThreads;
-      const int32_t off = !PAD || r0 + c / CPR < rows_left ? voff[i] : kAttnOob;
-      v[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, off, r0 * row_bytes, 0);
-    }
-  }
-  __device__ __forceinline__ void store(uint16_t* lds) const {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = tid + i * kAttnThreads;
-      const int r = SWZ ? swz(c / CPR) : c / CPR;
-      *reinterpret_cast<a_u32x4*>(lds + r * LROW + (c % CPR) * 8) = v[i];
-    }
-  }
-  // the same rows in natural order into [ROWS][L2] (for transposing reads)
-  template <int L2>
-  __device__ __forceinline__ void store_natural(uint16_t* lds) const {
-#pragma unroll
-    for (int i = 0; i < CPT; ++i) {
-      const int c = tid + i * kAttnThreads;
-      *reinterpret_cast<a_u32x4*>(lds + (c / CPR) * L2 + (c % CPR) * 8) = v[i];
-    }
-  }
-};
-
 typedef short a_s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) a_s16x4 a_lds_s16x4;
 typedef uint32_t a_u32x2 __attribute__((ext_vector_type(2)));
-// MFMA operand of 8 consecutive k from a [k][m] LDS tile (row length LROW)
-// by two ds_read_b64_tr_b16: lane l passes the address of k-row
-// k0 + (l%16)/4 (k0 = 8*(l/32)), element m0 + 16*((l/16)%2) + 4*(l%4)
-// (tr_lane gives that offset) and receives m = m0 + l%32, k = k0..k0+7.
-__device__ __forceinline__ int tr_lane(int lane, int lrow) {
-  return ((lane >> 5) * 8 + ((lane & 15) >> 2)) * lrow + ((lane >> 4) & 1) * 16 + (lane & 3) * 4;
+// ------------------------------------------------------- images in LDS --
+// A 64-row block of a tensor lies in LDS as it is in memory, except that chunk
+// c (8 columns, 16 bytes) of row r is at c ^ img_swz(r): the row reads of an
+// MFMA operand (16 lanes on 16 rows, one chunk) and the transposing
+// ds_read_b64_tr_b16 reads (4 rows x 64 bytes per 32 lanes) then both hit
+// distinct banks, so one image serves both.  It is filled by direct
+// global->LDS loads a whole block ahead: no register staging, no copy phase.
+// Each image is an array of its own, so the compiler can tell the loads into
+// one from the reads of another and puts no wait between them.
+__device__ __forceinline__ int xsw(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
+template <int D>
+__device__ __forceinline__ int img_swz(int r) {
+  if constexpr (D == 128)
+    return xsw(r);
+  else if constexpr (D == 64)  // 128-byte rows: bit 0 of r picks the half of the banks
+    return (((r >> 1) & 1) << 2) | (((r >> 3) & 1) << 1) | ((r >> 2) & 1);
+  else  // 192-byte rows start 64 bytes apart in the banks: within groups of four chunks
+    return (r >> 2) & 3;
 }
-__device__ __forceinline__ uint4 tr_frag(const uint16_t* p, int lrow) {
-  const a_u32x2 lo = __builtin_bit_cast(a_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((a_lds_s16x4*)p));
-  const a_u32x2 hi = __builtin_bit_cast(a_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((a_lds_s16x4*)(p + 4 * lrow)));
+// the four waves' direct loads: unit u (16 bytes) of the image holds row
+// u / CPR, chunk (u % CPR) ^ img_swz(row).  With PAD, rows at or past `seq`
+// and columns at or past `hd` read zeros.
+template <int D, bool PAD>
+struct ImgCopy {
+  static constexpr int CPR = D / 8;  // 16-byte chunks per row
+  static constexpr int PW = D / 32;  // 1 KB pieces per wave
+  int32_t off[PW];
+  int row[PW];
+  a_rsrc_t rs;
+  int32_t row_bytes;
+  int w, seq;
+  __device__ __forceinline__ void init(const AttnTensor& t, int b, int h, int hd, int s, int wave, int lane) {
+    rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(t.p), (short)0, (int)t.bytes, 0x00020000);
+    row_bytes = (int32_t)(t.ss * 2);
+    w = wave;
+    seq = s;
+#pragma unroll
+    for (int j = 0; j < PW; ++j) {
+      const int u = (w * PW + j) * 64 + lane;
+      const int r = u / CPR, c = (u % CPR) ^ img_swz<D>(r);
+      row[j] = r;
+      off[j] = !PAD || c * 8 < hd
+                   ? (int32_t)(((int64_t)b * t.sb + (int64_t)h * t.sh + (int64_t)r * t.ss + c * 8) * 2)
+                   : kAttnOob;
+    }
+  }
+  __device__ __forceinline__ void issue(uint16_t* S, int r0) const {
+#pragma unroll
+    for (int j = 0; j < PW; ++j) {
+      const int32_t o = !PAD || r0 + row[j] < seq ? off[j] : kAttnOob;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(S + (w * PW + j) * 512),
+                                               16, o, r0 * row_bytes, 0, 0);
+    }
+  }
+};
+// Row reads: row t*32 + swz(lane%32) (the swizzled order that makes the
+// result's layout the operand layout of the next product), chunk 2*ks + lane/32:
+// element offset of k-step ks within a 32-row tile.
+template <int D>
+__device__ __forceinline__ int img_row_off(int lane, int ks) {
+  const int r = swz(lane & 31);
+  return r * D + (((2 * ks + (lane >> 5)) ^ img_swz<D>(r)) << 3);
+}
+// Transposing reads: rows kk*16 + 8*(l/32) + (l%16)/4 (+4 for the second
+// read, hi), columns ct*32 + 16*((l/16)%2) + 4*(l%4): element offset within
+// the 16-row group kk.
+template <int D>
+__device__ __forceinline__ int img_tr_off(int lane, int ct, int hi) {
+  const int r = 8 * (lane >> 5) + ((lane & 15) >> 2) + 4 * hi;
+  const int c = 4 * ct + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+  return r * D + ((c ^ img_swz<D>(r)) << 3) + (lane & 1) * 4;
+}
+__device__ __forceinline__ uint4 img_tr(const uint16_t* p, int lo_off, int hi_off) {
+  const a_u32x2 lo = __builtin_bit_cast(a_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((a_lds_s16x4*)(p + lo_off)));
+  const a_u32x2 hi = __builtin_bit_cast(a_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((a_lds_s16x4*)(p + hi_off)));
   return make_uint4(lo.x, lo.y, hi.x, hi.y);
 }
 
 // ------------------------------------------------------------------ forward --
-// 4 waves x 32 queries; K/V blocks of 64 keys double-buffered in LDS (the
-// next block's global loads are in flight while this one is computed); two
-// workgroups per CU, so one wave's softmax overlaps the other's MFMAs.
+// 4 waves x 32 queries; K/V blocks of 64 keys in double-buffered images, one
+// barrier per block; two workgroups per CU, so one wave's softmax overlaps
+// another's MFMAs.
 template <int D, bool FP16, bool PAD>
 __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_kernel(AttnArgs a) {
   constexpr int KS = D / 16;  // k-steps over the head dim
   constexpr int DT = D / 32;  // 32-row tiles over the head dim
-  // K rows swizzled (see the file comment); V rows as they are, padded to
-  // D + 32 so the transposing reads of O^T = V^T P^T hit distinct banks
-  constexpr int VL = tr_row(D);
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[2][kBKV * (D + 8)];
-  __shared__ __attribute__((aligned(16))) uint16_t Vs[2][kBKV * VL];
+  __shared__ __attribute__((aligned(16))) uint16_t K0[kBKV * D];
+  __shared__ __attribute__((aligned(16))) uint16_t K1[kBKV * D];
+  __shared__ __attribute__((aligned(16))) uint16_t V0[kBKV * D];
+  __shared__ __attribute__((aligned(16))) uint16_t V1[kBKV * D];
 
   const int BH = a.B * a.H, nqb = (a.S + kBQ - 1) / kBQ;
   const int bh = blockIdx.x % BH, qb = nqb - 1 - blockIdx.x / BH;
@@ -234,6 +236,13 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_kernel(AttnArgs a) {
   const int q0 = qb * kBQ + w * 32;
   const int q = q0 + (lane & 31);
   const float sl2 = a.scale_log2;
+
+  ImgCopy<D, PAD> kc, vc;
+  kc.init(a.k, b, h, a.hd, a.S, w, lane);
+  vc.init(a.v, b, h, a.hd, a.S, w, lane);
+  const int nkv = (qb * kBQ + kBQ) / kBKV;  // blocks up to the diagonal
+  kc.issue(K0, 0);
+  vc.issue(V0, 0);
 
   uint4 qf[KS];
   {
@@ -248,237 +257,32 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_kernel(AttnArgs a) {
     for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
   float m = -1e30f, l = 0.f;  // running max (log2 units) and sum for query q
 
-  const int nkv = (qb * kBQ + kBQ) / kBKV;  // blocks up to the diagonal
-  BufTile<kBKV, D, D + 8, true, PAD> kt;
-  BufTile<kBKV, D, VL, false, PAD> vt;
-  kt.init(a.k, b, h, a.S, a.hd);
-  vt.init(a.v, b, h, a.S, a.hd);
-  kt.load(0);
-  vt.load(0);
-  kt.store(Ks[0]);
-  vt.store(Vs[0]);
-  const int vtr = tr_lane(lane, VL);
-  __syncthreads();
-  // the Q fragment loads may still be in flight here; waiting for them now
-  // (through the builtin, which the compiler's wait-count pass sees) keeps
-  // that pass from making every iteration's first MFMAs wait for the next
-  // block's prefetch loads
-  vm_wait_all();
-
-  for (int j = 0; j < nkv; ++j) {
-    const int st = j & 1;
-    const bool more = j + 1 < nkv;
-    if (more) {
-      kt.load((j + 1) * kBKV);
-      vt.load((j + 1) * kBKV);
-    }
-    const int kv0 = j * kBKV;
-    if (kv0 <= q0 + 31) {  // wave has at least one unmasked key in the block
-      // S^T = K Q^T (raw scores; lane = query, registers = 32 of the keys)
-      a_f32x16 s[2];
+  int aoff[KS], toff[DT][2];
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+  for (int ks = 0; ks < KS; ++ks) aoff[ks] = img_row_off<D>(lane, ks);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
-      // all K fragments of the first 32-key tile are read before its MFMAs,
-      // each register refilled with the second tile's fragment right after
-      // its MFMA issues (order pinned: left alone, the compiler reads each
-      // fragment one or two MFMAs before its use and waits on the LDS latency)
-      {
-        const uint16_t* kp0 = Ks[st] + (lane & 31) * (D + 8) + hl * 8;
-        const uint16_t* kp1 = kp0 + 32 * (D + 8);
-        uint4 kr[KS];
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) kr[ks] = *reinterpret_cast<const uint4*>(kp0 + ks * 16);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          s[0] = mma<FP16>(kr[ks], qf[ks], s[0]);
-          __builtin_amdgcn_sched_barrier(0);
-          kr[ks] = *reinterpret_cast<const uint4*>(kp1 + ks * 16);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) s[1] = mma<FP16>(kr[ks], qf[ks], s[1]);
-      }
-      if (kv0 + kBKV - 1 > q0) {  // diagonal block: mask keys after the query
-#pragma unroll
-        for (int t = 0; t < 2; ++t)
-#pragma unroll
-          for (int r = 0; r < 16; ++r)
-            if (kv0 + t * 32 + swz_row(r, hl) > q) s[t][r] = -1e30f;
-      }
-      float mx = s[0][0];
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[t][r]);
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      const float mnew = fmaxf(m, mx * sl2);
-      // m is the exponent offset, kept within kRescaleLog2 below the running
-      // max: O and l are rescaled only when some row's max grew past that,
-      // so p = exp2(s - m) stays <= 2^kRescaleLog2 (exact in fp32, the same
-      // relative precision in 16 bits) and most blocks skip the rescale;
-      // O / l and lse = m + log2(l) do not depend on the offset
-      if (__any(mnew > m + kRescaleLog2)) {
-        const float alpha = fast_exp2(m - mnew);
-        l *= alpha;
-#pragma unroll
-        for (int t = 0; t < DT; ++t)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
-        m = mnew;
-      }
-      float rs = 0.f;
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float p = fast_exp2(__builtin_fmaf(s[t][r], sl2, -m));
-          s[t][r] = p;
-          rs += p;
-        }
-      l += rs;
-      // O^T += V^T P^T over the 64 keys (4 k-steps of 16)
-#pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        const int t = kk >> 1, e0 = (kk & 1) * 8;
-        const uint4 pb = make_uint4(pack2<FP16>(s[t][e0 + 0], s[t][e0 + 1]), pack2<FP16>(s[t][e0 + 2], s[t][e0 + 3]),
-                                    pack2<FP16>(s[t][e0 + 4], s[t][e0 + 5]), pack2<FP16>(s[t][e0 + 6], s[t][e0 + 7]));
-        const uint16_t* vp = Vs[st] + vtr + kk * 16 * VL;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) o[dt] = mma<FP16>(tr_frag(vp + dt * 32, VL), pb, o[dt]);
-      }
-    }
-    if (more) {
-      kt.store(Ks[st ^ 1]);
-      vt.store(Vs[st ^ 1]);
-    }
-    __syncthreads();
-  }
-  l += __shfl_xor(l, 32, 64);
-  if (PAD && q >= a.S) return;  // a padding row of the last query block
-  const float inv = 1.0f / l;
-  uint16_t* op = row_ptr(a.out, q, b, h);
-#pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      if (PAD && t * 32 + g * 8 >= a.hd) continue;  // hd % 8 == 0: whole 8-column groups
-      uint2 v;
-      v.x = pack2<FP16>(o[t][g * 4 + 0] * inv, o[t][g * 4 + 1] * inv);
-      v.y = pack2<FP16>(o[t][g * 4 + 2] * inv, o[t][g * 4 + 3] * inv);
-      *reinterpret_cast<uint2*>(op + t * 32 + g * 8 + hl * 4) = v;
-    }
-  if (hl == 0) a.lse[(int64_t)bh * a.S + q] = m + log2f(l);
-}
-
-// -------------------------------------------------- forward, head_dim 128 --
-// attn_fwd_kernel for D = 128 with each 64-key block of K and V in an
-// XOR-swizzled LDS image (chunk c of row r at c ^ xsw(r), see
-// attn_bwd_dkdv_x128_kernel), double buffered and filled by direct
-// global->LDS loads a whole block ahead: no register staging, no copy
-// phase, one barrier per block.  K rows are read as A operands (S^T = K Q^T)
-// and V through transposing reads (O^T = V^T P^T); same arithmetic in the
-// same order as attn_fwd_kernel, so the results are bit-identical.
-__device__ __forceinline__ int xsw(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
-template <bool FP16, bool PAD>
-__global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_x128_kernel(AttnArgs a) {
-  constexpr int D = 128, KS = D / 16, DT = D / 32;
-  constexpr int IMG = kBKV * D;
-  __shared__ __attribute__((aligned(16))) uint16_t Kx[2 * IMG];
-  __shared__ __attribute__((aligned(16))) uint16_t Vx[2 * IMG];
-
-  const int BH = a.B * a.H, nqb = (a.S + kBQ - 1) / kBQ;
-  const int bh = blockIdx.x % BH, qb = nqb - 1 - blockIdx.x / BH;
-  const int b = bh / a.H, h = bh % a.H;
-  const int lane = threadIdx.x & 63, hl = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
-  const int q0 = qb * kBQ + w * 32;
-  const int q = q0 + (lane & 31);
-  const float sl2 = a.scale_log2;
-
-  // direct loads: each wave fills 4 pieces of the K image and 4 of the V image
-  const a_rsrc_t rsk = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.k.p), (short)0, (int)a.k.bytes,
-                                                         0x00020000);
-  const a_rsrc_t rsv = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.v.p), (short)0, (int)a.v.bytes,
-                                                         0x00020000);
-  int32_t koff[4], voff[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int u = (w * 4 + j) * 64 + lane;
-    const int r = u >> 4, c = (u & 15) ^ xsw(r);
-    koff[j] = c * 8 < a.hd ? (int32_t)(((int64_t)b * a.k.sb + (int64_t)h * a.k.sh + (int64_t)r * a.k.ss + c * 8) * 2)
-                           : kAttnOob;
-    voff[j] = c * 8 < a.hd ? (int32_t)(((int64_t)b * a.v.sb + (int64_t)h * a.v.sh + (int64_t)r * a.v.ss + c * 8) * 2)
-                           : kAttnOob;
-  }
-  const int32_t krow = (int32_t)(a.k.ss * 2), vrow = (int32_t)(a.v.ss * 2);
-  auto issue = [&](int slot, int r0) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const bool in = !PAD || r0 + (w * 4 + j) * 4 + (lane >> 4) < a.S;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsk, (__attribute__((address_space(3))) void*)(Kx + slot * IMG + (w * 4 + j) * 512), 16,
-          in ? koff[j] : kAttnOob, r0 * krow, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rsv, (__attribute__((address_space(3))) void*)(Vx + slot * IMG + (w * 4 + j) * 512), 16,
-          in ? voff[j] : kAttnOob, r0 * vrow, 0, 0);
-    }
-  };
-  const int nkv = (qb * kBQ + kBQ) / kBKV;  // blocks up to the diagonal
-  issue(0, 0);
-
-  uint4 qf[KS];
-  {
-    const uint16_t* qp = row_ptr(a.q, q, b, h);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = load_row16<PAD>(qp, q < a.S, ks * 16 + hl * 8, a.hd);
-  }
-  a_f32x16 o[DT];
-#pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
-  float m = -1e30f, l = 0.f;  // running max (log2 units) and sum for query q
-
-  // K rows as A operands: row t*32 + swz(lane%32) (the swizzled key order
-  // that makes S^T's result layout the B operand layout of P^T), chunk
-  // 2*ks + hl
-  int aoff[KS];
-  {
-    const int arow = swz(lane & 31), xa = xsw(arow);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) aoff[ks] = arow * D + (((2 * ks + hl) ^ xa) << 3);
-  }
-  // V^T through transposing reads: k-rows (keys) kk*16 + 8*(l/32) +
-  // (l%16)/4 (+4 for the second read), columns dt*32 + 16*((l/16)%2) + 4*(l%4)
-  int toff[DT][2];
-  {
-    const int R = (lane & 15) >> 2, L5 = lane >> 5, L4 = (lane >> 4) & 1, L1 = (lane >> 1) & 1;
-#pragma unroll
-    for (int d2 = 0; d2 < DT; ++d2)
-#pragma unroll
-      for (int hi = 0; hi < 2; ++hi) {
-        const int row = 8 * L5 + R + 4 * hi;
-        const int pc = 4 * (d2 ^ R) + ((2 * L4 + L1) ^ (2 * L5 + hi));
-        toff[d2][hi] = row * D + pc * 8 + (lane & 1) * 4;
-      }
-  }
+    for (int hi = 0; hi < 2; ++hi) toff[dt][hi] = img_tr_off<D>(lane, dt, hi);
   vm_wait_all();
   __syncthreads();
 
   auto block = [&](int j, auto cur_c) __attribute__((always_inline)) {
     constexpr int cur = decltype(cur_c)::value;
     const int kv0 = j * kBKV;
-    if (j + 1 < nkv) issue(cur ^ 1, kv0 + kBKV);  // the next block, a block ahead
+    if (j + 1 < nkv) {  // the next block, a block ahead
+      kc.issue(cur ? K0 : K1, kv0 + kBKV);
+      vc.issue(cur ? V0 : V1, kv0 + kBKV);
+    }
     if (kv0 <= q0 + 31) {  // wave has at least one unmasked key in the block
-      const uint16_t* ki = Kx + cur * IMG;
-      const uint16_t* vi = Vx + cur * IMG;
+      const uint16_t* ki = cur ? K1 : K0;
+      const uint16_t* vi = cur ? V1 : V0;
+      // S^T = K Q^T (raw scores; lane = query, registers = 32 of the keys)
       a_f32x16 sc[2];
       // all K fragments of the first 32-key tile are read before its MFMAs,
       // each register refilled with the second tile's fragment right after
-      // its MFMA issues (order pinned)
+      // its MFMA issues (order pinned: left alone, the compiler reads each
+      // fragment one or two MFMAs before its use and waits on the LDS latency)
       {
         uint4 kr[KS];
 #pragma unroll
@@ -508,6 +312,11 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_x128_kernel(AttnArgs
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sc[t][r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float mnew = fmaxf(m, mx * sl2);
+      // m is the exponent offset, kept within kRescaleLog2 below the running
+      // max: O and l are rescaled only when some row's max grew past that,
+      // so p = exp2(s - m) stays <= 2^kRescaleLog2 (exact in fp32, the same
+      // relative precision in 16 bits) and most blocks skip the rescale;
+      // O / l and lse = m + log2(l) do not depend on the offset
       if (__any(mnew > m + kRescaleLog2)) {
         const float alpha = fast_exp2(m - mnew);
         l *= alpha;
@@ -535,13 +344,7 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_x128_kernel(AttnArgs
                                     pack2<FP16>(sc[t][e0 + 4], sc[t][e0 + 5]), pack2<FP16>(sc[t][e0 + 6], sc[t][e0 + 7]));
         const uint16_t* vp = vi + kk * 16 * D;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-          const a_u32x2 lo =
-              __builtin_bit_cast(a_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((a_lds_s16x4*)(vp + toff[dt][0])));
-          const a_u32x2 hi =
-              __builtin_bit_cast(a_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((a_lds_s16x4*)(vp + toff[dt][1])));
-          o[dt] = mma<FP16>(make_uint4(lo.x, lo.y, hi.x, hi.y), pb, o[dt]);
-        }
+        for (int dt = 0; dt < DT; ++dt) o[dt] = mma<FP16>(img_tr(vp, toff[dt][0], toff[dt][1]), pb, o[dt]);
       }
     }
     vm_wait_all();  // the next block's rows have landed
@@ -561,7 +364,7 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_x128_kernel(AttnArgs
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
-      if (PAD && t * 32 + g * 8 >= a.hd) continue;
+      if (PAD && t * 32 + g * 8 >= a.hd) continue;  // hd % 8 == 0: whole 8-column groups
       uint2 v;
       v.x = pack2<FP16>(o[t][g * 4 + 0] * inv, o[t][g * 4 + 1] * inv);
       v.y = pack2<FP16>(o[t][g * 4 + 2] * inv, o[t][g * 4 + 3] * inv);
@@ -570,257 +373,30 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_x128_kernel(AttnArgs
   if (hl == 0) a.lse[(int64_t)bh * a.S + q] = m + log2f(l);
 }
 
-// ------------------------------------------------ backward: dK, dV paired --
-// Eight waves: wave w < 4 (the dV wave) and wave w + 4 (the dK wave) own the
-// same 32 keys and share a SIMD.  Per step of 64 queries the dV wave computes
-// S = Q K^T and P and hands P (fp32) to its partner through LDS; the dK wave
-// meanwhile computes dP = dO V^T and subtracts delta.  After the hand-over
-// the dV wave adds P^T dO into dV while the dK wave forms dS = P (dP - delta)
-// and adds dS^T Q into dK.  S and P are computed once per step (the split dV
-// and dK kernels each recompute them), and on every SIMD one wave's
-// exponentials or dS arithmetic overlap the other wave's MFMAs.  S = Q K^T
-// is computed with lane = key (the mirror image of the forward's layout,
-// query rows swizzled), so P and dS are already the A operands of
-// dV += P^T dO and dK += dS^T Q.
-//
-// The Q and dO rows of a step are kept twice in LDS: a row-swizzled copy
-// (rows of D + 8) read as A operands in the first half of the step, and a
-// natural copy (rows padded for the transposing reads) read as B operands
-// in the second half.  Both are filled by direct global->LDS loads, each in
-// the half-step before it is read: the next step's row-swizzled copy during
-// this step's second half, the next step's natural copy during its first
-// half.  A step therefore has two barriers (P handed over; step done) and
-// no copy phase of its own.
-template <int ROWS, int D, int UPR, bool SWZ>
-struct DmaCopy {
-  // one LDS copy of a ROWS x D tile, rows of UPR 16-byte units (the first
-  // D / 8 hold data, the rest padding), moved by the four waves of a role:
-  // lane l of piece j fills unit (piece * 64 + l) of the image
-  static constexpr int PIECES = ROWS * UPR / 64;
-  static constexpr int PW = (PIECES + 3) / 4;  // pieces per wave (the last wave may have fewer)
-  static_assert(ROWS * UPR % 64 == 0, "whole pieces");
-  int32_t off[PW];
-  int32_t row_in_tile[PW];  // image row of the unit (tile row via the swizzle), -1 for padding units
-  int w;                    // wave within the role (wave-uniform)
-  __device__ __forceinline__ void init(const AttnTensor& t, int b, int h, int hd, int wave, int lane) {
-    w = wave;
-#pragma unroll
-    for (int j = 0; j < PW; ++j) {
-      const int u = (w * PW + j) * 64 + lane;
-      const int p = u / UPR, c = u % UPR;
-      const int q = SWZ ? swz(p) : p;  // image row p holds tile row q
-      const bool data = c < D / 8 && c * 8 < hd && p < ROWS;
-      row_in_tile[j] = data ? q : -1;
-      off[j] = data ? (int32_t)(((int64_t)b * t.sb + (int64_t)h * t.sh + (int64_t)q * t.ss + c * 8) * 2) : kAttnOob;
-    }
-  }
-  // rows [r0, r0 + ROWS) of the tensor into the image at S; with PAD, rows
-  // at or past `seq` read zeros
-  template <bool PAD>
-  __device__ __forceinline__ void issue(uint16_t* S, a_rsrc_t rs, int32_t row_bytes, int r0, int seq) const {
-#pragma unroll
-    for (int j = 0; j < PW; ++j) {
-      if (w * PW + j >= PIECES) break;  // wave-uniform
-      const int32_t o = !PAD || (row_in_tile[j] >= 0 && r0 + row_in_tile[j] < seq) ? off[j] : kAttnOob;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)(S + (w * PW + j) * 512),
-                                               16, o, r0 * row_bytes, 0, 0);
-    }
-  }
-};
-
-template <int D, bool FP16, bool PAD>
-__global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_pair_kernel(AttnArgs a) {
-  constexpr int KS = D / 16, DT = D / 32;
-  constexpr int QN = tr_row(D);
-  constexpr int AL = D + 8;  // row length of the row-swizzled copy
-  typedef DmaCopy<kBQ2, D, AL / 8, true> RowCopy;
-  typedef DmaCopy<kBQ2, D, QN / 8, false> TrCopy;
-  __shared__ __attribute__((aligned(16))) uint16_t Qs[RowCopy::PIECES * 512];
-  __shared__ __attribute__((aligned(16))) uint16_t dOs[RowCopy::PIECES * 512];
-  __shared__ __attribute__((aligned(16))) uint16_t Qn[TrCopy::PIECES * 512];
-  __shared__ __attribute__((aligned(16))) uint16_t dOn[TrCopy::PIECES * 512];
-  // P of a step's two 32-query tiles per key group: registers 4g..4g+3 of a
-  // lane as 16 contiguous bytes, the 64 lanes side by side
-  __shared__ a_u32x4 Ps[4][2][4][64];
-  __shared__ float lse_s[kBQ2], del_s[kBQ2];
-
-  const int BH = a.B * a.H;
-  const int bh = blockIdx.x % BH, kb = blockIdx.x / BH;
-  const int b = bh / a.H, h = bh % a.H;
-  const int lane = threadIdx.x & 63, hl = lane >> 5;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
-  const int w = wv & 3;
-  const bool dkw = wv >= 4;                        // the dK wave of its pair
-  const int rt = threadIdx.x & (kAttnThreads - 1);  // thread index within the role
-  const int k0 = kb * kBKV2 + w * 32;
-  const int key = k0 + (lane & 31);
-
-  // B operands of the first product: K rows (S = Q K^T) in the dV wave, V
-  // rows (dP = dO V^T) in the dK wave
-  uint4 kf[KS];
-  {
-    const uint16_t* kp = row_ptr(dkw ? a.v : a.k, key, b, h);
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks) kf[ks] = load_row16<PAD>(kp, key < a.S, ks * 16 + hl * 8, a.hd);
-  }
-  a_f32x16 acc[DT];  // dV in the dV wave, dK in the dK wave
-#pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-
-  // the dV waves move the Q rows, the dK waves the dO rows
-  const AttnTensor& src = dkw ? a.dout : a.q;
-  const a_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(src.p), (short)0, (int)src.bytes,
-                                                        0x00020000);
-  const int32_t row_bytes = (int32_t)(src.ss * 2);
-  RowCopy rowc;
-  TrCopy trc;
-  rowc.init(src, b, h, a.hd, w, lane);
-  trc.init(src, b, h, a.hd, w, lane);
-  uint16_t* const rowimg = dkw ? dOs : Qs;
-  uint16_t* const trimg = dkw ? dOn : Qn;
-  const int qtr = tr_lane(lane, QN);
-  const int first = (kb * kBKV2) / kBQ2, nq = (a.S + kBQ2 - 1) / kBQ2;
-  // per-query statistics of a step: lse for the dV waves' P, delta for the
-  // dK waves' dS (a padding query gets lse = 1e30, so P = 0)
-  auto stat = [&](int qs) __attribute__((always_inline)) {
-    const bool real = !PAD || qs + rt < a.S;
-    const int64_t i = (int64_t)bh * a.S + qs + rt;
-    return dkw ? (real ? a.delta[i] : 0.f) : (real ? a.lse[i] : 1e30f);
-  };
-  float stat_n = 0.f;
-  rowc.template issue<PAD>(rowimg, rs, row_bytes, first * kBQ2, a.S);
-  trc.template issue<PAD>(trimg, rs, row_bytes, first * kBQ2, a.S);
-  if (rt < kBQ2) stat_n = stat(first * kBQ2);
-  vm_wait_all();
-  if (rt < kBQ2) (dkw ? del_s : lse_s)[rt] = stat_n;
-  __syncthreads();
-  for (int qb = first; qb < nq; ++qb) {
-    const int qs0 = qb * kBQ2;
-    const bool more = qb + 1 < nq;
-    // the natural copy of this step (read after the hand-over barrier)
-    if (qb != first) trc.template issue<PAD>(trimg, rs, row_bytes, qs0, a.S);
-    // a pair whose keys all follow every query of the step skips the work
-    // but not the barriers
-    const bool active = qs0 + kBQ2 - 1 >= k0;
-    const bool diag = qs0 < k0 + 31;
-    a_f32x16 x[2];  // S, then P (dV wave); dP - delta, then dS (dK wave)
-    if (active) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) x[t][r] = 0.f;
-        const uint16_t* ap = rowimg + (t * 32 + (lane & 31)) * AL + hl * 8;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) x[t] = mma<FP16>(*reinterpret_cast<const uint4*>(ap + ks * 16), kf[ks], x[t]);
-        if (!dkw) {
-          // P; query index of register r = t*32 + swz_row(r, hl); the causal
-          // mask only on the steps that cross the diagonal
-          auto probs = [&](auto masked) __attribute__((always_inline)) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              const int qi = t * 32 + swz_row(r, hl);
-              float p = fast_exp2(__builtin_fmaf(x[t][r], a.scale_log2, -lse_s[qi]));
-              if (decltype(masked)::value && key > qs0 + qi) p = 0.f;
-              x[t][r] = p;
-            }
-          };
-          if (diag)
-            probs(std::true_type{});
-          else
-            probs(std::false_type{});
-#pragma unroll
-          for (int g = 0; g < 4; ++g)
-            Ps[w][t][g][lane] = a_u32x4{__float_as_uint(x[t][4 * g]), __float_as_uint(x[t][4 * g + 1]),
-                                        __float_as_uint(x[t][4 * g + 2]), __float_as_uint(x[t][4 * g + 3])};
-        } else {
-#pragma unroll
-          for (int r = 0; r < 16; ++r) x[t][r] = x[t][r] - del_s[t * 32 + swz_row(r, hl)];
-        }
-      }
-    }
-    vm_wait_all();  // this step's natural copy has landed
-    __syncthreads();  // P handed over; every row-swizzled read of the step done
-    // the next step's row-swizzled copy and statistics, read after the
-    // step's closing barrier
-    if (more) {
-      rowc.template issue<PAD>(rowimg, rs, row_bytes, qs0 + kBQ2, a.S);
-      if (rt < kBQ2) stat_n = stat(qs0 + kBQ2);
-    }
-    if (active) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        if (dkw) {
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const a_u32x4 pv = Ps[w][t][g][lane];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) x[t][4 * g + e] = __uint_as_float(pv[e]) * x[t][4 * g + e];
-          }
-        }
-        // dV += P^T dO (dV wave) or dK += dS^T Q (dK wave) over the tile's
-        // 32 queries, two k-steps of 16
-        const uint16_t* bp = (dkw ? Qn : dOn) + qtr;
-#pragma unroll
-        for (int k2 = 0; k2 < 2; ++k2) {
-          const int kk = t * 2 + k2, e0 = k2 * 8;
-          const uint4 pa = make_uint4(pack2<FP16>(x[t][e0 + 0], x[t][e0 + 1]), pack2<FP16>(x[t][e0 + 2], x[t][e0 + 3]),
-                                      pack2<FP16>(x[t][e0 + 4], x[t][e0 + 5]), pack2<FP16>(x[t][e0 + 6], x[t][e0 + 7]));
-#pragma unroll
-          for (int d2 = 0; d2 < DT; ++d2) acc[d2] = mma<FP16>(pa, tr_frag(bp + kk * 16 * QN + d2 * 32, QN), acc[d2]);
-        }
-      }
-    }
-    vm_wait_all();  // the next step's row-swizzled copy and statistics have landed
-    if (more && rt < kBQ2) (dkw ? del_s : lse_s)[rt] = stat_n;
-    __syncthreads();  // step done: both copies and P free for the next step
-  }
-  // lane holds d = t*32 + lane%32 for keys k0 + acc_row(r, hl)
-#pragma unroll
-  for (int t = 0; t < DT; ++t)
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int kr = k0 + acc_row(r, hl);
-      const int d = t * 32 + (lane & 31);
-      if (PAD && (kr >= a.S || d >= a.hd)) continue;
-      if (dkw)
-        row_ptr(a.dk, kr, b, h)[d] = from_f<FP16>(acc[t][r] * a.scale);
-      else
-        row_ptr(a.dv, kr, b, h)[d] = from_f<FP16>(acc[t][r]);
-    }
-}
-
 // ------------------------------ backward: dK, dV paired, head_dim 128 --
-// The pairing above for D = 128, skewed by half a step so that each step
-// has one barrier and both waves of a SIMD mix MFMAs and VALU work: in step
-// m the dV wave computes S(m) and P(m) (handing P to LDS) and then adds
-// P(m)^T dO(m) into dV, while the dK wave first finishes step m-1 -- reads
-// P(m-1), forms dS = P (dP - delta) and adds dS^T Q(m-1) into dK -- and then
-// computes dP(m) - delta.  One wave's exponentials or dS arithmetic then
-// fall between the other wave's MFMAs instead of after them.
+// Eight waves: wave w < 4 (the dV wave) and wave w + 4 (the dK wave) own the
+// same 32 keys and share a SIMD.  In step m (64 queries) the dV wave computes
+// S(m) = Q K^T and P(m), hands P (fp32) over through LDS and adds P(m)^T dO(m)
+// into dV, while the dK wave first finishes step m-1 -- reads P(m-1), forms
+// dS = P (dP - delta) and adds dS^T Q(m-1) into dK -- and then computes
+// dP(m) - delta.  S and P are computed once, each step has one barrier, and
+// one wave's exponentials or dS arithmetic fall between the other wave's
+// MFMAs.  S is computed with lane = key (the mirror image of the forward's
+// layout, query rows swizzled), so P and dS are already the A operands of
+// dV += P^T dO and dK += dS^T Q.  (At this width the accumulators of both
+// gradients and their operands do not fit one wave's registers; narrower
+// heads take attn_bwd_dkdv_kernel.)
 //
-// LDS holds one image per tile of 64 query rows: the 16 chunks of 8 columns
-// of a row, chunk c of row r at position c ^ xsw(r); xsw swaps the two
-// 2-bit fields of r mod 16, so the row reads of the A operands (16 lanes on
-// 16 rows, one chunk) and the transposing reads of the B operands (4 rows x
-// 64 bytes per 32 lanes) both hit distinct banks, and one image serves
-// both.  Step m reads Q(m-1), Q(m) and dO(m), and the rows of step m+1 load
-// directly into idle images a whole step ahead: three Q images, two dO
-// images and two P buffers (145 KB in all).  The arithmetic per element is
-// that of the kernel above, in the same order, with one exception: dP's
-// accumulator starts at -delta instead of having delta subtracted after
-// the product.  dV is therefore bit-identical to the kernel above, and dK
-// may differ from it in the last bit of the 16-bit result (about 0.02 % of
-// the elements at the benchmarked shape), the fp32 sum being rounded in
-// another order.
-
+// Step m reads Q(m-1), Q(m) and dO(m), and the rows of step m+1 load directly
+// into idle images: three Q images, two dO images and two P buffers (145 KB
+// in all).  dP's accumulator starts at -delta.
 template <bool FP16, bool PAD>
 __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel(AttnArgs a) {
   constexpr int D = 128, KS = D / 16, DT = D / 32;
   constexpr int IMG = kBQ2 * D;  // elements of one image
   __shared__ __attribute__((aligned(16))) uint16_t Qx[3 * IMG];
-  __shared__ __attribute__((aligned(16))) uint16_t dOx[2 * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t O0[IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t O1[IMG];
   __shared__ a_u32x4 Ps[2][4][2][4][64];
   __shared__ __attribute__((aligned(16))) float lse_s[2][kBQ2];
   __shared__ __attribute__((aligned(16))) float del_s[2][kBQ2];
@@ -865,45 +441,24 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
     doff[j] = c * 8 < a.hd ? (int32_t)(((int64_t)b * src.sb + (int64_t)h * src.sh + (int64_t)r * src.ss + c * 8) * 2)
                            : kAttnOob;
   }
-  uint16_t* const ldsimg = dkw ? dOx : Qx;
-  auto issue = [&](int slot, int r0) __attribute__((always_inline)) {
+  auto issue = [&](uint16_t* img, int r0) __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int32_t o = !PAD || r0 + (w * 4 + j) * 4 + (lane >> 4) < a.S ? doff[j] : kAttnOob;
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rs, (__attribute__((address_space(3))) void*)(ldsimg + slot * IMG + (w * 4 + j) * 512), 16, o,
+          rs, (__attribute__((address_space(3))) void*)(img + (w * 4 + j) * 512), 16, o,
           r0 * row_bytes, 0, 0);
     }
   };
-  // A-operand rows: tile row t*32 + swz(lane%32), chunk 2*ks + hl at
-  // position (2*ks + hl) ^ xsw(row) = 2*(ks ^ (xa >> 1)) + (hl ^ (xa & 1))
-  int aoff[KS];
-  {
-    const int arow = swz(lane & 31), xa = xsw(arow);
+  int aoff[KS], toff[DT][2];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) aoff[ks] = arow * D + (((2 * ks + hl) ^ xa) << 3);
-  }
-  // B-operand transposing reads: k-rows kk*16 + 8*(l/32) + (l%16)/4 (+4 for
-  // the second read), columns d2*32 + 16*((l/16)%2) + 4*(l%4)
-  int toff[DT][2];
-  {
-    const int R = (lane & 15) >> 2, L5 = lane >> 5, L4 = (lane >> 4) & 1, L1 = (lane >> 1) & 1;
+  for (int ks = 0; ks < KS; ++ks) aoff[ks] = img_row_off<D>(lane, ks);
 #pragma unroll
-    for (int d2 = 0; d2 < DT; ++d2)
+  for (int d2 = 0; d2 < DT; ++d2)
 #pragma unroll
-      for (int hi = 0; hi < 2; ++hi) {
-        const int row = 8 * L5 + R + 4 * hi;
-        const int pc = 4 * (d2 ^ R) + ((2 * L4 + L1) ^ (2 * L5 + hi));
-        toff[d2][hi] = row * D + pc * 8 + (lane & 1) * 4;
-      }
-  }
+    for (int hi = 0; hi < 2; ++hi) toff[d2][hi] = img_tr_off<D>(lane, d2, hi);
   auto bfrag = [&](const uint16_t* img, int kk, int d2) __attribute__((always_inline)) {
-    const uint16_t* bp = img + kk * 16 * D;
-    const a_u32x2 lo =
-        __builtin_bit_cast(a_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((a_lds_s16x4*)(bp + toff[d2][0])));
-    const a_u32x2 hi =
-        __builtin_bit_cast(a_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((a_lds_s16x4*)(bp + toff[d2][1])));
-    return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    return img_tr(img + kk * 16 * D, toff[d2][0], toff[d2][1]);
   };
   // acc += X^T B over a step's 64 queries: X (P or dS, one 32-query tile
   // per t) as the A operand, B from the transposing reads of `img`.  Four
@@ -971,13 +526,21 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
   auto stat = [&](int qs) __attribute__((always_inline)) {
     const bool real = !PAD || qs + rt < a.S;
     const int64_t i = (int64_t)bh * a.S + qs + rt;
-    return dkw ? (real ? -a.delta[i] : 0.f) : (real ? a.lse[i] : 1e30f);
+    return dkw ? (real ? a.delta[i] : 0.f) : (real ? a.lse[i] : 1e30f);
+  };
+  // (delta is negated here: at the load, the use would wait for the step's
+  // direct loads too)
+  auto stat_store = [&](int p, float v) __attribute__((always_inline)) {
+    if (dkw)
+      del_s[p][rt] = -v;
+    else
+      lse_s[p][rt] = v;
   };
   float stat_n = 0.f;
-  issue(0, first * kBQ2);
+  issue(dkw ? O0 : Qx, first * kBQ2);
   if (rt < kBQ2) stat_n = stat(first * kBQ2);
   vm_wait_all();
-  if (rt < kBQ2) (dkw ? del_s : lse_s)[0][rt] = stat_n;
+  if (rt < kBQ2) stat_store(0, stat_n);
   __syncthreads();
 
   a_f32x16 x[2];  // S then P (dV wave); dP - delta, then dS (dK wave)
@@ -988,10 +551,16 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
     constexpr bool DKW = decltype(role_c)::value;  // the role, a constant here
     const int m = first + j, qs0 = m * kBQ2;
     const int qnext = qslot == 2 ? 0 : qslot + 1, qprev = qslot == 0 ? 2 : qslot - 1;
-    if (j + 1 < n) {  // the next step's rows into idle images, a step ahead
-      issue(dkw ? P ^ 1 : qnext, qs0 + kBQ2);
-      if (rt < kBQ2) stat_n = stat(qs0 + kBQ2);
-    }
+    // the next step's rows into idle images; the dV waves issue theirs behind
+    // their reads of this step's Q (one array holds the three Q images, so
+    // the compiler waits for loads in flight to it before a read)
+    auto next = [&]() __attribute__((always_inline)) {
+      if (j + 1 < n) {
+        issue(DKW ? (P ? O0 : O1) : Qx + qnext * IMG, qs0 + kBQ2);
+        if (rt < kBQ2) stat_n = stat(qs0 + kBQ2);
+      }
+    };
+    if constexpr (DKW) next();
     // a pair whose keys all follow every query of a step skips its work
     const bool active = qs0 + kBQ2 - 1 >= k0;
     const bool active_prev = j > 0 && qs0 - 1 >= k0;
@@ -1002,7 +571,11 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
     if constexpr (!DKW) {
       if (active) {
         first_product(x, Qx + qslot * IMG, [](int) { return a_f32x16{}; });
-        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      next();
+      __builtin_amdgcn_sched_barrier(0);
+      if (active) {
         const bool diag = qs0 < k0 + 31;
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -1034,7 +607,7 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
                                            __float_as_uint(x[t][4 * g + 2]), __float_as_uint(x[t][4 * g + 3])};
         }
         __builtin_amdgcn_sched_barrier(0);
-        second(x, dOx + P * IMG, nullptr);
+        second(x, P ? O1 : O0, nullptr);
       }
     } else {
       if (active_prev)  // finish step m-1: dS = P (dP - delta), dK += dS^T Q
@@ -1042,7 +615,7 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
       __builtin_amdgcn_sched_barrier(0);
       if (active) {
         // dP - delta: the accumulator starts at -delta (stored negated)
-        first_product(x, dOx + P * IMG, [&](int t) __attribute__((always_inline)) {
+        first_product(x, P ? O1 : O0, [&](int t) __attribute__((always_inline)) {
           a_f32x16 d;
 #pragma unroll
           for (int g = 0; g < 4; ++g) {
@@ -1058,7 +631,7 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
     }
     __builtin_amdgcn_sched_barrier(0);
     vm_wait_all();  // the next step's rows and statistics have landed
-    if (j + 1 < n && rt < kBQ2) (dkw ? del_s : lse_s)[P ^ 1][rt] = stat_n;
+    if (j + 1 < n && rt < kBQ2) stat_store(P ^ 1, stat_n);
     __syncthreads();  // P(m) handed over; images of step m-1 free
   };
   // each role runs its own copy of the step loop (the same barriers in the
@@ -1109,16 +682,207 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
   }
 }
 
+// ------------------------------------- backward: dK, dV, head dims to 96 --
+// dK and dV of 32 keys per wave in one wave: both accumulators, the K and V
+// fragments and one 32-query tile of S and dP fit 256 registers up to a head
+// dim of 96, so nothing is handed from wave to wave, a workgroup is four
+// independent waves with one barrier per 64 queries, and two workgroups share
+// a CU, one computing probabilities while the other's MFMAs run.  S = Q K^T
+// and dP = dO V^T are computed with lane = key (query rows swizzled), so P and
+// dS are already the A operands of dV += P^T dO and dK += dS^T Q.
+//
+// The Q and dO rows of a step load directly into LDS a step ahead, one image
+// each, double buffered: chunk c (8 columns) of row r at c ^ img_swz(r), which
+// puts both the row reads of the A operands (16 rows, one chunk) and the
+// transposing reads of the B operands (4 rows x 64 bytes per 32 lanes) in
+// distinct banks.  dP's accumulator starts at -delta.
+template <int D, bool FP16, bool PAD>
+__global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dkdv_kernel(AttnArgs a) {
+  static_assert(D == 64 || D == 96, "wider heads run on the paired kernel");
+  constexpr int KS = D / 16, DT = D / 32, CPR = D / 8;
+  constexpr int IMG = kBQ2 * D;             // elements of one image
+  // an array per image, so the compiler can tell the direct loads into one
+  // from the fragment reads of another
+  __shared__ __attribute__((aligned(16))) uint16_t Q0[IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t Q1[IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t O0[IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t O1[IMG];
+  __shared__ __attribute__((aligned(16))) float lse_s[2][kBQ2];
+  __shared__ __attribute__((aligned(16))) float del_s[2][kBQ2];
+
+  const int BH = a.B * a.H;
+  const int bh = blockIdx.x % BH, kb = blockIdx.x / BH;
+  const int b = bh / a.H, h = bh % a.H;
+  const int lane = threadIdx.x & 63, hl = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int k0 = kb * kBKV2 + w * 32;
+  const int key = k0 + (lane & 31);
+
+  ImgCopy<D, PAD> qc, oc;
+  qc.init(a.q, b, h, a.hd, a.S, w, lane);
+  oc.init(a.dout, b, h, a.hd, a.S, w, lane);
+  // per-query statistics: threads 0-63 lse, 64-127 delta (a padding query gets
+  // lse = 1e30, so P = 0); delta is negated when it is stored, not here, where
+  // the use would wait for every load in flight
+  const float* stats = (threadIdx.x < 64 ? a.lse : a.delta) + (int64_t)bh * a.S;
+  const int si = threadIdx.x & 63;
+  auto stat = [&](int qs) __attribute__((always_inline)) {
+    float v = threadIdx.x < 64 ? 1e30f : 0.f;
+    if (!PAD || qs + si < a.S) v = stats[qs + si];
+    return v;
+  };
+  auto stat_store = [&](int p, float v) __attribute__((always_inline)) {
+    if (threadIdx.x < 64)
+      lse_s[p][threadIdx.x] = v;
+    else if (threadIdx.x < 128)
+      del_s[p][threadIdx.x - 64] = -v;
+  };
+  const int first = (kb * kBKV2) / kBQ2, nq = (a.S + kBQ2 - 1) / kBQ2;
+  qc.issue(Q0, first * kBQ2);
+  oc.issue(O0, first * kBQ2);
+  float stat_n = 0.f;
+  if (threadIdx.x < 128) stat_n = stat(first * kBQ2);
+
+  uint4 kf[KS], vf[KS];  // this lane's key: K and V rows, the B operands of S and dP
+  {
+    const uint16_t* kp = row_ptr(a.k, key, b, h);
+    const uint16_t* vp = row_ptr(a.v, key, b, h);
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      kf[ks] = load_row16<PAD>(kp, key < a.S, ks * 16 + hl * 8, a.hd);
+      vf[ks] = load_row16<PAD>(vp, key < a.S, ks * 16 + hl * 8, a.hd);
+    }
+  }
+  a_f32x16 dk[DT], dv[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t) dk[t] = dv[t] = a_f32x16{};
+
+  int aoff[KS], toff[DT][2];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) aoff[ks] = img_row_off<D>(lane, ks);
+#pragma unroll
+  for (int d2 = 0; d2 < DT; ++d2)
+#pragma unroll
+    for (int hi = 0; hi < 2; ++hi) toff[d2][hi] = img_tr_off<D>(lane, d2, hi);
+  auto bfrag = [&](const uint16_t* img, int kk, int d2) __attribute__((always_inline)) {
+    return img_tr(img + kk * 16 * D, toff[d2][0], toff[d2][1]);
+  };
+  vm_wait_all();
+  stat_store(0, stat_n);
+  __syncthreads();
+
+  auto step = [&](int m, auto par_c) __attribute__((always_inline)) {
+    constexpr int P = decltype(par_c)::value;
+    const int qs0 = m * kBQ2;
+    const bool more = m + 1 < nq;
+    if (more) {  // the next step's rows into the other images, a step ahead
+      qc.issue(P ? Q0 : Q1, qs0 + kBQ2);
+      oc.issue(P ? O0 : O1, qs0 + kBQ2);
+      if (threadIdx.x < 128) stat_n = stat(qs0 + kBQ2);
+    }
+    const uint16_t* qi = P ? Q1 : Q0;
+    const uint16_t* oi = P ? O1 : O0;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const int qt = qs0 + t * 32;
+      if (qt + 31 < k0) continue;  // every query of the tile precedes the wave's keys
+      a_f32x16 s = a_f32x16{}, dp;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 d4 = *reinterpret_cast<const float4*>(&del_s[P][t * 32 + swz_row(4 * g, hl)]);
+        dp[4 * g + 0] = d4.x;
+        dp[4 * g + 1] = d4.y;
+        dp[4 * g + 2] = d4.z;
+        dp[4 * g + 3] = d4.w;
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        s = mma<FP16>(*reinterpret_cast<const uint4*>(qi + t * 32 * D + aoff[ks]), kf[ks], s);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks)
+        dp = mma<FP16>(*reinterpret_cast<const uint4*>(oi + t * 32 * D + aoff[ks]), vf[ks], dp);
+      // P; query of register r = qt + swz_row(r, hl); the causal mask only on
+      // the tiles that cross the diagonal
+      auto probs = [&](auto masked) __attribute__((always_inline)) {
+        const int kq = key - qt - 8 * hl;  // masked when > swz_row(r, 0)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 l4 = *reinterpret_cast<const float4*>(&lse_s[P][t * 32 + swz_row(4 * g, hl)]);
+          const float lv[4] = {l4.x, l4.y, l4.z, l4.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int r = 4 * g + e;
+            float p = fast_exp2(__builtin_fmaf(s[r], a.scale_log2, -lv[e]));
+            if (decltype(masked)::value && kq > swz_row(r, 0)) p = 0.f;
+            s[r] = p;
+          }
+        }
+      };
+      if (qt < k0 + 31)
+        probs(std::true_type{});
+      else
+        probs(std::false_type{});
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2) {
+        const int kk = t * 2 + k2, e0 = k2 * 8;
+        const uint4 pa = make_uint4(pack2<FP16>(s[e0 + 0], s[e0 + 1]), pack2<FP16>(s[e0 + 2], s[e0 + 3]),
+                                    pack2<FP16>(s[e0 + 4], s[e0 + 5]), pack2<FP16>(s[e0 + 6], s[e0 + 7]));
+#pragma unroll
+        for (int d2 = 0; d2 < DT; ++d2) dv[d2] = mma<FP16>(pa, bfrag(oi, kk, d2), dv[d2]);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dp[r] = s[r] * dp[r];
+#pragma unroll
+      for (int k2 = 0; k2 < 2; ++k2) {
+        const int kk = t * 2 + k2, e0 = k2 * 8;
+        const uint4 sa = make_uint4(pack2<FP16>(dp[e0 + 0], dp[e0 + 1]), pack2<FP16>(dp[e0 + 2], dp[e0 + 3]),
+                                    pack2<FP16>(dp[e0 + 4], dp[e0 + 5]), pack2<FP16>(dp[e0 + 6], dp[e0 + 7]));
+#pragma unroll
+        for (int d2 = 0; d2 < DT; ++d2) dk[d2] = mma<FP16>(sa, bfrag(qi, kk, d2), dk[d2]);
+      }
+    }
+    vm_wait_all();  // the next step's rows and statistics have landed
+    if (more) stat_store(P ^ 1, stat_n);
+    __syncthreads();  // this step's images free, the next step's visible
+  };
+  int m = first;
+  for (; m + 1 < nq; m += 2) {
+    step(m, std::integral_constant<int, 0>{});
+    step(m + 1, std::integral_constant<int, 1>{});
+  }
+  if (m < nq) step(m, std::integral_constant<int, 0>{});
+
+  // out through LDS in 16-byte row chunks: lane holds d = t*32 + lane%32 for
+  // keys acc_row(r, hl); dV by way of the dO images, dK of the Q images
+  static_assert(2 * 32 * D <= IMG, "two waves' staging fits an image");
+  uint16_t* sv = (w < 2 ? O0 : O1) + (w & 1) * 32 * D;
+  uint16_t* sk = (w < 2 ? Q0 : Q1) + (w & 1) * 32 * D;
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int o = acc_row(r, hl) * D + t * 32 + (lane & 31);
+      sv[o] = from_f<FP16>(dv[t][r]);
+      sk[o] = from_f<FP16>(dk[t][r] * a.scale);
+    }
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): a wave reads back only its own rows
+#pragma unroll
+  for (int i = 0; i < 32 * CPR / 64; ++i) {
+    const int c = i * 64 + lane, kr = c / CPR, col = (c % CPR) * 8;
+    if (PAD && (k0 + kr >= a.S || col >= a.hd)) continue;
+    *reinterpret_cast<uint4*>(row_ptr(a.dv, k0 + kr, b, h) + col) = *reinterpret_cast<const uint4*>(sv + kr * D + col);
+    *reinterpret_cast<uint4*>(row_ptr(a.dk, k0 + kr, b, h) + col) = *reinterpret_cast<const uint4*>(sk + kr * D + col);
+  }
+}
+
 // ------------------------------------------------------------ backward: dQ --
 template <int D, bool FP16, bool PAD>
 __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a) {
   constexpr int KS = D / 16, DT = D / 32;
-  // K and V rows swizzled for S^T and dP^T; K also in natural order, padded
-  // to D + 32, for the transposing reads of dQ^T = K^T dS^T
-  constexpr int KN = tr_row(D);
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[kBKV * (D + 8)];
-  __shared__ __attribute__((aligned(16))) uint16_t Vs[kBKV * (D + 8)];
-  __shared__ __attribute__((aligned(16))) uint16_t Kn[kBKV * KN];
+  __shared__ __attribute__((aligned(16))) uint16_t K0[kBKV * D];
+  __shared__ __attribute__((aligned(16))) uint16_t K1[kBKV * D];
+  __shared__ __attribute__((aligned(16))) uint16_t V0[kBKV * D];
+  __shared__ __attribute__((aligned(16))) uint16_t V1[kBKV * D];
 
   const int BH = a.B * a.H, nqb = (a.S + kBQ - 1) / kBQ;
   const int bh = blockIdx.x % BH, qb = nqb - 1 - blockIdx.x / BH;
@@ -1127,6 +891,13 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
   const int q0 = qb * kBQ + w * 32;
   const int q = q0 + (lane & 31);
+
+  ImgCopy<D, PAD> kc, vc;
+  kc.init(a.k, b, h, a.hd, a.S, w, lane);
+  vc.init(a.v, b, h, a.hd, a.S, w, lane);
+  const int nkv = (qb * kBQ + kBQ) / kBKV;
+  kc.issue(K0, 0);
+  vc.issue(V0, 0);
 
   const bool real = !PAD || q < a.S;  // false on padding rows of the last block
   uint4 qf[KS], of[KS];
@@ -1166,51 +937,49 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a
 #pragma unroll
     for (int r = 0; r < 16; ++r) dq[t][r] = 0.f;
 
-  BufTile<kBKV, D, D + 8, true, PAD> kt, vt;
-  kt.init(a.k, b, h, a.S, a.hd);
-  vt.init(a.v, b, h, a.S, a.hd);
-  const int ktr = tr_lane(lane, KN);
-  const int nkv = (qb * kBQ + kBQ) / kBKV;
-  // the next block's K / V rows are loaded while this block computes
-  kt.load(0);
-  vt.load(0);
-  for (int j = 0; j < nkv; ++j) {
+  int aoff[KS], toff[DT][2];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) aoff[ks] = img_row_off<D>(lane, ks);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int hi = 0; hi < 2; ++hi) toff[dt][hi] = img_tr_off<D>(lane, dt, hi);
+  vm_wait_all();
+  __syncthreads();
+
+  auto block = [&](int j, auto cur_c) __attribute__((always_inline)) {
+    constexpr int cur = decltype(cur_c)::value;
     const int kv0 = j * kBKV;
-    __syncthreads();
-    kt.store(Ks);
-    kt.template store_natural<KN>(Kn);
-    vt.store(Vs);
-    __syncthreads();
-    if (j + 1 < nkv) {
-      kt.load(kv0 + kBKV);
-      vt.load(kv0 + kBKV);
+    if (j + 1 < nkv) {  // the next block, a block ahead
+      kc.issue(cur ? K0 : K1, kv0 + kBKV);
+      vc.issue(cur ? V0 : V1, kv0 + kBKV);
     }
-    if (kv0 > q0 + 31) continue;
-    const bool diag = kv0 + kBKV - 1 > q0;
+    const uint16_t* ki = cur ? K1 : K0;
+    const uint16_t* vi = cur ? V1 : V0;
     // one 32-key tile at a time: S^T = K Q^T, dP^T = V dO^T (lane = query),
     // dS^T, then dQ^T += K^T dS^T over those 32 keys
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
+      const int kt0 = kv0 + t * 32;
+      if (kt0 > q0 + 31) continue;  // every key of the tile follows the wave's queries
       a_f32x16 s, dp;
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
-      const uint16_t* kp = Ks + (t * 32 + (lane & 31)) * (D + 8) + hl * 8;
-      const uint16_t* vp = Vs + (t * 32 + (lane & 31)) * (D + 8) + hl * 8;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        s = mma<FP16>(*reinterpret_cast<const uint4*>(kp + ks * 16), qf[ks], s);
-        dp = mma<FP16>(*reinterpret_cast<const uint4*>(vp + ks * 16), of[ks], dp);
+        s = mma<FP16>(*reinterpret_cast<const uint4*>(ki + t * 32 * D + aoff[ks]), qf[ks], s);
+        dp = mma<FP16>(*reinterpret_cast<const uint4*>(vi + t * 32 * D + aoff[ks]), of[ks], dp);
       }
-      // causal mask only on the blocks that cross the diagonal (see dK/dV)
+      // causal mask only on the tiles that cross the diagonal
       auto dsoft = [&](auto masked) __attribute__((always_inline)) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           float p = fast_exp2(__builtin_fmaf(s[r], a.scale_log2, -lse));
-          if (decltype(masked)::value && kv0 + t * 32 + swz_row(r, hl) > q) p = 0.f;
+          if (decltype(masked)::value && kt0 + swz_row(r, hl) > q) p = 0.f;
           dp[r] = p * (dp[r] - del);
         }
       };
-      if (diag)
+      if (kt0 + 31 > q0)
         dsoft(std::true_type{});
       else
         dsoft(std::false_type{});
@@ -1219,12 +988,20 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a
         const int kk = t * 2 + k2, e0 = k2 * 8;
         const uint4 sb = make_uint4(pack2<FP16>(dp[e0 + 0], dp[e0 + 1]), pack2<FP16>(dp[e0 + 2], dp[e0 + 3]),
                                     pack2<FP16>(dp[e0 + 4], dp[e0 + 5]), pack2<FP16>(dp[e0 + 6], dp[e0 + 7]));
-        const uint16_t* ktp = Kn + ktr + kk * 16 * KN;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) dq[dt] = mma<FP16>(tr_frag(ktp + dt * 32, KN), sb, dq[dt]);
+        for (int dt = 0; dt < DT; ++dt)
+          dq[dt] = mma<FP16>(img_tr(ki + kk * 16 * D, toff[dt][0], toff[dt][1]), sb, dq[dt]);
       }
     }
+    vm_wait_all();  // the next block's rows have landed
+    __syncthreads();  // this block's images free, the next block's visible
+  };
+  int j = 0;
+  for (; j + 1 < nkv; j += 2) {
+    block(j, std::integral_constant<int, 0>{});
+    block(j + 1, std::integral_constant<int, 1>{});
   }
+  if (j < nkv) block(j, std::integral_constant<int, 0>{});
   if (PAD && !real) return;
   uint16_t* dqp = row_ptr(a.dq, q, b, h);
 #pragma unroll
@@ -1273,6 +1050,16 @@ static AttnOut tout(void* p, const int64_t* st) {
   return t;
 }
 
+// dQ first: it also writes delta, which dK/dV reads
+template <int D, bool FP16, bool PAD>
+static void launch_bwd(const AttnArgs& a, int g_q, int g_kv, hipStream_t s) {
+  attn_bwd_dq_kernel<D, FP16, PAD><<<g_q, kAttnThreads, 0, s>>>(a);
+  if constexpr (D == 128)
+    attn_bwd_dkdv_x128_kernel<FP16, PAD><<<g_kv, 2 * kAttnThreads, 0, s>>>(a);
+  else
+    attn_bwd_dkdv_kernel<D, FP16, PAD><<<g_kv, kAttnThreads, 0, s>>>(a);
+}
+
 static bool aligned_rows(const void* p, const int64_t* st) {
   return ((uintptr_t)p & 15) == 0 && st[0] % 8 == 0 && st[1] % 8 == 0 && st[2] % 8 == 0;
 }
@@ -1312,13 +1099,7 @@ extern "C" int eth_attn_fwd(const eth_attn_desc_t* d, const void* q, const void*
     else attn_fwd_kernel<D, false, false><<<grid, kAttnThreads, 0, s>>>(a);            \
   }
   if (a.hd > 96) {
-    if (pad) {
-      if (fp16) attn_fwd_x128_kernel<true, true><<<grid, kAttnThreads, 0, s>>>(a);
-      else attn_fwd_x128_kernel<false, true><<<grid, kAttnThreads, 0, s>>>(a);
-    } else {
-      if (fp16) attn_fwd_x128_kernel<true, false><<<grid, kAttnThreads, 0, s>>>(a);
-      else attn_fwd_x128_kernel<false, false><<<grid, kAttnThreads, 0, s>>>(a);
-    }
+    ETH_ATTN_FWD(128)
   } else if (a.hd > 64) {
     ETH_ATTN_FWD(96)
   } else {
@@ -1366,18 +1147,11 @@ extern "C" int eth_attn_bwd(const eth_attn_desc_t* d, const void* q, const void*
   const int width = a.hd > 96 ? 128 : a.hd > 64 ? 96 : 64;
   static_assert(kBKV2 == kBQ, "one padding rule for the three backward kernels");
   const bool pad = a.S % kBKV2 != 0 || a.hd != width;
-#define ETH_ATTN_BWD_P(D, F, P)                                                    \
-  attn_bwd_dq_kernel<D, F, P><<<g_q, kAttnThreads, 0, s>>>(a);                   \
-  if constexpr (D == 128)                                                         \
-    attn_bwd_dkdv_x128_kernel<F, P><<<g_kv, 2 * kAttnThreads, 0, s>>>(a);         \
-  else                                                                            \
-    attn_bwd_dkdv_pair_kernel<D, F, P><<<g_kv, 2 * kAttnThreads, 0, s>>>(a);
-#define ETH_ATTN_BWD(D, F)        \
-  if (pad) {                      \
-    ETH_ATTN_BWD_P(D, F, true)    \
-  } else {                        \
-    ETH_ATTN_BWD_P(D, F, false)   \
-  }
+#define ETH_ATTN_BWD(D, F)                          \
+  if (pad)                                          \
+    launch_bwd<D, F, true>(a, g_q, g_kv, s);        \
+  else                                              \
+    launch_bwd<D, F, false>(a, g_q, g_kv, s);
   if (a.hd > 96) {
     if (fp16) { ETH_ATTN_BWD(128, true) } else { ETH_ATTN_BWD(128, false) }
   } else if (a.hd > 64) {
@@ -1386,7 +1160,6 @@ extern "C" int eth_attn_bwd(const eth_attn_desc_t* d, const void* q, const void*
     if (fp16) { ETH_ATTN_BWD(64, true) } else { ETH_ATTN_BWD(64, false) }
   }
 #undef ETH_ATTN_BWD
-#undef ETH_ATTN_BWD_P
   ETH_CHECK_LAUNCH("eth_attn_bwd");
   return ETH_OK;
 }
