@@ -124,15 +124,16 @@ __global__ void __launch_bounds__(kEwThreads) bda_fwd_kernel(const uint16_t* __r
     const uint16_t* be = reinterpret_cast<const uint16_t*>(&br);
     uint4 o;
     uint16_t* oe = reinterpret_cast<uint16_t*>(&o);
+    float t[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      float t = cin<FP16>(cout<FP16>(cin<FP16>(xe[j]) + cin<FP16>(be[j])));
-      if (thresh) {
-        const bool keep = hash_u32(seed, (uint64_t)v * 8 + j) >= thresh;
-        t = cin<FP16>(cout<FP16>(keep ? t * keep_scale : 0.f));
-      }
-      oe[j] = cout<FP16>(cin<FP16>(re[j]) + t);
+    for (int j = 0; j < 8; ++j) t[j] = cin<FP16>(cout<FP16>(cin<FP16>(xe[j]) + cin<FP16>(be[j])));
+    if (thresh) {
+      dropout8(t, seed, (uint64_t)v * 8, thresh, keep_scale);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) t[j] = cin<FP16>(cout<FP16>(t[j]));
     }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) oe[j] = cout<FP16>(cin<FP16>(re[j]) + t[j]);
     reinterpret_cast<uint4*>(out)[v] = o;
   }
 }
@@ -148,11 +149,12 @@ __global__ void __launch_bounds__(kEwThreads) dropout_bwd_kernel(const uint16_t*
     const uint16_t* de = reinterpret_cast<const uint16_t*>(&dr);
     uint4 o;
     uint16_t* oe = reinterpret_cast<uint16_t*>(&o);
+    float t[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const bool keep = hash_u32(seed, (uint64_t)v * 8 + j) >= thresh;
-      oe[j] = cout<FP16>(keep ? cin<FP16>(de[j]) * keep_scale : 0.f);
-    }
+    for (int j = 0; j < 8; ++j) t[j] = cin<FP16>(de[j]);
+    dropout8(t, seed, (uint64_t)v * 8, thresh, keep_scale);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) oe[j] = cout<FP16>(t[j]);
     reinterpret_cast<uint4*>(dx)[v] = o;
   }
 }

@@ -147,14 +147,17 @@ __global__ void __launch_bounds__(64 * kLnWaves) bda_ln_fwd_kernel(
       const uint16_t* be = reinterpret_cast<const uint16_t*>(&br);
       uint4 hr;
       uint16_t* he = reinterpret_cast<uint16_t*>(&hr);
+      float t[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) t[j] = cvt_in<FP16>(cvt_out<FP16>(cvt_in<FP16>(xe[j]) + cvt_in<FP16>(be[j])));
+      if (thresh) {
+        dropout8(t, seed, (uint64_t)(base + c), thresh, keep_scale);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) t[j] = cvt_in<FP16>(cvt_out<FP16>(t[j]));
+      }
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        float t = cvt_in<FP16>(cvt_out<FP16>(cvt_in<FP16>(xe[j]) + cvt_in<FP16>(be[j])));
-        if (thresh) {
-          const bool keep = hash_u32(seed, (uint64_t)(base + c + j)) >= thresh;
-          t = cvt_in<FP16>(cvt_out<FP16>(keep ? t * keep_scale : 0.f));
-        }
-        he[j] = cvt_out<FP16>(cvt_in<FP16>(re[j]) + t);
+        he[j] = cvt_out<FP16>(cvt_in<FP16>(re[j]) + t[j]);
         v[i][j] = cvt_in<FP16>(he[j]);
         s += v[i][j];
       }
