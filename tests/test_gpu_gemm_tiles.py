@@ -145,6 +145,10 @@ def test_deep_product_takes_splits(cuda):
     assert splits == 16 and K._splitk_pays(M, N, Kd, splits, 1, 0)
     assert not K._splitk_pays(M, N, Kd + 8, splits, 1, 0) and not K._splitk_pays(M, N, Kd, splits, 0, 1)
     assert not K._splitk_pays(2048, 2048, 2048, 2, 1, 1)
+    # half a round of wide tiles splits in two, one tile more does not
+    half = torch.empty(2048, 4096, dtype=torch.bfloat16, device=cuda)
+    assert K._splitk_splits(2048, 4096, 16384, half) == 2 and K._splitk_pays(2048, 4096, 16384, 2, 1, 1)
+    assert K._splitk_splits(2049, 4096, 16384, half) == 1
     a, b, ad, bd = _operands(M, N, Kd, True, False, torch.bfloat16, cuda, 5)
     got = K.gemm(ad, bd)
     _check(got, a @ b, a.abs() @ b.abs(), Kd, torch.bfloat16, "deep")
