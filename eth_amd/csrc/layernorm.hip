@@ -205,12 +205,12 @@ __global__ void __launch_bounds__(64 * kLnWaves) bda_ln_fwd_kernel(
 }
 
 // Backward.  A workgroup of kLnBwdWaves waves owns rows g, g + G, g + 2G, ...;
-// T waves share a row (T = 1 up to 1024 columns, 2 up to 2048, 4 up to
-// 4096, 8 up to 8192), each covering NVW <= 2 vectors of 512 columns (the
+// T waves share a row, each covering NVW <= 3 vectors of 512 columns (the
 // per-lane state then fits the 256 registers of two waves per SIMD without
-// spilling), so a group of T waves
-// ("team") handles one row per iteration and the workgroup kLnBwdWaves / T
-// rows.  The next row's x / dy / dresid are loaded while the current one is
+// spilling): (T, NVW) = (1, 1) up to 512 columns, (1, 2) up to 1024, (2, 2)
+// up to 2048, (4, 2) up to 4096, (8, 2) up to 8192, and (2, 3) up to 3072 and
+// (4, 3) up to 6144 where the rows are many (ln_bwd_three).  A group of T waves ("team") handles one row per iteration and the workgroup
+// kLnBwdWaves / T rows.  The next row's x / dy / dresid are loaded while the current one is
 // computed.  Per lane fp32 column sums of dy * xhat (dgamma), dy (dbeta) and,
 // with CSUM, of the stored dx (the bias gradient of the bias-dropout-add whose
 // output this LayerNorm normalised) stay in registers for all of the group's
@@ -393,13 +393,22 @@ __global__ void __launch_bounds__(64 * kLnBwdWaves) ln_bwd_kernel(
   }
 }
 
+// Widths that three vectors per wave cover with fewer idle lanes than two:
+// from 384 rows on.  The third vector lengthens the closing fold of the column
+// sums, which is most of a shorter launch (us, two / three vectors, with
+// residual and column sums: [64, 2240] 8.7 / 9.5, [512, 2240] 11.6 / 10.8,
+// [8192, 2560] 44 / 37, [4096, 5120] 45 / 38).
+inline bool ln_bwd_three(int64_t rows, int64_t cols) {
+  return rows >= 384 && ((cols > 2048 && cols <= 3072) || (cols > 4096 && cols <= 6144));
+}
 // Row groups of the backward: at most 256 workgroups (one per CU), each with
 // at least one row per team.
-inline int ln_bwd_team_waves(int64_t cols) {
-  return cols <= 1024 ? 1 : (cols <= 2048 ? 2 : (cols <= 4096 ? 4 : 8));
+inline int ln_bwd_team_waves(int64_t rows, int64_t cols) {
+  const int t = cols <= 1024 ? 1 : (cols <= 2048 ? 2 : (cols <= 4096 ? 4 : 8));
+  return ln_bwd_three(rows, cols) ? t / 2 : t;
 }
 inline int ln_bwd_groups(int64_t rows, int64_t cols) {
-  const int64_t teams = kLnBwdWaves / ln_bwd_team_waves(cols);
+  const int64_t teams = kLnBwdWaves / ln_bwd_team_waves(rows, cols);
   int64_t g = (rows + teams - 1) / teams;
   if (g > 256) g = 256;
   if (g < 1) g = 1;
@@ -453,6 +462,8 @@ static void launch_bwd(const uint16_t* dy, const uint16_t* x, const float* mean,
   if (nv == 1) ETH_LN_BWD(1, 1);
   else if (nv == 2) ETH_LN_BWD(1, 2);
   else if (nv <= 4) ETH_LN_BWD(2, 2);
+  else if (ln_bwd_three(rows, cols) && nv <= 6) ETH_LN_BWD(2, 3);
+  else if (ln_bwd_three(rows, cols)) ETH_LN_BWD(4, 3);
   else if (nv <= 8) ETH_LN_BWD(4, 2);
   else ETH_LN_BWD(8, 2);
 #undef ETH_LN_BWD
