@@ -18,7 +18,7 @@
 // lane owns one query (MFMA column) and 32 of the 64 keys of a block sit in
 // its registers: row max / row sum need one cross-lane exchange (lane ^ 32),
 // and the per-query softmax statistics are per-lane scalars.  K rows are
-// stored in LDS with bits 2 and 3 of the row index swapped, which makes the
+// read from LDS with bits 2 and 3 of the row index swapped, which makes the
 // MFMA result layout of S^T equal to the operand layout of P^T in
 // O^T = V^T P^T, so P never leaves registers.  The dK/dV kernel uses the
 // mirror image (S = Q K^T, lane = key, query rows swizzled) and computes S
@@ -27,11 +27,18 @@
 // results are deterministic.  The dQ kernel runs first and also writes
 // delta = rowsum(dO * O), which the dK/dV kernel reads.
 //
-// Tiles arrive through buffer loads (fixed per-thread offsets, a scalar row
-// advance).  Operands that an MFMA needs transposed (V for O^T = V^T P^T, K
-// for dQ^T = K^T dS^T, Q and dO for dK and dV) are kept in LDS in natural
-// row order, padded to D + 32 so four k-rows fall in distinct banks, and
-// read with ds_read_b64_tr_b16.  Softmax runs in fp32 base-2 (exp2) with the scale folded.
+// Tiles load directly from global memory into swizzled LDS images (fixed
+// per-thread offsets, a scalar row advance).  Operands that an MFMA needs
+// transposed (V for O^T = V^T P^T, K for dQ^T = K^T dS^T, Q and dO for dK and
+// dV) are read from the same images with ds_read_b64_tr_b16.  Softmax runs in
+// fp32 base-2 (exp2) with the scale folded.
+//
+// Forward / backward alone, against kernels that staged the 64- and 96-wide
+// tiles through registers into padded copies (us): 4096 x 2 x 16 heads of 64
+// 97 / 321 -> 90 / 262, 1500 x 2 x 32 of 80 49 / 175 -> 47 / 142, 2048 x 4 x 16
+// of 128 85 / 289 -> 84 / 272, 2048 x 1 x 16 of 128 50 / 124 -> 41 / 114.
+// Bound by a wave's own VALU work (5.5 instructions per forward MFMA, one of
+// them an exponential), which runs in series with its MFMAs.
 #include <type_traits>
 
 #include "common.h"
