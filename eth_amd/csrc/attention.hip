@@ -226,20 +226,29 @@ __device__ __forceinline__ uint4 img_tr(const uint16_t* p, int lo_off, int hi_of
 // 4 waves x 32 queries; K/V blocks of 64 keys in double-buffered images, one
 // barrier per block; two workgroups per CU, so one wave's softmax overlaps
 // another's MFMAs.
-template <int D, bool FP16, bool PAD>
-__global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_kernel(AttnArgs a) {
+//
+// G = 2: two such groups of waves in a workgroup take alternate key blocks of
+// the same queries, each with images of its own, and the first adds the
+// second's sums through LDS at the end.  A query block is a chain of up to
+// seq / 64 steps, so a grid that leaves half of the CUs' wave slots empty
+// takes as long as its longest chain: this halves it (attn_groups).
+static_assert(kBQ % (2 * kBKV) == 0, "both groups take the same number of key blocks");
+template <int D, bool FP16, bool PAD, int G>
+__global__ void __launch_bounds__(G * kAttnThreads, 2) attn_fwd_kernel(AttnArgs a) {
   constexpr int KS = D / 16;  // k-steps over the head dim
   constexpr int DT = D / 32;  // 32-row tiles over the head dim
-  __shared__ __attribute__((aligned(16))) uint16_t K0[kBKV * D];
-  __shared__ __attribute__((aligned(16))) uint16_t K1[kBKV * D];
-  __shared__ __attribute__((aligned(16))) uint16_t V0[kBKV * D];
-  __shared__ __attribute__((aligned(16))) uint16_t V1[kBKV * D];
+  constexpr int IMG = kBKV * D;  // elements of one image
+  __shared__ __attribute__((aligned(16))) uint16_t K0[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t K1[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t V0[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t V1[G * IMG];
 
   const int BH = a.B * a.H, nqb = (a.S + kBQ - 1) / kBQ;
   const int bh = blockIdx.x % BH, qb = nqb - 1 - blockIdx.x / BH;
   const int b = bh / a.H, h = bh % a.H;
   const int lane = threadIdx.x & 63, hl = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int w = wid & 3, grp = G == 1 ? 0 : wid >> 2;
   const int q0 = qb * kBQ + w * 32;
   const int q = q0 + (lane & 31);
   const float sl2 = a.scale_log2;
@@ -247,9 +256,9 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_kernel(AttnArgs a) {
   ImgCopy<D, PAD> kc, vc;
   kc.init(a.k, b, h, a.hd, a.S, w, lane);
   vc.init(a.v, b, h, a.hd, a.S, w, lane);
-  const int nkv = (qb * kBQ + kBQ) / kBKV;  // blocks up to the diagonal
-  kc.issue(K0, 0);
-  vc.issue(V0, 0);
+  const int nkv = (qb * kBQ + kBQ) / kBKV / G;  // a group's blocks up to the diagonal
+  kc.issue(K0 + grp * IMG, grp * kBKV);
+  vc.issue(V0 + grp * IMG, grp * kBKV);
 
   uint4 qf[KS];
   {
@@ -276,14 +285,14 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_kernel(AttnArgs a) {
 
   auto block = [&](int j, auto cur_c) __attribute__((always_inline)) {
     constexpr int cur = decltype(cur_c)::value;
-    const int kv0 = j * kBKV;
-    if (j + 1 < nkv) {  // the next block, a block ahead
-      kc.issue(cur ? K0 : K1, kv0 + kBKV);
-      vc.issue(cur ? V0 : V1, kv0 + kBKV);
+    const int kv0 = (j * G + grp) * kBKV;
+    if (j + 1 < nkv) {  // the group's next block, a block ahead
+      kc.issue((cur ? K0 : K1) + grp * IMG, kv0 + G * kBKV);
+      vc.issue((cur ? V0 : V1) + grp * IMG, kv0 + G * kBKV);
     }
     if (kv0 <= q0 + 31) {  // wave has at least one unmasked key in the block
-      const uint16_t* ki = cur ? K1 : K0;
-      const uint16_t* vi = cur ? V1 : V0;
+      const uint16_t* ki = (cur ? K1 : K0) + grp * IMG;
+      const uint16_t* vi = (cur ? V1 : V0) + grp * IMG;
       // S^T = K Q^T (raw scores; lane = query, registers = 32 of the keys)
       a_f32x16 sc[2];
       // all K fragments of the first 32-key tile are read before its MFMAs,
@@ -364,6 +373,35 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_fwd_kernel(AttnArgs a) {
   }
   if (j < nkv) block(j, std::integral_constant<int, 0>{});
   l += __shfl_xor(l, 32, 64);
+  if constexpr (G == 2) {
+    // (the images are free: every group passed the last block's barrier)
+    float4* so = reinterpret_cast<float4*>(w < 2 ? K0 : K1) + (w & 1) * (DT * 4 * 64) + lane;
+    float2* sml = reinterpret_cast<float2*>(V0) + w * 64 + lane;
+    if (grp == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          so[(t * 4 + g) * 64] = make_float4(o[t][g * 4], o[t][g * 4 + 1], o[t][g * 4 + 2], o[t][g * 4 + 3]);
+      *sml = make_float2(m, l);
+    }
+    __syncthreads();
+    if (grp == 1) return;
+    const float2 ml = *sml;
+    const float mn = fmaxf(m, ml.x), f0 = fast_exp2(m - mn), f1 = fast_exp2(ml.x - mn);
+    m = mn;
+    l = l * f0 + ml.y * f1;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 u = so[(t * 4 + g) * 64];
+        o[t][g * 4 + 0] = o[t][g * 4 + 0] * f0 + u.x * f1;
+        o[t][g * 4 + 1] = o[t][g * 4 + 1] * f0 + u.y * f1;
+        o[t][g * 4 + 2] = o[t][g * 4 + 2] * f0 + u.z * f1;
+        o[t][g * 4 + 3] = o[t][g * 4 + 3] * f0 + u.w * f1;
+      }
+  }
   if (PAD && q >= a.S) return;  // a padding row of the last query block
   const float inv = 1.0f / l;
   uint16_t* op = row_ptr(a.out, q, b, h);
@@ -883,28 +921,31 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dkdv_kernel(AttnArgs
 }
 
 // ------------------------------------------------------------ backward: dQ --
-template <int D, bool FP16, bool PAD>
-__global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a) {
+// G = 2 as in the forward.
+template <int D, bool FP16, bool PAD, int G>
+__global__ void __launch_bounds__(G * kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a) {
   constexpr int KS = D / 16, DT = D / 32;
-  __shared__ __attribute__((aligned(16))) uint16_t K0[kBKV * D];
-  __shared__ __attribute__((aligned(16))) uint16_t K1[kBKV * D];
-  __shared__ __attribute__((aligned(16))) uint16_t V0[kBKV * D];
-  __shared__ __attribute__((aligned(16))) uint16_t V1[kBKV * D];
+  constexpr int IMG = kBKV * D;  // elements of one image
+  __shared__ __attribute__((aligned(16))) uint16_t K0[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t K1[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t V0[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t V1[G * IMG];
 
   const int BH = a.B * a.H, nqb = (a.S + kBQ - 1) / kBQ;
   const int bh = blockIdx.x % BH, qb = nqb - 1 - blockIdx.x / BH;
   const int b = bh / a.H, h = bh % a.H;
   const int lane = threadIdx.x & 63, hl = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int w = wid & 3, grp = G == 1 ? 0 : wid >> 2;
   const int q0 = qb * kBQ + w * 32;
   const int q = q0 + (lane & 31);
 
   ImgCopy<D, PAD> kc, vc;
   kc.init(a.k, b, h, a.hd, a.S, w, lane);
   vc.init(a.v, b, h, a.hd, a.S, w, lane);
-  const int nkv = (qb * kBQ + kBQ) / kBKV;
-  kc.issue(K0, 0);
-  vc.issue(V0, 0);
+  const int nkv = (qb * kBQ + kBQ) / kBKV / G;
+  kc.issue(K0 + grp * IMG, grp * kBKV);
+  vc.issue(V0 + grp * IMG, grp * kBKV);
 
   const bool real = !PAD || q < a.S;  // false on padding rows of the last block
   uint4 qf[KS], of[KS];
@@ -936,7 +977,7 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a
       }
     }
     del += __shfl_xor(del, 32, 64);
-    if (hl == 0 && real) a.delta[(int64_t)bh * a.S + q] = del;
+    if (grp == 0 && hl == 0 && real) a.delta[(int64_t)bh * a.S + q] = del;
   }
   a_f32x16 dq[DT];
 #pragma unroll
@@ -956,13 +997,13 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a
 
   auto block = [&](int j, auto cur_c) __attribute__((always_inline)) {
     constexpr int cur = decltype(cur_c)::value;
-    const int kv0 = j * kBKV;
-    if (j + 1 < nkv) {  // the next block, a block ahead
-      kc.issue(cur ? K0 : K1, kv0 + kBKV);
-      vc.issue(cur ? V0 : V1, kv0 + kBKV);
+    const int kv0 = (j * G + grp) * kBKV;
+    if (j + 1 < nkv) {  // the group's next block, a block ahead
+      kc.issue((cur ? K0 : K1) + grp * IMG, kv0 + G * kBKV);
+      vc.issue((cur ? V0 : V1) + grp * IMG, kv0 + G * kBKV);
     }
-    const uint16_t* ki = cur ? K1 : K0;
-    const uint16_t* vi = cur ? V1 : V0;
+    const uint16_t* ki = (cur ? K1 : K0) + grp * IMG;
+    const uint16_t* vi = (cur ? V1 : V0) + grp * IMG;
     // one 32-key tile at a time: S^T = K Q^T, dP^T = V dO^T (lane = query),
     // dS^T, then dQ^T += K^T dS^T over those 32 keys
 #pragma unroll
@@ -1009,6 +1050,29 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a
     block(j + 1, std::integral_constant<int, 1>{});
   }
   if (j < nkv) block(j, std::integral_constant<int, 0>{});
+  if constexpr (G == 2) {
+    // (the images are free: every group passed the last block's barrier)
+    float4* sq = reinterpret_cast<float4*>(w < 2 ? K0 : K1) + (w & 1) * (DT * 4 * 64) + lane;
+    if (grp == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          sq[(t * 4 + g) * 64] = make_float4(dq[t][g * 4], dq[t][g * 4 + 1], dq[t][g * 4 + 2], dq[t][g * 4 + 3]);
+    }
+    __syncthreads();
+    if (grp == 1) return;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 u = sq[(t * 4 + g) * 64];
+        dq[t][g * 4 + 0] += u.x;
+        dq[t][g * 4 + 1] += u.y;
+        dq[t][g * 4 + 2] += u.z;
+        dq[t][g * 4 + 3] += u.w;
+      }
+  }
   if (PAD && !real) return;
   uint16_t* dqp = row_ptr(a.dq, q, b, h);
 #pragma unroll
@@ -1057,10 +1121,35 @@ static AttnOut tout(void* p, const int64_t* st) {
   return t;
 }
 
+// Groups of four waves that share a query block of the forward and dQ: two
+// where one group per block leaves wave slots empty, from the start (up to one
+// workgroup per CU) or once the short chains of a grid of up to two have
+// ended, and the chain is long enough to pay for the second group's start and
+// the closing addition.  Measured on both sides of the lines, forward /
+// backward with dK and dV, one group -> two (us; workgroups, sequence x head
+// dim): 256, 2048 x 128 42.1 / 115.8 -> 36.5 / 106.7; 128, 1024 x 64 16.1 /
+// 44.3 -> 14.3 / 41.7; 84, 777 x 96 15.9 / 53.1 -> 15.0 / 51.1; 64, 512 x 64
+// 12.3 / 26.0 -> 12.1 / 25.5; 48, 300 x 96 12.3 / 27.4 -> 12.5 / 27.7; 512,
+// 4096 x 128 94.3 / 274 -> 87.0 / 256; 384, 1500 x 80 31.8 / 104 -> 28.0 / 101;
+// 384, 1024 x 128 28.9 / 79.8 -> 29.8 / 80.8; 512, 512 x 64 14.1 / 35.8 -> 15.9
+// / 40.8; 768, 1500 x 80 50.7 / 140 -> 54.3 / 149.
+static int attn_groups(int grid, int seq) { return seq > (grid <= 256 ? 512 : 1024) && grid <= 512 ? 2 : 1; }
+
+template <int D, bool FP16, bool PAD>
+static void launch_fwd(const AttnArgs& a, int grid, hipStream_t s) {
+  if (attn_groups(grid, a.S) == 2)
+    attn_fwd_kernel<D, FP16, PAD, 2><<<grid, 2 * kAttnThreads, 0, s>>>(a);
+  else
+    attn_fwd_kernel<D, FP16, PAD, 1><<<grid, kAttnThreads, 0, s>>>(a);
+}
+
 // dQ first: it also writes delta, which dK/dV reads
 template <int D, bool FP16, bool PAD>
 static void launch_bwd(const AttnArgs& a, int g_q, int g_kv, hipStream_t s) {
-  attn_bwd_dq_kernel<D, FP16, PAD><<<g_q, kAttnThreads, 0, s>>>(a);
+  if (attn_groups(g_q, a.S) == 2)
+    attn_bwd_dq_kernel<D, FP16, PAD, 2><<<g_q, 2 * kAttnThreads, 0, s>>>(a);
+  else
+    attn_bwd_dq_kernel<D, FP16, PAD, 1><<<g_q, kAttnThreads, 0, s>>>(a);
   if constexpr (D == 128)
     attn_bwd_dkdv_x128_kernel<FP16, PAD><<<g_kv, 2 * kAttnThreads, 0, s>>>(a);
   else
@@ -1097,20 +1186,17 @@ extern "C" int eth_attn_fwd(const eth_attn_desc_t* d, const void* q, const void*
   const int width = a.hd > 96 ? 128 : a.hd > 64 ? 96 : 64;
   // full blocks (every row and head-dim column real) take the unguarded kernels
   const bool pad = a.S % kBQ != 0 || a.hd != width;
-#define ETH_ATTN_FWD(D)                                                                \
-  if (pad) {                                                                           \
-    if (fp16) attn_fwd_kernel<D, true, true><<<grid, kAttnThreads, 0, s>>>(a);         \
-    else attn_fwd_kernel<D, false, true><<<grid, kAttnThreads, 0, s>>>(a);             \
-  } else {                                                                             \
-    if (fp16) attn_fwd_kernel<D, true, false><<<grid, kAttnThreads, 0, s>>>(a);        \
-    else attn_fwd_kernel<D, false, false><<<grid, kAttnThreads, 0, s>>>(a);            \
-  }
+#define ETH_ATTN_FWD(D, F)                   \
+  if (pad)                                   \
+    launch_fwd<D, F, true>(a, grid, s);      \
+  else                                       \
+    launch_fwd<D, F, false>(a, grid, s);
   if (a.hd > 96) {
-    ETH_ATTN_FWD(128)
+    if (fp16) { ETH_ATTN_FWD(128, true) } else { ETH_ATTN_FWD(128, false) }
   } else if (a.hd > 64) {
-    ETH_ATTN_FWD(96)
+    if (fp16) { ETH_ATTN_FWD(96, true) } else { ETH_ATTN_FWD(96, false) }
   } else {
-    ETH_ATTN_FWD(64)
+    if (fp16) { ETH_ATTN_FWD(64, true) } else { ETH_ATTN_FWD(64, false) }
   }
 #undef ETH_ATTN_FWD
   ETH_CHECK_LAUNCH("eth_attn_fwd");
