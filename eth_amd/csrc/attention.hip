@@ -741,52 +741,61 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
 // puts both the row reads of the A operands (16 rows, one chunk) and the
 // transposing reads of the B operands (4 rows x 64 bytes per 32 lanes) in
 // distinct banks.  dP's accumulator starts at -delta.
-template <int D, bool FP16, bool PAD>
-__global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dkdv_kernel(AttnArgs a) {
+//
+// G = 2 as in the forward: the groups take alternate query blocks.
+template <int D, bool FP16, bool PAD, int G>
+__global__ void __launch_bounds__(G * kAttnThreads, 2) attn_bwd_dkdv_kernel(AttnArgs a) {
   static_assert(D == 64 || D == 96, "wider heads run on the paired kernel");
   constexpr int KS = D / 16, DT = D / 32, CPR = D / 8;
   constexpr int IMG = kBQ2 * D;             // elements of one image
   // an array per image, so the compiler can tell the direct loads into one
   // from the fragment reads of another
-  __shared__ __attribute__((aligned(16))) uint16_t Q0[IMG];
-  __shared__ __attribute__((aligned(16))) uint16_t Q1[IMG];
-  __shared__ __attribute__((aligned(16))) uint16_t O0[IMG];
-  __shared__ __attribute__((aligned(16))) uint16_t O1[IMG];
-  __shared__ __attribute__((aligned(16))) float lse_s[2][kBQ2];
-  __shared__ __attribute__((aligned(16))) float del_s[2][kBQ2];
+  __shared__ __attribute__((aligned(16))) uint16_t Q0[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t Q1[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t O0[G * IMG];
+  __shared__ __attribute__((aligned(16))) uint16_t O1[G * IMG];
+  __shared__ __attribute__((aligned(16))) float lse_s[2][G][kBQ2];
+  __shared__ __attribute__((aligned(16))) float del_s[2][G][kBQ2];
 
   const int BH = a.B * a.H;
   const int bh = blockIdx.x % BH, kb = blockIdx.x / BH;
   const int b = bh / a.H, h = bh % a.H;
   const int lane = threadIdx.x & 63, hl = lane >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
+  const int w = wid & 3, grp = G == 1 ? 0 : wid >> 2;
+  const int rt = threadIdx.x & (kAttnThreads - 1);  // thread of the group
   const int k0 = kb * kBKV2 + w * 32;
   const int key = k0 + (lane & 31);
 
   ImgCopy<D, PAD> qc, oc;
   qc.init(a.q, b, h, a.hd, a.S, w, lane);
   oc.init(a.dout, b, h, a.hd, a.S, w, lane);
-  // per-query statistics: threads 0-63 lse, 64-127 delta (a padding query gets
+  // per-query statistics: a group's threads 0-63 lse, 64-127 delta (a padding query gets
   // lse = 1e30, so P = 0); delta is negated when it is stored, not here, where
   // the use would wait for every load in flight
-  const float* stats = (threadIdx.x < 64 ? a.lse : a.delta) + (int64_t)bh * a.S;
-  const int si = threadIdx.x & 63;
+  const float* stats = (rt < 64 ? a.lse : a.delta) + (int64_t)bh * a.S;
+  const int si = rt & 63;
   auto stat = [&](int qs) __attribute__((always_inline)) {
-    float v = threadIdx.x < 64 ? 1e30f : 0.f;
+    float v = rt < 64 ? 1e30f : 0.f;
     if (!PAD || qs + si < a.S) v = stats[qs + si];
     return v;
   };
   auto stat_store = [&](int p, float v) __attribute__((always_inline)) {
-    if (threadIdx.x < 64)
-      lse_s[p][threadIdx.x] = v;
-    else if (threadIdx.x < 128)
-      del_s[p][threadIdx.x - 64] = -v;
+    if (rt < 64)
+      lse_s[p][grp][rt] = v;
+    else if (rt < 128)
+      del_s[p][grp][rt - 64] = -v;
   };
   const int first = (kb * kBKV2) / kBQ2, nq = (a.S + kBQ2 - 1) / kBQ2;
-  qc.issue(Q0, first * kBQ2);
-  oc.issue(O0, first * kBQ2);
+  // steps of a group (an odd count of blocks leaves the second group's last
+  // one empty) and its first block
+  const int steps = (nq - first + G - 1) / G, mine = first + grp;
   float stat_n = 0.f;
-  if (threadIdx.x < 128) stat_n = stat(first * kBQ2);
+  if (mine < nq) {
+    qc.issue(Q0 + grp * IMG, mine * kBQ2);
+    oc.issue(O0 + grp * IMG, mine * kBQ2);
+    if (rt < 128) stat_n = stat(mine * kBQ2);
+  }
 
   uint4 kf[KS], vf[KS];  // this lane's key: K and V rows, the B operands of S and dP
   {
@@ -816,25 +825,25 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dkdv_kernel(AttnArgs
   stat_store(0, stat_n);
   __syncthreads();
 
-  auto step = [&](int m, auto par_c) __attribute__((always_inline)) {
+  auto step = [&](int i, auto par_c) __attribute__((always_inline)) {
     constexpr int P = decltype(par_c)::value;
-    const int qs0 = m * kBQ2;
-    const bool more = m + 1 < nq;
+    const int m = mine + i * G, qs0 = m * kBQ2;
+    const bool more = m + G < nq;
     if (more) {  // the next step's rows into the other images, a step ahead
-      qc.issue(P ? Q0 : Q1, qs0 + kBQ2);
-      oc.issue(P ? O0 : O1, qs0 + kBQ2);
-      if (threadIdx.x < 128) stat_n = stat(qs0 + kBQ2);
+      qc.issue((P ? Q0 : Q1) + grp * IMG, qs0 + G * kBQ2);
+      oc.issue((P ? O0 : O1) + grp * IMG, qs0 + G * kBQ2);
+      if (rt < 128) stat_n = stat(qs0 + G * kBQ2);
     }
-    const uint16_t* qi = P ? Q1 : Q0;
-    const uint16_t* oi = P ? O1 : O0;
+    const uint16_t* qi = (P ? Q1 : Q0) + grp * IMG;
+    const uint16_t* oi = (P ? O1 : O0) + grp * IMG;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int qt = qs0 + t * 32;
-      if (qt + 31 < k0) continue;  // every query of the tile precedes the wave's keys
+      if ((G == 2 && m >= nq) || qt + 31 < k0) continue;  // no block, or every query of the tile precedes the wave's keys
       a_f32x16 s = a_f32x16{}, dp;
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const float4 d4 = *reinterpret_cast<const float4*>(&del_s[P][t * 32 + swz_row(4 * g, hl)]);
+        const float4 d4 = *reinterpret_cast<const float4*>(&del_s[P][grp][t * 32 + swz_row(4 * g, hl)]);
         dp[4 * g + 0] = d4.x;
         dp[4 * g + 1] = d4.y;
         dp[4 * g + 2] = d4.z;
@@ -852,7 +861,7 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dkdv_kernel(AttnArgs
         const int kq = key - qt - 8 * hl;  // masked when > swz_row(r, 0)
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          const float4 l4 = *reinterpret_cast<const float4*>(&lse_s[P][t * 32 + swz_row(4 * g, hl)]);
+          const float4 l4 = *reinterpret_cast<const float4*>(&lse_s[P][grp][t * 32 + swz_row(4 * g, hl)]);
           const float lv[4] = {l4.x, l4.y, l4.z, l4.w};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
@@ -890,18 +899,51 @@ __global__ void __launch_bounds__(kAttnThreads, 2) attn_bwd_dkdv_kernel(AttnArgs
     if (more) stat_store(P ^ 1, stat_n);
     __syncthreads();  // this step's images free, the next step's visible
   };
-  int m = first;
-  for (; m + 1 < nq; m += 2) {
-    step(m, std::integral_constant<int, 0>{});
-    step(m + 1, std::integral_constant<int, 1>{});
+  int i = 0;
+  for (; i + 1 < steps; i += 2) {
+    step(i, std::integral_constant<int, 0>{});
+    step(i + 1, std::integral_constant<int, 1>{});
   }
-  if (m < nq) step(m, std::integral_constant<int, 0>{});
+  if (i < steps) step(i, std::integral_constant<int, 0>{});
+
+  if constexpr (G == 2) {
+    // (the images are free: every group passed the last step's barrier)
+    const int at = (w & 1) * (DT * 4 * 64) + lane;
+    float4* mv = reinterpret_cast<float4*>(w < 2 ? O0 : O1) + at;
+    float4* mk = reinterpret_cast<float4*>(w < 2 ? Q0 : Q1) + at;
+    if (grp == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          mv[(t * 4 + g) * 64] = make_float4(dv[t][g * 4], dv[t][g * 4 + 1], dv[t][g * 4 + 2], dv[t][g * 4 + 3]);
+          mk[(t * 4 + g) * 64] = make_float4(dk[t][g * 4], dk[t][g * 4 + 1], dk[t][g * 4 + 2], dk[t][g * 4 + 3]);
+        }
+    }
+    __syncthreads();
+    if (grp == 1) return;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const float4 u = mv[(t * 4 + g) * 64], x = mk[(t * 4 + g) * 64];
+        dv[t][g * 4 + 0] += u.x;
+        dv[t][g * 4 + 1] += u.y;
+        dv[t][g * 4 + 2] += u.z;
+        dv[t][g * 4 + 3] += u.w;
+        dk[t][g * 4 + 0] += x.x;
+        dk[t][g * 4 + 1] += x.y;
+        dk[t][g * 4 + 2] += x.z;
+        dk[t][g * 4 + 3] += x.w;
+      }
+  }
 
   // out through LDS in 16-byte row chunks: lane holds d = t*32 + lane%32 for
   // keys acc_row(r, hl); dV by way of the dO images, dK of the Q images
+  // (with two groups, within the wave's own part of the sums above)
   static_assert(2 * 32 * D <= IMG, "two waves' staging fits an image");
-  uint16_t* sv = (w < 2 ? O0 : O1) + (w & 1) * 32 * D;
-  uint16_t* sk = (w < 2 ? Q0 : Q1) + (w & 1) * 32 * D;
+  uint16_t* sv = (w < 2 ? O0 : O1) + (w & 1) * G * 32 * D;
+  uint16_t* sk = (w < 2 ? Q0 : Q1) + (w & 1) * G * 32 * D;
 #pragma unroll
   for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -1121,18 +1163,19 @@ static AttnOut tout(void* p, const int64_t* st) {
   return t;
 }
 
-// Groups of four waves that share a query block of the forward and dQ: two
-// where one group per block leaves wave slots empty, from the start (up to one
-// workgroup per CU) or once the short chains of a grid of up to two have
-// ended, and the chain is long enough to pay for the second group's start and
-// the closing addition.  Measured on both sides of the lines, forward /
-// backward with dK and dV, one group -> two (us; workgroups, sequence x head
-// dim): 256, 2048 x 128 42.1 / 115.8 -> 36.5 / 106.7; 128, 1024 x 64 16.1 /
-// 44.3 -> 14.3 / 41.7; 84, 777 x 96 15.9 / 53.1 -> 15.0 / 51.1; 64, 512 x 64
-// 12.3 / 26.0 -> 12.1 / 25.5; 48, 300 x 96 12.3 / 27.4 -> 12.5 / 27.7; 512,
-// 4096 x 128 94.3 / 274 -> 87.0 / 256; 384, 1500 x 80 31.8 / 104 -> 28.0 / 101;
-// 384, 1024 x 128 28.9 / 79.8 -> 29.8 / 80.8; 512, 512 x 64 14.1 / 35.8 -> 15.9
-// / 40.8; 768, 1500 x 80 50.7 / 140 -> 54.3 / 149.
+// Groups of four waves that share a block of the forward, dQ, and dK/dV up to
+// a head dim of 96: two where one group per block leaves wave slots empty,
+// from the start (up to one workgroup per CU) or once the short chains of a
+// grid of up to two have ended, and the chain is long enough to pay for the
+// second group's start and the closing addition.  Measured on both sides of
+// the lines, forward / backward, one group -> two (us; workgroups, sequence x
+// head dim): 256, 2048 x 128 42.1 / 115.8 -> 36.5 / 106.7; 256, 2048 x 64 - /
+// 72.3 (dK/dV in one) -> 22.2 / 60.7; 128, 1024 x 64 16.1 / 44.3 -> 13.4 / 36.9;
+// 84, 777 x 96 15.9 / 53.1 -> 14.6 / 47.9; 48, 300 x 96 12.3 / 27.4 -> 12.5 /
+// 27.7; 512, 4096 x 128 94.3 / 274 -> 87.0 / 256; 512, 4096 x 64 60.5 / 172 ->
+// 54.0 / 143; 384, 1500 x 80 31.8 / 104 -> 28.4 / 94.0; 384, 1024 x 128 28.9 /
+// 79.8 -> 29.8 / 80.8; 512, 512 x 64 14.1 / 35.8 -> 15.9 / 40.8 (dK/dV in one);
+// 768, 1500 x 80 50.7 / 140 -> 54.3 / 149 (dK/dV in one).
 static int attn_groups(int grid, int seq) { return seq > (grid <= 256 ? 512 : 1024) && grid <= 512 ? 2 : 1; }
 
 template <int D, bool FP16, bool PAD>
@@ -1152,8 +1195,10 @@ static void launch_bwd(const AttnArgs& a, int g_q, int g_kv, hipStream_t s) {
     attn_bwd_dq_kernel<D, FP16, PAD, 1><<<g_q, kAttnThreads, 0, s>>>(a);
   if constexpr (D == 128)
     attn_bwd_dkdv_x128_kernel<FP16, PAD><<<g_kv, 2 * kAttnThreads, 0, s>>>(a);
+  else if (attn_groups(g_kv, a.S) == 2)
+    attn_bwd_dkdv_kernel<D, FP16, PAD, 2><<<g_kv, 2 * kAttnThreads, 0, s>>>(a);
   else
-    attn_bwd_dkdv_kernel<D, FP16, PAD><<<g_kv, kAttnThreads, 0, s>>>(a);
+    attn_bwd_dkdv_kernel<D, FP16, PAD, 1><<<g_kv, kAttnThreads, 0, s>>>(a);
 }
 
 static bool aligned_rows(const void* p, const int64_t* st) {

@@ -1,6 +1,6 @@
 """GPU parity of causal attention on both sides of the lines where two groups
-of waves share a query block (forward and dQ): odd numbers of rows past whole
-blocks, query blocks whose second group has no keys for some waves, and grids
+of waves share a block (forward, dQ, and dK/dV up to a head dim of 96): odd
+numbers of rows past whole blocks, odd counts of query blocks for the two groups, query blocks whose second group has no keys for some waves, and grids
 just above one workgroup per CU.
 
 Outputs and gradients are held to the bounds of the 16-bit roundings of P and
@@ -28,6 +28,7 @@ def _err(out, ref):
 @pytest.mark.parametrize("s,b,n,d,dtype", [
     (512, 1, 2, 64, torch.bfloat16),  # one group
     (513, 1, 2, 64, torch.bfloat16),
+    (640, 1, 2, 64, torch.float16),
     (640, 1, 2, 128, torch.float16),
     (777, 1, 3, 96, torch.float16),
     (641, 2, 1, 128, torch.bfloat16),
