@@ -1128,6 +1128,14 @@ static int launch_256(const GemmArgs& a, int a_k, int b_k, hipStream_t s, int sp
 // Taken where the model promises 7 %; all of C where not.  Also measured
 // (us): [6144, 2816] x 2816 113 -> 80, [4400, 4608] x 1536 70 -> 63,
 // [2500, 8192] x 2048 87 -> 77, [1024, 50304] x 1024 107 -> 97.
+// From 1024 deep on and where the last round holds 24 to 128 tiles, 2 % will
+// do: 68 measured there ran at 0.916 to 1.010 of one launch, 0.964 in the
+// mean ([2048, 50304] x 2048 347 -> 329, its weight gradient 407 -> 377,
+// [8472, 10176] x 3392 446 -> 424, [14400, 4800] x 1600 216 -> 217).  On the
+// other sides a promise of 2 to 7 % was not kept: shallower 0.95 to 1.13
+// ([2832, 50304] x 512 201 -> 227), fewer tiles left 0.99 to 1.03 (they start
+// on the CUs that end a round early), more 1.00 to 1.03 ([2344, 50304] x 3072
+// 592 -> 607).
 struct GemmCut {
   int64_t m, n;
 };
@@ -1137,7 +1145,8 @@ static GemmCut plan_cut(int64_t M, int64_t N, int64_t K, bool wide) {
   const int tile = plan_tile(M, N, K, wide);
   const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256, rounds = tm * tn / 256;
   if (tile != 256 || rounds < 1 || tm * tn % 256 == 0) return best;
-  double t = 0.93 * tile_time(256, M, N, K, 1);
+  const int64_t last = tm * tn % 256;
+  double t = (K >= 1024 && last >= 24 && last <= 128 ? 0.98 : 0.93) * tile_time(256, M, N, K, 1);
   auto rest = [&](int64_t m, int64_t n) { return tile_time(plan_tile(m, n, K, wide), m, n, K, 1); };
   const int64_t m1 = rounds * 256 / tn * 256, n1 = rounds * 256 / tm * 256;
   if (m1 > 0 && m1 < M) {

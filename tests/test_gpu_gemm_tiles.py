@@ -86,6 +86,7 @@ def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd):
     (False, False, 7680, 2552, 520),  # 300 wide tiles: 250 and a rest of rows
     (True, True, 2304, 8192, 512),    # 288: a rest of columns, with bias
     (True, False, 8200, 2048, 512),   # 264: eight rows past a whole round
+    (True, True, 4552, 11224, 1024),  # 792: a last round of 24, deep enough for a smaller promise
 ])
 def test_products_past_whole_rounds(cuda, a_k, b_k, M, N, Kd):
     """Grids a little over a whole number of rounds run in two launches."""
