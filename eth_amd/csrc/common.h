@@ -94,23 +94,28 @@ __device__ __forceinline__ void store_elem(void* p, int64_t i, int dtype, float 
 }
 
 // Sum over the wavefront, in every lane.  Called with all 64 lanes active.
-// Data-parallel-primitive moves within the VALU (partial sums run up each row
-// of 16, then across rows into lane 63): the same sum by lane exchanges goes
-// through LDS six times, which a row's LayerNorm waits for twice in a chain
-// (LayerNorm backward of [8192, 2048] 32.4 -> 30.7 us, of [4096, 5120] 46.5 ->
-// 43.8 us).
-template <int CTRL, int ROWS, int BANKS>
+// Pairs 32, 16, 8, 4, 2 and 1 lanes apart are added in that order, all within
+// the VALU: the two halves and the pairs of rows by lane swaps, then
+// data-parallel-primitive moves inside a row of 16 (a rotation by 8 or 4 meets
+// the same pairs as the exchange, whose sums repeat with that period).  The
+// same tree by lane exchanges goes through LDS six times, which a row's
+// LayerNorm waits for twice in a chain (LayerNorm backward of [8192, 2048]
+// 32.4 -> 30.7 us, of [4096, 5120] 46.5 -> 43.8 us).
+template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
-  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, BANKS, false));
+  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 __device__ __forceinline__ float wave_sum(float v) {
-  v = dpp_add<0x111, 0xf, 0xf>(v);  // row_shr:1
-  v = dpp_add<0x112, 0xf, 0xf>(v);  // row_shr:2
-  v = dpp_add<0x114, 0xf, 0xe>(v);  // row_shr:4, into lanes 4-15
-  v = dpp_add<0x118, 0xf, 0xc>(v);  // row_shr:8, into lanes 8-15
-  v = dpp_add<0x142, 0xa, 0xf>(v);  // row_bcast:15, into rows 1 and 3
-  v = dpp_add<0x143, 0xc, 0xf>(v);  // row_bcast:31, into rows 2 and 3
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+  // each swap turns (v, v) into the two addends of every lane
+  u32x2 p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(p.x) + __uint_as_float(p.y);
+  p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(p.x) + __uint_as_float(p.y);
+  v = dpp_add<0x128>(v);     // row_ror:8
+  v = dpp_add<0x124>(v);     // row_ror:4
+  v = dpp_add<0x4e>(v);      // quad_perm:[2,3,0,1]
+  return dpp_add<0xb1>(v);   // quad_perm:[1,0,3,2]
 }
 
 // Block-wide sum for blockDim.x == NT (multiple of 64).  `red` must hold

@@ -1,11 +1,13 @@
 """GPU: the LayerNorm backward at the widths and row counts where its team
-split changes, against fp64.
+split changes, against fp64; the forward's row mean bit for bit in the order
+its wave adds.
 
 dx rounds once to 16 bits (2^-9 of a bf16 value; with the residual gradient
 the sum of two rounded values rounds again, so twice that of each); its fp32
 arithmetic and the fp32 column sums over `rows` rows add at most rows * 2^-23
 of the summed magnitudes."""
 
+import numpy as np
 import pytest
 import torch
 
@@ -43,3 +45,24 @@ def test_backward_widths(cuda, rows, cols):
             sums = K.reduce_partials(part, torch.empty(cols, device=cuda), accumulate=False)
             mag = dx.double().abs().sum(0)
             assert bool(((sums.double() - dx.double().sum(0)).abs() <= rows * 2.0**-23 * mag + 1e-6).all())
+
+
+@pytest.mark.parametrize("cols", [8, 264, 512, 1536, 2048, 8192])
+def test_row_mean_adds_lanes_in_pairs(cuda, cols):
+    """A lane adds its columns (eight of every 512) in order; the wave then
+    adds lanes 32, 16, 8, 4, 2 and 1 apart, every addition in fp32."""
+    rows = 37
+    announce(f"layer norm mean order {rows}x{cols}")
+    gen = torch.Generator().manual_seed(cols)
+    x = (torch.randn(rows, cols, generator=gen) * 2 + 0.5).bfloat16()
+    one = torch.ones(cols).bfloat16().to(cuda)
+    mean = K.layer_norm_fwd(x.to(cuda), one, one)[1]
+    padded = np.zeros((rows, -(-cols // 512) * 512), np.float32)
+    padded[:, :cols] = x.float().numpy()
+    lanes = np.zeros((rows, 64), np.float32)
+    for vec in padded.reshape(rows, -1, 64, 8).transpose(1, 3, 0, 2).reshape(-1, rows, 64):
+        lanes = lanes + vec
+    for apart in (32, 16, 8, 4, 2, 1):
+        lanes = lanes + lanes[:, np.arange(64) ^ apart]
+    assert lanes.dtype == np.float32
+    assert np.array_equal(mean.cpu().numpy(), lanes[:, 0] / np.float32(cols))
