@@ -43,7 +43,7 @@ class StreamedGradSync:
 
     def start(self, normalization_scale=1.0):
         """Arm the sync for the backward about to run."""
-        main = torch.cuda.current_stream(self.device)
+        self.origin = main = torch.cuda.current_stream(self.device)
         self.stream.wait_stream(main)
         with torch.cuda.stream(self.stream):
             self.ex.begin(normalization_scale)
@@ -66,6 +66,8 @@ class StreamedGradSync:
     def _launch(self, b):
         main = torch.cuda.current_stream(self.device)
         self.stream.wait_stream(main)
+        if main != self.origin:  # the step's stream: weight gradients that stayed in line
+            self.stream.wait_stream(self.origin)
         self.stream.wait_stream(K.side_stream(self.device))
         with torch.cuda.stream(self.stream):
             for p in self.buckets[b]:

@@ -12,36 +12,57 @@ from its fp32 reduction -- and the DDP hook adds it into main_grad, a second
 rounding, as the reference's `main_grad.add_(param.grad)` does.
 """
 
+import threading
+
 import torch
 
 from .. import kernels as K
 from .distributed import grad_written, main_grad_target, materialize_main_grad
 
 
-_overlap = {"wgrad": False}
+# open overlapped_wgrad contexts (of every thread) and the stream that the
+# first of them was entered on
+_overlap = {"wgrad": 0, "home": None}
+_overlap_lock = threading.Lock()
 
 
 class overlapped_wgrad:
-    """Within this context, LinearFn's weight-gradient GEMMs into main_grad
-    run on a side stream, overlapped with the data-gradient chain; on exit
-    the current stream waits for them, so main_grad is complete for
-    whatever runs next."""
+    """Within this context, LinearFn's large weight-gradient GEMMs into
+    main_grad run on a side stream, overlapped with the data-gradient chain.
+    Small ones (_SIDE_MIN_FLOPS) stay in line where their node runs on the
+    stream the context was entered on.  Contributions to one weight are
+    ordered whatever streams their nodes run on, and on exit the current
+    stream waits for all of them, so the weights' main grads are complete for
+    whatever runs next on it.  Contexts entered on different streams without
+    a wait between them are the caller's to order."""
 
     def __enter__(self):
-        self._prev = _overlap["wgrad"]
         self._mark = K.side_mark()
-        _overlap["wgrad"] = True
+        with _overlap_lock:
+            if _overlap["wgrad"] == 0:
+                _overlap["home"] = torch.cuda.current_stream() if torch.cuda.is_initialized() else None
+            _overlap["wgrad"] += 1
+            self._home = _overlap["home"]
         return self
 
     def __exit__(self, *exc):
-        _overlap["wgrad"] = self._prev
+        with _overlap_lock:
+            _overlap["wgrad"] -= 1
+            if _overlap["wgrad"] == 0:
+                _overlap["home"] = None
+        if self._home is not None:
+            now = torch.cuda.current_stream(self._home.device)
+            if now != self._home:
+                now.wait_stream(self._home)
         K.join_side_streams(since=self._mark)
         return False
 
 
 # A weight gradient below this many FLOPs stays on the data-gradient chain's
-# stream: the two cross-stream waits of the side stream take the host 30-40 us
-# and the GPU 8-12 us, as long as such a product runs (8.6 GFLOP: 18 us).
+# stream, where that is the context's (a product in line on another stream
+# would need waits of its own to stay ordered): the two cross-stream waits of
+# the side stream take the host 30-40 us and the GPU 8-12 us, as long as such a
+# product runs (8.6 GFLOP: 18 us).
 _SIDE_MIN_FLOPS = 1.2e10
 
 
@@ -79,16 +100,19 @@ def _flat(x):
 
 
 def _wgrad(weight, dy2, x2, mg, accumulate):
-    """weight's gradient into its fp32 main grad: inside overlapped_wgrad and
-    when large enough, on a side stream."""
-    main = None
-    if _overlap["wgrad"] and dy2.is_cuda:
-        main = torch.cuda.current_stream(dy2.device)
-    if main is None or 2.0 * dy2.numel() * x2.shape[1] < _SIDE_MIN_FLOPS:
-        if main is not None and getattr(weight, "_eth_side_grad", False):
-            # an earlier contribution may still be running on the side stream
+    """weight's gradient into its fp32 main grad: inside overlapped_wgrad on a
+    side stream, or in line when it is small and the node runs on the
+    context's own stream.  `weight._eth_side_grad` says which of the two the
+    last contribution took; each waits for the other, so contributions to a
+    weight form one chain."""
+    if not _overlap["wgrad"] or not dy2.is_cuda:
+        K.gemm(dy2.t(), x2, out=mg, accumulate=accumulate)
+        return
+    main, home = torch.cuda.current_stream(dy2.device), _overlap["home"]
+    if main == home and 2.0 * dy2.numel() * x2.shape[1] < _SIDE_MIN_FLOPS:
+        if getattr(weight, "_eth_side_grad", False):
             main.wait_stream(K.side_stream(dy2.device))
-            weight._eth_side_grad = False
+        weight._eth_side_grad = False
         K.gemm(dy2.t(), x2, out=mg, accumulate=accumulate)
         return
     # the weight gradient only feeds main_grad: it runs on a side stream,
@@ -96,8 +120,10 @@ def _wgrad(weight, dy2, x2, mg, accumulate):
     # gradient sync reads the buffer
     side = K.side_stream(dy2.device)
     K.mark_side_launch()
-    weight._eth_side_grad = True
     side.wait_stream(main)
+    if main != home and home is not None and not getattr(weight, "_eth_side_grad", True):
+        side.wait_stream(home)
+    weight._eth_side_grad = True
     with torch.cuda.stream(side):
         K.gemm(dy2.t(), x2, out=mg, accumulate=accumulate)
     dy2.record_stream(side)

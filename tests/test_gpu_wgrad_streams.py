@@ -1,5 +1,7 @@
 """GPU: weight gradients inside overlapped_wgrad, on the side stream or in
-line by their size, accumulate alike in every order."""
+line by their size, accumulate alike in every order.  A bounded delay queued
+on the stream that a later step has to wait for keeps its work pending when
+that step is issued, and results are read right after the context."""
 
 import pytest
 import torch
@@ -9,6 +11,8 @@ from eth_amd.model import functional as Fn
 from tests.conftest import announce
 
 pytestmark = pytest.mark.gpu
+
+DELAY = 2_000_000  # clock ticks: 1 ms at 2 GHz, 20 ms at 100 MHz
 
 
 @pytest.mark.parametrize("order", ["small first", "large first"])
@@ -32,10 +36,13 @@ def test_one_weight_with_small_and_large_contributions(cuda, order):
     for _ in range(3):
         w.main_grad.zero_()
         outs = [Fn.LinearFn.apply(x, w, None) for x in xs]
+        with torch.cuda.stream(K.side_stream(w.device)):
+            torch.cuda._sleep(DELAY)
         with Fn.overlapped_wgrad():
             for o, dy in zip(outs, dys):
                 torch.autograd.backward(o, dy)
-        assert torch.equal(w.main_grad, want)
+        got = w.main_grad.clone()
+        assert torch.equal(got, want)
 
 
 def test_join_waits_only_for_new_side_work(cuda):
@@ -46,3 +53,41 @@ def test_join_waits_only_for_new_side_work(cuda):
     assert K.side_mark() == mark
     K.mark_side_launch()
     assert K.side_mark() != mark
+
+
+@pytest.mark.parametrize("tokens", [64, 4096])
+def test_node_of_another_stream_and_nested_contexts(cuda, tokens):
+    """One weight used by a product on the context's stream and one on
+    another stream that is behind; an inner context that launches nothing
+    leaves the wait to the outer one."""
+    announce(f"wgrad streams nested {tokens}")
+    h = 2048
+    gen = torch.Generator(device=cuda).manual_seed(tokens)
+    xs = [torch.randn(tokens, h, device=cuda, generator=gen).bfloat16() for _ in range(2)]
+    dys = [torch.randn(tokens, h, device=cuda, generator=gen).bfloat16() for _ in range(2)]
+    want = torch.zeros(h, h, device=cuda)
+    for x, dy in zip(xs, dys):
+        K.gemm(dy.t(), x, out=want, accumulate=True)
+    w = torch.nn.Parameter(torch.randn(h, h, device=cuda, generator=gen).bfloat16())
+    w.main_grad = torch.zeros(h, h, device=cuda)
+    other = torch.cuda.Stream()
+    for order in (0, 1):
+        w.main_grad.fill_(7.0)
+        w._eth_main_grad_stale = True  # the first contribution stores
+        outs = [Fn.LinearFn.apply(xs[0], w, None)]
+        other.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(other):
+            outs.append(Fn.LinearFn.apply(xs[1], w, None))
+        torch.cuda.synchronize()
+        first, second = (0, 1) if order == 0 else (1, 0)
+        with Fn.overlapped_wgrad():
+            with torch.cuda.stream(other):
+                torch.cuda._sleep(DELAY)
+            for i in (first, second):
+                torch.autograd.backward(outs[i], dys[i])
+            with Fn.overlapped_wgrad():
+                pass
+        got = w.main_grad.clone()
+        # (the two sums of one pair of products: fp32 addition commutes)
+        assert torch.equal(got, want)
+        torch.cuda.synchronize()
