@@ -98,20 +98,6 @@ def _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig):
     return bool(nat.value("eth_gemm_splitk_pays", M, N, K, splits))
 
 
-_scratch = {}
-
-
-def _scratch_f32(numel, device):
-    """An fp32 workspace per (device, stream), reused across calls and grown
-    on demand: launches on one stream are ordered, so they may share it."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
-    buf = _scratch.get(key)
-    if buf is None or buf.numel() < numel:
-        buf = torch.empty(numel, dtype=torch.float32, device=device)
-        _scratch[key] = buf
-    return buf[:numel]
-
-
 _side = {}
 _side_launches = itertools.count(1)
 _side_last = 0  # a value no earlier launch had, set at every side-stream launch
@@ -490,7 +476,8 @@ def embedding_bwd(tokens, positions, dout, dword, dpos):
             raise ValueError("embedding gradients must be contiguous fp32 [rows, hidden]")
     V = dword.shape[0] if dword is not None else 1
     P = dpos.shape[0] if dpos is not None else 1
-    ws = _scratch_f32(-(-nat.value("eth_embedding_bwd_workspace", b, s) // 4), dout.device)
+    # (the call's own: its two launches may have another thread's between them)
+    ws = torch.empty(nat.value("eth_embedding_bwd_workspace", b, s), dtype=torch.uint8, device=dout.device)
     nat.call("eth_embedding_bwd", nat.ptr(tokens), nat.ptr(positions), nat.ptr(dout), nat.ptr(dword), nat.ptr(dpos),
              nat.ptr(ws), b, s, h, V, P, code, nat.stream_ptr(dout.device))
 
