@@ -79,6 +79,11 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 // s_waitcnt vmcnt(0) (expcnt, lgkmcnt unconstrained) as the builtin, so the
 // compiler's own wait-count tracking knows that no vector load is pending
 __device__ __forceinline__ void vm_wait_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+// Between a wave's LDS accesses of one type and its accesses of another to the
+// same memory, all of them its own: its LDS operations execute in order, but
+// the compiler may take float, 16-bit and 16-byte accesses to be apart and
+// move one past the other.  The clobber holds them in place.
+__device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 // 8 fp32 -> one 16-byte MFMA operand
 template <bool FP16>
 __device__ __forceinline__ uint4 pack8(const float* v) {
@@ -716,7 +721,7 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       stage[acc_row(r, hl) * SL + t * 32 + (lane & 31)] = from_f<FP16>(dkw ? acc[t][r] * a.scale : acc[t][r]);
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's staging writes are done (the wave reads only its own)
+  wave_lds_fence();  // the wave reads back only its own rows
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int c = i * 64 + lane, kr = c >> 4, col = (c & 15) * 8;  // key row, first column of the chunk
@@ -936,6 +941,7 @@ __global__ void __launch_bounds__(G * kAttnThreads, 2) attn_bwd_dkdv_kernel(Attn
         dk[t][g * 4 + 2] += x.z;
         dk[t][g * 4 + 3] += x.w;
       }
+    wave_lds_fence();  // the rows below go where these sums were
   }
 
   // out through LDS in 16-byte row chunks: lane holds d = t*32 + lane%32 for
@@ -952,7 +958,7 @@ __global__ void __launch_bounds__(G * kAttnThreads, 2) attn_bwd_dkdv_kernel(Attn
       sv[o] = from_f<FP16>(dv[t][r]);
       sk[o] = from_f<FP16>(dk[t][r] * a.scale);
     }
-  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): a wave reads back only its own rows
+  wave_lds_fence();  // a wave reads back only its own rows
 #pragma unroll
   for (int i = 0; i < 32 * CPR / 64; ++i) {
     const int c = i * 64 + lane, kr = c / CPR, col = (c % CPR) * 8;
