@@ -1163,6 +1163,14 @@ static GemmCut plan_cut(int64_t M, int64_t N, int64_t K, bool wide) {
   return best;
 }
 
+// The 256x256 kernels take C rows of whole four-column vectors (vector
+// stores), a C extent plus one tile of rows below 2 GiB (their buffer offsets)
+// and the K of each layout.
+static bool wide_takes(int64_t M, int64_t N, int64_t K, int a_kcontig, int b_kcontig, int64_t ldc, int esz,
+                       bool c_vec) {
+  return K % (a_kcontig ? 64 : b_kcontig ? 128 : 8) == 0 && c_vec && ((M + 255) * ldc + N) * esz < (1LL << 31);
+}
+
 static int launch_planned(const GemmArgs& a, int a_k, int b_k, bool fp16, bool wide, hipStream_t s) {
   switch (plan_tile(a.M, a.N, a.K, wide)) {
     case 256:
@@ -1217,16 +1225,12 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
   a.flags = flags;
   a.alpha = alpha;
   hipStream_t s = (hipStream_t)stream;
-  // the 256x256 kernels: C rows 16-byte aligned (vector stores), C extent
-  // plus one tile of rows below 2 GiB (its buffer offsets), and the K each
-  // layout takes
   const int esz = c_dtype == ETH_F32 ? 4 : 2;
-  const int64_t c_extent = ((M - 1) * ldc + N) * esz;
   a.c_vec = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C % (4 * esz)) == 0;
   a.k_split = 0;
   a.c_split_stride = 0;
-  const bool wide = K % (a_kcontig ? 64 : b_kcontig ? 128 : 8) == 0 && a.c_vec && c_extent + 256 * ldc * esz < (1LL << 31);
-  a.c_bytes = wide ? (uint32_t)c_extent : 0;
+  const bool wide = wide_takes(M, N, K, a_kcontig, b_kcontig, ldc, esz, a.c_vec);
+  a.c_bytes = wide ? (uint32_t)(((M - 1) * ldc + N) * esz) : 0;
   const bool fp16 = in_dtype == ETH_F16;
   const GemmCut cut = plan_cut(M, N, K, wide);
   if (cut.m == M && cut.n == N) return launch_planned(a, a_kcontig, b_kcontig, fp16, wide, s);
@@ -1255,6 +1259,23 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
   }
   const int rc = launch_planned(a, a_kcontig, b_kcontig, fp16, wide, s);
   return rc != ETH_OK ? rc : launch_planned(r, a_kcontig, b_kcontig, fp16, wide, s);
+}
+
+extern "C" int eth_gemm_plan(int64_t M, int64_t N, int64_t K, int a_kcontig, int b_kcontig, int64_t ldc, int c_dtype,
+                             int64_t* plan) {
+  ETH_CHECK_ARG(plan, "eth_gemm_plan: null pointer");
+  ETH_CHECK_ARG(valid_dtype(c_dtype), "eth_gemm_plan: bad output dtype %d", c_dtype);
+  ETH_CHECK_ARG(M > 0 && N > 0 && K > 0 && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31) && ldc >= N,
+                "eth_gemm_plan: bad shape %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
+  const bool wide = wide_takes(M, N, K, a_kcontig, b_kcontig, ldc, c_dtype == ETH_F32 ? 4 : 2,
+                               ldc % 4 == 0 && N % 4 == 0);
+  const GemmCut cut = plan_cut(M, N, K, wide);
+  plan[0] = plan_tile(cut.m, cut.n, K, wide);
+  plan[1] = cut.m;
+  plan[2] = cut.n;
+  const int64_t m = cut.m < M ? M - cut.m : M, n = cut.n < N ? N - cut.n : N;
+  plan[3] = cut.m == M && cut.n == N ? 0 : plan_tile(m, n, K, wide);
+  return ETH_OK;
 }
 
 namespace eth {

@@ -238,6 +238,14 @@ int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t l
              int64_t M, int64_t N, int64_t K, int in_dtype, int flags, float alpha,
              void* stream);
 
+/* What eth_gemm launches for such a product with 4-column aligned C rows of
+ * stride ldc (host only, no launch): plan[0] the tile (256, 128 or 64) of the
+ * launch over the rows [0, plan[1]) and columns [0, plan[2]) of C; where that
+ * is not all of C, plan[3] is the tile of the second launch over the rest,
+ * else 0. */
+int eth_gemm_plan(int64_t M, int64_t N, int64_t K, int a_kcontig, int b_kcontig, int64_t ldc, int c_dtype,
+                  int64_t* plan);
+
 /* Split-K form of the fp32 product (C += A B with accumulate != 0, else
  * C = A B; alpha 1, no bias) for grids too small to fill the chip, such as
  * the [h, h] weight gradient of the attention projection: `splits` k-ranges
@@ -247,6 +255,9 @@ int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t l
  * N % 4 == 0, 16-byte aligned C rows.
  * Same reference seam as eth_gemm's ETH_GEMM_ACCUMULATE form
  * (model/distributed.py:116-123 over mpu/layers.py:452-470). */
+int eth_gemm_splitk(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,
+                    float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int in_dtype, int splits,
+                    int accumulate, float* workspace, void* stream);
 int64_t eth_gemm_splitk_workspace(int64_t M, int64_t N, int splits);
 /* The same for every output eth_gemm writes: C of c_dtype, alpha and bias
  * applied to the sum of the partials, which is rounded once.  K % 64 == 0
@@ -256,12 +267,9 @@ int64_t eth_gemm_splitk_workspace(int64_t M, int64_t N, int splits);
 int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,
                         void* C, int64_t ldc, int c_dtype, const void* bias, int64_t M, int64_t N, int64_t K,
                         int in_dtype, int flags, float alpha, int splits, float* workspace, void* stream);
-/* 1 where eth_gemm_splitk with `splits` is expected to finish before
+/* 1 where the split-K form with `splits` is expected to finish before
  * eth_gemm on the same [M, N] x K product, else 0. */
 int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits);
-int eth_gemm_splitk(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,
-                    float* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int in_dtype, int splits,
-                    int accumulate, float* workspace, void* stream);
 
 /* ------------------------------------------------------------------------
  * LayerNorm (bf16/fp16 rows of `cols` elements, cols % 8 == 0, <= 8192).

@@ -7,6 +7,8 @@ than sum |a||b| (doubled for the order inside an MFMA), and the result rounds
 once to its dtype (2^-9 of a bf16 value, 2^-12 of an fp16 one, with fp16's
 subnormal spacing as a floor)."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -17,6 +19,14 @@ from tests.conftest import announce
 pytestmark = pytest.mark.gpu
 
 LAYOUTS = [(True, True), (True, False), (False, False), (False, True)]
+
+
+def _plan(M, N, Kd, a_k, b_k, dtype, ldc=None):
+    """(tile, rows, columns) of the first launch and the tile of the second
+    (0: none), as the library plans it."""
+    plan = (ctypes.c_int64 * 4)()
+    nat.call("eth_gemm_plan", M, N, Kd, int(a_k), int(b_k), ldc or N, nat.dtype_code(dtype), plan)
+    return tuple(plan)
 
 
 def _operands(M, N, Kd, a_k, b_k, dtype, cuda, seed):
@@ -43,10 +53,28 @@ def _check(got, ref, mag, Kd, out_dtype, what):
     (128, 128, 192),    # three k-tiles: the remainder steps alone
     (120, 248, 264),    # four k-tiles and a tail
     (200, 328, 1000),   # ragged everywhere
-    (2048, 1024, 328),  # 128x128 tiles, k-tail of one chunk
-    (1928, 2056, 520),  # 128x128 tiles, ragged edges
+    (2048, 1024, 328),  # a whole round and k-tail of one chunk
+    (1928, 2056, 520),  # past a whole round, ragged edges
 ])
 def test_products_at_tile_edges(cuda, M, N, Kd, a_k, b_k):
+    """64x64 tiles."""
+    assert _plan(M, N, Kd, a_k, b_k, torch.float32) == (64, M, N, 0)
+    _products(cuda, M, N, Kd, a_k, b_k)
+
+
+@pytest.mark.parametrize("a_k,b_k,M,N,Kd", [
+    # ragged edges, 33 to 36 k-tiles (every remainder of a trip round the
+    # four stages), the last one short in three of them
+    *((a_k, b_k, 1928, 1032, Kd) for a_k, b_k in LAYOUTS for Kd in (2056, 2120, 2184, 2304)),
+    # two rounds of few k-tiles (weight gradients take wide tiles there)
+    (True, True, 4088, 2044, 328), (True, False, 4088, 2040, 328), (False, True, 4088, 2044, 328),
+])
+def test_128_tiles(cuda, a_k, b_k, M, N, Kd):
+    assert _plan(M, N, Kd, a_k, b_k, torch.float32) == (128, M, N, 0)
+    _products(cuda, M, N, Kd, a_k, b_k)
+
+
+def _products(cuda, M, N, Kd, a_k, b_k):
     announce(f"gemm {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
     for dtype in (torch.bfloat16, torch.float16):
         a, b, ad, bd = _operands(M, N, Kd, a_k, b_k, dtype, cuda, M + 3 * N + 7 * Kd)
@@ -73,6 +101,7 @@ def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd):
     """128 tiles of 256x256 with ragged edges, every k-tile count the loop
     and its prologue treat apart."""
     M, N = 4088, 2040
+    assert _plan(M, N, Kd, a_k, b_k, torch.float32) == _plan(M, N, Kd, a_k, b_k, torch.bfloat16) == (256, M, N, 0)
     announce(f"gemm wide {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
     a, b, ad, bd = _operands(M, N, Kd, a_k, b_k, torch.bfloat16, cuda, Kd)
     ref, mag = a @ b, a.abs() @ b.abs()
@@ -82,26 +111,36 @@ def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd):
     _check(K.gemm(ad, bd), ref, mag, Kd, torch.bfloat16, "16-bit")
 
 
-@pytest.mark.parametrize("a_k,b_k,M,N,Kd", [
-    (False, False, 7680, 2552, 520),  # 300 wide tiles: 250 and a rest of rows
-    (True, True, 2304, 8192, 512),    # 288: a rest of columns, with bias
-    (True, False, 8200, 2048, 512),   # 264: eight rows past a whole round
-    (True, True, 4552, 11224, 1024),  # 792: a last round of 24, deep enough for a smaller promise
+@pytest.mark.parametrize("a_k,b_k,M,N,Kd,dtype,plan", [
+    # 300 wide tiles: 250 and a rest of rows
+    (False, False, 7680, 2552, 520, torch.bfloat16, (256, 6400, 2552, 128)),
+    (True, True, 2304, 8192, 512, torch.float16, (256, 2048, 8192, 64)),
+    (True, False, 8200, 2048, 512, torch.bfloat16, (256, 8192, 2048, 64)),  # eight rows past a whole round
+    # 792: a last round of 24, deep enough for a smaller promise
+    (True, True, 4552, 11224, 1024, torch.bfloat16, (256, 4352, 11224, 128)),
+    # a rest of columns (of B's, the bias's and C's rows), in every layout
+    (True, True, 8192, 2304, 512, torch.bfloat16, (256, 8192, 2048, 64)),
+    (True, False, 8184, 2312, 512, torch.float16, (256, 8184, 2048, 128)),
+    (False, False, 8184, 2312, 520, torch.float16, (256, 8184, 2048, 128)),
+    (False, True, 8184, 2308, 512, torch.bfloat16, (256, 8184, 2048, 128)),
+    # a rest of rows of the same layout
+    (False, True, 2552, 7684, 512, torch.float16, (256, 2048, 7684, 128)),
 ])
-def test_products_past_whole_rounds(cuda, a_k, b_k, M, N, Kd):
+def test_products_past_whole_rounds(cuda, a_k, b_k, M, N, Kd, dtype, plan):
     """Grids a little over a whole number of rounds run in two launches."""
+    assert _plan(M, N, Kd, a_k, b_k, torch.float32) == _plan(M, N, Kd, a_k, b_k, dtype, N + 8) == plan
     announce(f"gemm rounds {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
     gen = torch.Generator(device=cuda).manual_seed(M + N)
-    a = torch.randn(*((M, Kd) if a_k else (Kd, M)), device=cuda, generator=gen).bfloat16()
-    b = torch.randn(*((N, Kd) if b_k else (Kd, N)), device=cuda, generator=gen).bfloat16()
+    a = torch.randn(*((M, Kd) if a_k else (Kd, M)), device=cuda, generator=gen).to(dtype)
+    b = torch.randn(*((N, Kd) if b_k else (Kd, N)), device=cuda, generator=gen).to(dtype)
     ad, bd = a if a_k else a.t(), b.t() if b_k else b
-    bias = torch.linspace(-1, 1, N, device=cuda).bfloat16()
+    bias = torch.linspace(-1, 1, N, device=cuda).to(dtype)
     ref = (ad.double() @ bd.double()).cpu()
     mag = (ad.double().abs() @ bd.double().abs()).cpu()
     extra = bias.double().cpu()
-    wide = torch.full((M, N + 8), 9.0, dtype=torch.bfloat16, device=cuda)
+    wide = torch.full((M, N + 8), 9.0, dtype=dtype, device=cuda)
     K.gemm(ad, bd, out=wide[:, :N], bias=bias)
-    _check(wide[:, :N], ref + extra, mag + extra.abs(), Kd, torch.bfloat16, "strided output with bias")
+    _check(wide[:, :N], ref + extra, mag + extra.abs(), Kd, dtype, "strided output with bias")
     assert bool((wide[:, N:] == 9).all())
     acc = torch.full((M, N), 0.5, device=cuda)
     K.gemm(ad, bd, out=acc, accumulate=True)
@@ -156,13 +195,23 @@ def test_deep_product_takes_splits(cuda):
     assert torch.equal(got, K.gemm(ad, bd))
 
 
-@pytest.mark.parametrize("N", [3, 7, 66, 131])
-def test_products_with_unaligned_output_rows(cuda, N):
-    """Output widths and row strides that take no vector stores."""
-    M, Kd = 70, 136
+@pytest.mark.parametrize("M,Kd,N,tile", [(70, 136, 3, 64), (70, 136, 7, 64), (70, 136, 66, 64), (70, 136, 131, 64),
+                                         (1928, 2056, 1031, 128)])
+def test_products_with_unaligned_output_rows(cuda, M, Kd, N, tile):
+    """Output widths and row strides that take no vector stores, 16-bit and
+    accumulated."""
     announce(f"gemm {M}x{N}x{Kd} unaligned C")
-    a, b, ad, bd = _operands(M, N, Kd, True, True, torch.bfloat16, cuda, N)
-    wide = torch.full((M, N + 3), 9.0, dtype=torch.bfloat16, device=cuda)
-    K.gemm(ad, bd, out=wide[:, 1 : N + 1])
-    _check(wide[:, 1 : N + 1], a @ b, a.abs() @ b.abs(), Kd, torch.bfloat16, "strided output")
-    assert bool((wide[:, 0] == 9).all()) and bool((wide[:, N + 1 :] == 9).all())
+    for a_k, dtype in ((True, torch.bfloat16), (False, torch.float16)):
+        m = M - M % 8 if not a_k else M  # rows of a row-contiguous A are whole 16-byte units
+        assert _plan(m, N, Kd, a_k, True, dtype, N + 3) == (tile, m, N, 0)
+        a, b, ad, bd = _operands(m, N, Kd, a_k, True, dtype, cuda, N)
+        ref, mag = a @ b, a.abs() @ b.abs()
+        bias = torch.linspace(-1, 1, N).to(dtype)
+        wide = torch.full((m, N + 3), 9.0, dtype=dtype, device=cuda)
+        K.gemm(ad, bd, out=wide[:, 1 : N + 1], bias=bias.to(cuda))
+        _check(wide[:, 1 : N + 1], ref + bias.double(), mag + bias.double().abs(), Kd, dtype, "strided output")
+        assert bool((wide[:, 0] == 9).all()) and bool((wide[:, N + 1 :] == 9).all())
+        acc = torch.full((m, N + 3), 0.5, device=cuda)
+        K.gemm(ad, bd, out=acc[:, 1 : N + 1], accumulate=True)
+        _check(acc[:, 1 : N + 1], ref + 0.5, mag + 0.5, Kd, torch.float32, "accumulated")
+        assert bool((acc[:, 0] == 0.5).all()) and bool((acc[:, N + 1 :] == 0.5).all())
