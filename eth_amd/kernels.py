@@ -90,12 +90,14 @@ def _splitk_splits(M, N, K, out):
 
 @functools.lru_cache(maxsize=4096)
 def _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig):
-    """Whether the split-K form takes this product and finishes before the
-    plain one (sizes and layout only; the smaller tiles fill the chip
-    without a second pass unless K is deep)."""
+    """fp32 elements of workspace if the split-K form takes this product and
+    finishes before the plain one, else 0 (sizes and layout only; the smaller
+    tiles fill the chip without a second pass unless K is deep)."""
     if splits < 2 or K % (64 if a_kcontig else 128 * splits if b_kcontig else 8) or 4 * (M + 256) * N >= 2**31:
-        return False
-    return bool(nat.value("eth_gemm_splitk_pays", M, N, K, splits))
+        return 0
+    if not nat.value("eth_gemm_splitk_pays", M, N, K, splits):
+        return 0
+    return nat.value("eth_gemm_splitk_workspace", M, N, splits) // 4
 
 
 _side = {}
@@ -163,9 +165,10 @@ def gemm(a, b, out=None, bias=None, accumulate=False, out_dtype=None, alpha=1.0)
         flags |= nat.GEMM_BIAS
     _observe("gemm", "begin", 2.0 * M * N * K)
     splits = _splitk_splits(M, N, K, out)
-    if _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig):
+    partials = _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig)
+    if partials:
         # (a fresh buffer per call: two threads may share the stream)
-        ws = torch.empty(splits * M * N, dtype=torch.float32, device=a.device)
+        ws = torch.empty(partials, dtype=torch.float32, device=a.device)
         nat.call(
             "eth_gemm_splitk_out",
             nat.ptr(a), lda, a_kcontig,

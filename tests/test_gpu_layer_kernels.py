@@ -89,39 +89,73 @@ def test_gemm_pipelined_kernel_layouts(cuda, dtype, a_k, b_k):
 
 @pytest.mark.parametrize("a_k,b_k", [(True, True), (True, False), (False, False), (False, True)])
 def test_gemm_splitk_accumulate(cuda, a_k, b_k):
-    """Small-grid fp32 accumulation (20 tiles of 256, K 4096) takes the
-    split-K path: 4 k-splits into a workspace, added in order.  Matches the
-    fp32 reference and is bit-identical run to run."""
+    """fp32 accumulation over 4 k-splits in a workspace, added in order.
+    Matches the fp32 reference and is bit-identical run to run, to the store
+    form and to the general split-K entry; K.gemm takes the same path for a
+    product deep enough."""
     from eth_amd import _native as nat
 
-    M, N, Kd = 1024, 1032, 4096
-    assert K._splitk_splits(M, N, Kd, torch.empty(M, N, device=cuda)) == 4
+    M, N, Kd, splits = 1024, 1032, 4096, 4
     announce(f"gemm split-K a_k={a_k} b_k={b_k} {M}x{N}x{Kd}")
     gen = torch.Generator().manual_seed(23 + 2 * a_k + b_k)
     a = _rand((M, Kd), torch.bfloat16, gen)
     b = _rand((Kd, N), torch.bfloat16, gen, 0.05)
     ad = a.to(cuda) if a_k else a.t().contiguous().to(cuda).t()
     bd = b.t().contiguous().to(cuda).t() if b_k else b.to(cuda)
+    lda = ad.stride(0) if a_k else ad.stride(1)
+    ldb = bd.stride(1) if b_k else bd.stride(0)
+    code = nat.dtype_code(torch.bfloat16)
+    assert nat.value("eth_gemm_splitk_workspace", M, N, splits) == 4 * splits * M * N
+    ws = torch.empty(splits * M * N, dtype=torch.float32, device=cuda)
+
+    def splitk(out, accumulate):
+        ws.fill_(float("nan"))  # every partial is written before it is read
+        nat.call("eth_gemm_splitk", nat.ptr(ad), lda, int(a_k), nat.ptr(bd), ldb, int(b_k), nat.ptr(out), N, M, N, Kd,
+                 code, splits, int(accumulate), nat.ptr(ws), nat.stream_ptr(cuda))
+        return out.cpu()
+
     ref = 0.25 + a.float() @ b.float()
-    outs = []
-    for _ in range(2):
-        acc = torch.full((M, N), 0.25, dtype=torch.float32, device=cuda)
-        K.gemm(ad, bd, out=acc, accumulate=True)
-        outs.append(acc.cpu())
+    outs = [splitk(torch.full((M, N), 0.25, dtype=torch.float32, device=cuda), True) for _ in range(2)]
     err = (outs[0] - ref).abs().max().item()
     assert err <= 1e-4 * ref.abs().max().item(), f"split-K err {err}"
     assert torch.equal(outs[0], outs[1])
     # store form (C = A B): the same partial sums, written over garbage
-    st = torch.full((M, N), 9.0, dtype=torch.float32, device=cuda)
-    K.gemm(ad, bd, out=st, accumulate=False)
-    assert torch.equal(st.cpu() + 0.25, outs[0])  # one fp32 add of the same sum, either order
+    st = splitk(torch.full((M, N), 9.0, dtype=torch.float32, device=cuda), False)
+    assert torch.equal(st + 0.25, outs[0])  # one fp32 add of the same sum, either order
+    general = torch.full((M, N), 9.0, dtype=torch.float32, device=cuda)
+    ws.fill_(float("nan"))
+    nat.call("eth_gemm_splitk_out", nat.ptr(ad), lda, int(a_k), nat.ptr(bd), ldb, int(b_k), nat.ptr(general), N,
+             nat.ETH_F32, None, M, N, Kd, code, 0, 1.0, splits, nat.ptr(ws), nat.stream_ptr(cuda))
+    assert torch.equal(general.cpu(), st)
     # the single-pass kernel agrees to fp32 summation-order noise
     one = torch.full((M, N), 0.25, dtype=torch.float32, device=cuda)
-    lda = ad.stride(0) if a_k else ad.stride(1)
-    ldb = bd.stride(1) if b_k else bd.stride(0)
     nat.call("eth_gemm", nat.ptr(ad), lda, int(a_k), nat.ptr(bd), ldb, int(b_k), nat.ptr(one), N, nat.ETH_F32,
-             None, M, N, Kd, nat.dtype_code(torch.bfloat16), nat.GEMM_ACCUMULATE, 1.0, nat.stream_ptr(cuda))
+             None, M, N, Kd, code, nat.GEMM_ACCUMULATE, 1.0, nat.stream_ptr(cuda))
     assert (one.cpu() - outs[0]).abs().max().item() <= 1e-5 * ref.abs().max().item()
+
+
+@pytest.mark.parametrize("a_k,b_k", [(True, True), (True, False), (False, False), (False, True)])
+def test_gemm_takes_splitk_for_deep_products(cuda, a_k, b_k):
+    """A product K.gemm runs in splits: the bits of the split-K entry."""
+    from eth_amd import _native as nat
+
+    M, N, Kd = 512, 520, 16384
+    announce(f"gemm split-K chosen a_k={a_k} b_k={b_k} {M}x{N}x{Kd}")
+    gen = torch.Generator(device=cuda).manual_seed(5 + 2 * a_k + b_k)
+    ad = torch.randn(*((M, Kd) if a_k else (Kd, M)), device=cuda, generator=gen).bfloat16()
+    bd = torch.randn(*((N, Kd) if b_k else (Kd, N)), device=cuda, generator=gen).bfloat16()
+    av, bv = ad if a_k else ad.t(), bd.t() if b_k else bd
+    acc = torch.full((M, N), 0.25, dtype=torch.float32, device=cuda)
+    splits = K._splitk_splits(M, N, Kd, acc)
+    assert splits > 1 and K._splitk_pays(M, N, Kd, splits, int(a_k), int(b_k)) == splits * M * N
+    K.gemm(av, bv, out=acc, accumulate=True)
+    want = torch.full((M, N), 0.25, dtype=torch.float32, device=cuda)
+    ws = torch.full((splits * M * N,), float("nan"), device=cuda)
+    nat.call("eth_gemm_splitk", nat.ptr(ad), ad.stride(0), int(a_k), nat.ptr(bd), bd.stride(0), int(b_k),
+             nat.ptr(want), N, M, N, Kd, nat.dtype_code(torch.bfloat16), splits, 1, nat.ptr(ws), nat.stream_ptr(cuda))
+    assert torch.equal(acc, want)
+    ref = 0.25 + av.float().cpu() @ bv.float().cpu()
+    assert (acc.cpu() - ref).abs().max().item() <= 1e-4 * ref.abs().max().item()
 
 
 def test_gemm_rejects_bad_shapes(cuda):
