@@ -26,12 +26,15 @@
 //    stores.  m16 (v_mfma_f32_16x16x32, single-buffered fragments) serves
 //    the forward, data-gradient and weight-gradient products (for the last,
 //    both operands row-contiguous, through asm MFMAs); m32
-//    (v_mfma_f32_32x32x16) a row-contiguous A with a K-contiguous B.  Both
-//    need 16-byte aligned C rows; m16 takes any K % 64 == 0, and any K for
-//    weight gradients, m32 K % 128 == 0.
+//    (v_mfma_f32_32x32x16) a row-contiguous A with a K-contiguous B and
+//    K % 128 == 0.  Where K is no multiple of 64 (128 in the last layout) m16
+//    runs in an instantiation whose last k-tile is short (TAIL), in every
+//    layout: forward of [8448, 3648] x 416 took 77 us on 128x128 ring tiles
+//    and 68 on the register-staged ones before them, now 41; [12384, 14368] x
+//    1496 861, 686, now 485.  C rows must be aligned to four columns.
 //  * gemm_ring_kernel: 128x128 or 64x64 tiles with four LDS stages, for the
 //    grids that 256x256 tiles leave mostly idle and for every shape and
-//    alignment (any K % 8 == 0).
+//    alignment.
 // plan_tile() chooses among them by the time each would take.
 // Tiles are assigned XCD-aware (consecutive workgroups land on different
 // XCDs, so the tile id is remapped to give each XCD a contiguous range) and
@@ -314,13 +317,12 @@ __global__ void __launch_bounds__(256, 1) gemm256_m16_kernel(GemmArgs g) {
 
   const int span = (g.k_split ? min(g.K, kb + g.k_split) : g.K) - kb;
   const int nk = (span + BK - 1) / BK;
-  // TAIL: the last k-tile lacks rows of k (left of them are there; with
-  // left == 0 tail stays past it).  Weight gradients only, where K is the
-  // number of tokens, and an instantiation of their own (the branch in the
-  // loop costs 0.5 % of a layer's time): the other layouts' builtin MFMAs
-  // get their accumulators copied around with it (77 vs 51 us for
-  // [2048, 8192] x 2048), so they take K % 64 == 0 (model widths) here and
-  // leave other K to the ring kernel.
+  // TAIL: the last k-tile is short; its loads past K read zeros (left of its
+  // k are there; with left == 0 tail stays past it).  An instantiation of its
+  // own: the branch in the loop and the scalars it keeps (8 to 18 spilled to
+  // vector lanes with a row-contiguous operand) cost 0.5 % of a layer's time.
+  // Its MFMAs are asm in every layout: with the builtin ones the branch gets
+  // the accumulators copied around ([2048, 8192] x 2048: 77 vs 51 us).
   const int left = span % BK, tail = left ? nk - 1 : nk + 2;
   const rsrc_t ra = make_rsrc(g.A, g.a_bytes), rb = make_rsrc(g.B, g.b_bytes);
   // empty ranges: the loads issued past the last k-tile read zeros
@@ -398,7 +400,7 @@ __global__ void __launch_bounds__(256, 1) gemm256_m16_kernel(GemmArgs g) {
   fb[J] = B_K ? *reinterpret_cast<const uint4*>((BASE) + b_frag[KS] + (J) * 16 * BK) \
               : tr_frag((BASE) + b_frag[KS] + (J) * 16, LM);
 #define MM(I, J)                                  \
-  if constexpr (A_K)                              \
+  if constexpr (A_K && !TAIL)                     \
     acc[I][J] = mfma16<FP16>(fb[J], fa[I], acc[I][J]); \
   else                                            \
     mfma16_asm<FP16>(acc[I][J], fb[J], fa[I]);
@@ -461,7 +463,7 @@ __global__ void __launch_bounds__(256, 1) gemm256_m16_kernel(GemmArgs g) {
     ITER(smem1, smem, kt + 1)
   }
   // asm MFMAs: wait states before any instruction reads their accumulators
-  if constexpr (!A_K) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
+  if constexpr (!A_K || TAIL) asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" ::: "memory");
 #undef PIN_ACC
 #undef LIMIT_IF
 #undef ITER
@@ -1073,29 +1075,35 @@ static int launch_ring(const GemmArgs& a, int a_k, int b_k, hipStream_t s) {
 // for 64x64, whose 64 KB of LDS leaves room for a second) times the k-tiles of
 // 64 at the measured pace plus the prologue and epilogue.  A 256x256 k-tile
 // runs faster when half the CUs idle (more clock and bandwidth for the rest),
-// in a last round too.
-static double tile_time(int tile, int64_t M, int64_t N, int64_t K, int splits) {
+// in a last round too; less so where the rows of both operands start off
+// 128-byte lines (skew: both K-contiguous, K % 64 != 0), which also slows the
+// ring: alone, [2176, 3072] x 1000 forward took 30.3 us on wide tiles and 32.3
+// on 128x128 ones, [768, 7936] x 2016 45.9 and 48.3 on 64x64 ones, and
+// [1008, 6640] x 3928 89.5 on wide tiles (split in two, which is chosen, 69).
+static bool skewed(int64_t K, int a_kcontig, int b_kcontig) { return a_kcontig && b_kcontig && K % 64; }
+static double tile_time(int tile, int64_t M, int64_t N, int64_t K, int splits, bool skew) {
   const double tiles = (double)((M + tile - 1) / tile) * (double)((N + tile - 1) / tile) * splits;
   const double nk = (double)(((K + splits - 1) / splits + 63) / 64);
   if (tile == 256) {
     const double rounds = floor(tiles / 256), last = tiles - 256 * rounds;
     const double full = nk * 1.20 + 9.0;
-    return 3.0 + rounds * full + (last > 128 ? full : last > 0 ? nk * 0.93 + 9.0 : 0.0);
+    return 3.0 + rounds * full + (last > 128 ? full : last > 0 ? nk * (skew ? 1.08 : 0.93) + 9.0 : 0.0);
   }
-  if (tile == 128) return 2.0 + ceil(tiles / 256) * (nk * 0.52 + 6.0);
-  return tiles <= 256 ? 2.0 + nk * 0.24 + 1.0 : 1.0 + ceil(tiles / 512) * (nk * 0.36 + 2.7);
+  const double pace = skew ? 1.1 * nk : nk;
+  if (tile == 128) return 2.0 + ceil(tiles / 256) * (pace * 0.52 + 6.0);
+  return tiles <= 256 ? 2.0 + pace * 0.24 + 1.0 : 1.0 + ceil(tiles / 512) * (pace * 0.36 + 2.7);
 }
 
 // The tile that finishes first.  Measured on both sides of the lines (us, 256
 // / 128 / 64): [2048, 2048] x 2048 deep 39 / 24 / 29, [2048, 6144] x 2048 45 /
 // 66 / 76, [1024, 1024] x 4096 69 / 37 / 17, [1024, 4096] x 1024 24 / 16 / 18,
 // [3000, 2560] x 2560 48 / 53 / 66.
-static int plan_tile(int64_t M, int64_t N, int64_t K, bool wide) {
+static int plan_tile(int64_t M, int64_t N, int64_t K, bool wide, bool skew) {
   int best = 64;
-  double t = tile_time(64, M, N, K, 1);
+  double t = tile_time(64, M, N, K, 1, skew);
   for (int tile : {128, 256}) {
     if (tile == 256 && !wide) continue;
-    const double u = tile_time(tile, M, N, K, 1);
+    const double u = tile_time(tile, M, N, K, 1, skew);
     if (u <= t) {
       t = u;
       best = tile;
@@ -1107,16 +1115,20 @@ static int plan_tile(int64_t M, int64_t N, int64_t K, bool wide) {
 template <bool FP16>
 static int launch_256(const GemmArgs& a, int a_k, int b_k, hipStream_t s, int splits = 1) {
   const int tiles = ((a.M + 255) / 256) * ((a.N + 255) / 256) * splits;
+  const bool tail = a.K % 64;
   if (a_k && b_k)
-    gemm256_m16_kernel<true, true, FP16><<<tiles, 256, 0, s>>>(a);
-  else if (a_k && !b_k)
-    gemm256_m16_kernel<true, false, FP16><<<tiles, 256, 0, s>>>(a);
-  else if (!a_k && !b_k && a.K % 64)
-    gemm256_m16_kernel<false, false, FP16, true><<<tiles, 256, 0, s>>>(a);
-  else if (!a_k && !b_k)
-    gemm256_m16_kernel<false, false, FP16><<<tiles, 256, 0, s>>>(a);
-  else
-    gemm256_m32_kernel<false, true, FP16><<<tiles, 256, 0, s>>>(a);
+    tail ? gemm256_m16_kernel<true, true, FP16, true><<<tiles, 256, 0, s>>>(a)
+         : gemm256_m16_kernel<true, true, FP16><<<tiles, 256, 0, s>>>(a);
+  else if (a_k)
+    tail ? gemm256_m16_kernel<true, false, FP16, true><<<tiles, 256, 0, s>>>(a)
+         : gemm256_m16_kernel<true, false, FP16><<<tiles, 256, 0, s>>>(a);
+  else if (!b_k)
+    tail ? gemm256_m16_kernel<false, false, FP16, true><<<tiles, 256, 0, s>>>(a)
+         : gemm256_m16_kernel<false, false, FP16><<<tiles, 256, 0, s>>>(a);
+  else  // (m32: pairs of whole k-tiles, in every split alike)
+    a.K % (a.k_split ? a.k_split : 128) || a.k_split % 128
+        ? gemm256_m16_kernel<false, true, FP16, true><<<tiles, 256, 0, s>>>(a)
+        : gemm256_m32_kernel<false, true, FP16><<<tiles, 256, 0, s>>>(a);
   ETH_CHECK_LAUNCH("eth_gemm");
   return ETH_OK;
 }
@@ -1139,40 +1151,38 @@ static int launch_256(const GemmArgs& a, int a_k, int b_k, hipStream_t s, int sp
 struct GemmCut {
   int64_t m, n;
 };
-static GemmCut plan_cut(int64_t M, int64_t N, int64_t K, bool wide) {
+static GemmCut plan_cut(int64_t M, int64_t N, int64_t K, bool wide, bool skew) {
   GemmCut best{M, N};
   if (!wide) return best;
-  const int tile = plan_tile(M, N, K, wide);
+  const int tile = plan_tile(M, N, K, wide, skew);
   const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256, rounds = tm * tn / 256;
   if (tile != 256 || rounds < 1 || tm * tn % 256 == 0) return best;
   const int64_t last = tm * tn % 256;
-  double t = (K >= 1024 && last >= 24 && last <= 128 ? 0.98 : 0.93) * tile_time(256, M, N, K, 1);
-  auto rest = [&](int64_t m, int64_t n) { return tile_time(plan_tile(m, n, K, wide), m, n, K, 1); };
+  double t = (K >= 1024 && last >= 24 && last <= 128 ? 0.98 : 0.93) * tile_time(256, M, N, K, 1, skew);
+  auto rest = [&](int64_t m, int64_t n) { return tile_time(plan_tile(m, n, K, wide, skew), m, n, K, 1, skew); };
   const int64_t m1 = rounds * 256 / tn * 256, n1 = rounds * 256 / tm * 256;
   if (m1 > 0 && m1 < M) {
-    const double u = tile_time(256, m1, N, K, 1) + rest(M - m1, N);
+    const double u = tile_time(256, m1, N, K, 1, skew) + rest(M - m1, N);
     if (u < t) {
       t = u;
       best = GemmCut{m1, N};
     }
   }
   if (n1 > 0 && n1 < N) {
-    const double u = tile_time(256, M, n1, K, 1) + rest(M, N - n1);
+    const double u = tile_time(256, M, n1, K, 1, skew) + rest(M, N - n1);
     if (u < t) best = GemmCut{M, n1};
   }
   return best;
 }
 
-// The 256x256 kernels take C rows of whole four-column vectors (vector
-// stores), a C extent plus one tile of rows below 2 GiB (their buffer offsets)
-// and the K of each layout.
-static bool wide_takes(int64_t M, int64_t N, int64_t K, int a_kcontig, int b_kcontig, int64_t ldc, int esz,
-                       bool c_vec) {
-  return K % (a_kcontig ? 64 : b_kcontig ? 128 : 8) == 0 && c_vec && ((M + 255) * ldc + N) * esz < (1LL << 31);
+// The 256x256 kernels take C rows of whole four-column vectors (vector stores)
+// and a C extent plus one tile of rows below 2 GiB (their buffer offsets).
+static bool wide_takes(int64_t M, int64_t N, int64_t ldc, int esz, bool c_vec) {
+  return c_vec && ((M + 255) * ldc + N) * esz < (1LL << 31);
 }
 
 static int launch_planned(const GemmArgs& a, int a_k, int b_k, bool fp16, bool wide, hipStream_t s) {
-  switch (plan_tile(a.M, a.N, a.K, wide)) {
+  switch (plan_tile(a.M, a.N, a.K, wide, skewed(a.K, a_k, b_k))) {
     case 256:
       return fp16 ? launch_256<true>(a, a_k, b_k, s) : launch_256<false>(a, a_k, b_k, s);
     case 128:
@@ -1229,10 +1239,10 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
   a.c_vec = ldc % 4 == 0 && N % 4 == 0 && ((uintptr_t)C % (4 * esz)) == 0;
   a.k_split = 0;
   a.c_split_stride = 0;
-  const bool wide = wide_takes(M, N, K, a_kcontig, b_kcontig, ldc, esz, a.c_vec);
+  const bool wide = wide_takes(M, N, ldc, esz, a.c_vec);
   a.c_bytes = wide ? (uint32_t)(((M - 1) * ldc + N) * esz) : 0;
   const bool fp16 = in_dtype == ETH_F16;
-  const GemmCut cut = plan_cut(M, N, K, wide);
+  const GemmCut cut = plan_cut(M, N, K, wide, skewed(K, a_kcontig, b_kcontig));
   if (cut.m == M && cut.n == N) return launch_planned(a, a_kcontig, b_kcontig, fp16, wide, s);
   // the part of whole rounds, then the rest (rows or columns of C)
   const int64_t M2 = M - cut.m, N2 = N - cut.n;
@@ -1267,14 +1277,14 @@ extern "C" int eth_gemm_plan(int64_t M, int64_t N, int64_t K, int a_kcontig, int
   ETH_CHECK_ARG(valid_dtype(c_dtype), "eth_gemm_plan: bad output dtype %d", c_dtype);
   ETH_CHECK_ARG(M > 0 && N > 0 && K > 0 && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31) && ldc >= N,
                 "eth_gemm_plan: bad shape %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
-  const bool wide = wide_takes(M, N, K, a_kcontig, b_kcontig, ldc, c_dtype == ETH_F32 ? 4 : 2,
-                               ldc % 4 == 0 && N % 4 == 0);
-  const GemmCut cut = plan_cut(M, N, K, wide);
-  plan[0] = plan_tile(cut.m, cut.n, K, wide);
+  const bool wide = wide_takes(M, N, ldc, c_dtype == ETH_F32 ? 4 : 2, ldc % 4 == 0 && N % 4 == 0);
+  const bool skew = skewed(K, a_kcontig, b_kcontig);
+  const GemmCut cut = plan_cut(M, N, K, wide, skew);
+  plan[0] = plan_tile(cut.m, cut.n, K, wide, skew);
   plan[1] = cut.m;
   plan[2] = cut.n;
   const int64_t m = cut.m < M ? M - cut.m : M, n = cut.n < N ? N - cut.n : N;
-  plan[3] = cut.m == M && cut.n == N ? 0 : plan_tile(m, n, K, wide);
+  plan[3] = cut.m == M && cut.n == N ? 0 : plan_tile(m, n, K, wide, skew);
   return ETH_OK;
 }
 
@@ -1340,12 +1350,13 @@ extern "C" int64_t eth_gemm_splitk_workspace(int64_t M, int64_t N, int splits) {
   return splits > 0 && M > 0 && N > 0 ? (int64_t)splits * M * N * 4 : 0;
 }
 
-extern "C" int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits) {
+extern "C" int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits, int a_kcontig, int b_kcontig) {
   if (M <= 0 || N <= 0 || K <= 0 || splits < 2) return 0;
   // the second kernel: a launch, and the partials and C at about 4.5 TB/s
   const double sum = 5.0 + 4.0 * (double)M * (double)N * (splits + 1) / 4.5e6;
-  const double one = tile_time(plan_tile(M, N, K, true), M, N, K, 1);
-  return tile_time(256, M, N, K, splits) + sum < one;
+  const bool skew = skewed(K, a_kcontig, b_kcontig);
+  const double one = tile_time(plan_tile(M, N, K, true, skew), M, N, K, 1, skew);
+  return tile_time(256, M, N, K, splits, skew) + sum < one;
 }
 
 extern "C" int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb,
@@ -1358,9 +1369,7 @@ extern "C" int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, co
   ETH_CHECK_ARG(splits >= 1 && splits <= 16, "eth_gemm_splitk: splits must be in [1, 16] (got %d)", splits);
   ETH_CHECK_ARG(M > 0 && N > 0 && K > 0 && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31),
                 "eth_gemm_splitk: bad shape %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
-  ETH_CHECK_ARG(K % (a_kcontig ? 64 : b_kcontig ? 128LL * splits : 8) == 0,
-                "eth_gemm_splitk: K (%lld) must be a multiple of 64 (K-contiguous A), 8 (both operands "
-                "row-contiguous) or 128 * splits", (long long)K);
+  ETH_CHECK_ARG(K % 8 == 0, "eth_gemm_splitk: K (%lld) must be a multiple of 8", (long long)K);
   const int esz = c_dtype == ETH_F32 ? 4 : 2;
   ETH_CHECK_ARG(N % 4 == 0 && ldc % 4 == 0 && ldc >= N && ((uintptr_t)C % (4 * esz)) == 0 &&
                     ((uintptr_t)workspace & 15) == 0,
@@ -1393,10 +1402,9 @@ extern "C" int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, co
   a.flags = 0;
   a.alpha = 1.0f;
   a.c_bytes = (uint32_t)(slice * 4);
-  // whole k-tiles per split (pairs for m32), the last split shorter; few
-  // k-tiles may leave fewer splits than asked for
-  const int unit = !a_kcontig && b_kcontig ? 128 : 64;
-  a.k_split = (int)(((K + splits - 1) / splits + unit - 1) / unit * unit);
+  // whole k-tiles per split, the last split shorter; few k-tiles may leave
+  // fewer splits than asked for
+  a.k_split = (int)(((K + splits - 1) / splits + 63) / 64 * 64);
   splits = (int)((K + a.k_split - 1) / a.k_split);
   a.c_split_stride = slice;
   hipStream_t s = (hipStream_t)stream;

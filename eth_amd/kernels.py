@@ -93,9 +93,9 @@ def _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig):
     """fp32 elements of workspace if the split-K form takes this product and
     finishes before the plain one, else 0 (sizes and layout only; the smaller
     tiles fill the chip without a second pass unless K is deep)."""
-    if splits < 2 or K % (64 if a_kcontig else 128 * splits if b_kcontig else 8) or 4 * (M + 256) * N >= 2**31:
+    if splits < 2 or K % 8 or 4 * (M + 256) * N >= 2**31:
         return 0
-    if not nat.value("eth_gemm_splitk_pays", M, N, K, splits):
+    if not nat.value("eth_gemm_splitk_pays", M, N, K, splits, a_kcontig, b_kcontig):
         return 0
     return nat.value("eth_gemm_splitk_workspace", M, N, splits) // 4
 

@@ -238,8 +238,8 @@ int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t l
              int64_t M, int64_t N, int64_t K, int in_dtype, int flags, float alpha,
              void* stream);
 
-/* What eth_gemm launches for such a product with 4-column aligned C rows of
- * stride ldc (host only, no launch): plan[0] the tile (256, 128 or 64) of the
+/* What eth_gemm launches for such a product with C at an address aligned to
+ * four columns and rows of stride ldc (host only, no launch): plan[0] the tile (256, 128 or 64) of the
  * launch over the rows [0, plan[1]) and columns [0, plan[2]) of C; where that
  * is not all of C, plan[3] is the tile of the second launch over the rest,
  * else 0. */
@@ -260,16 +260,15 @@ int eth_gemm_splitk(const void* A, int64_t lda, int a_kcontig, const void* B, in
                     int accumulate, float* workspace, void* stream);
 int64_t eth_gemm_splitk_workspace(int64_t M, int64_t N, int splits);
 /* The same for every output eth_gemm writes: C of c_dtype, alpha and bias
- * applied to the sum of the partials, which is rounded once.  K % 64 == 0
- * with a K-contiguous A, any K % 8 == 0 with both operands row-contiguous,
- * K % (128 * splits) == 0 otherwise; N % 4 == 0 and C rows aligned to four
- * columns.  Deterministic; the partials stay fp32. */
+ * applied to the sum of the partials, which is rounded once.  K % 8 == 0,
+ * N % 4 == 0 and C rows aligned to four columns.  Deterministic; the partials
+ * stay fp32. */
 int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb, int b_kcontig,
                         void* C, int64_t ldc, int c_dtype, const void* bias, int64_t M, int64_t N, int64_t K,
                         int in_dtype, int flags, float alpha, int splits, float* workspace, void* stream);
 /* 1 where the split-K form with `splits` is expected to finish before
  * eth_gemm on the same [M, N] x K product, else 0. */
-int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits);
+int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits, int a_kcontig, int b_kcontig);
 
 /* ------------------------------------------------------------------------
  * LayerNorm (bf16/fp16 rows of `cols` elements, cols % 8 == 0, <= 8192).

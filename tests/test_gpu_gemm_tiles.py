@@ -62,12 +62,11 @@ def test_products_at_tile_edges(cuda, M, N, Kd, a_k, b_k):
     _products(cuda, M, N, Kd, a_k, b_k)
 
 
-@pytest.mark.parametrize("a_k,b_k,M,N,Kd", [
+@pytest.mark.parametrize("a_k,b_k", LAYOUTS)
+@pytest.mark.parametrize("M,N,Kd", [
     # ragged edges, 33 to 36 k-tiles (every remainder of a trip round the
     # four stages), the last one short in three of them
-    *((a_k, b_k, 1928, 1032, Kd) for a_k, b_k in LAYOUTS for Kd in (2056, 2120, 2184, 2304)),
-    # two rounds of few k-tiles (weight gradients take wide tiles there)
-    (True, True, 4088, 2044, 328), (True, False, 4088, 2040, 328), (False, True, 4088, 2044, 328),
+    (1928, 1032, 2056), (1928, 1032, 2120), (1928, 1032, 2184), (1928, 1032, 2304),
 ])
 def test_128_tiles(cuda, a_k, b_k, M, N, Kd):
     assert _plan(M, N, Kd, a_k, b_k, torch.float32) == (128, M, N, 0)
@@ -90,25 +89,41 @@ def _products(cuda, M, N, Kd, a_k, b_k):
         assert torch.equal(acc, once)
 
 
-@pytest.mark.parametrize("a_k,b_k,Kd", [
-    # weight gradients: any number of tokens, the last k-tile short (one,
-    # two, three, four and six k-tiles)
-    (False, False, 8), (False, False, 72), (False, False, 184), (False, False, 200), (False, False, 328),
-    # forward and data gradients: an odd number of whole k-tiles
-    (True, True, 64), (True, True, 192), (True, False, 64), (True, False, 192),
+@pytest.mark.parametrize("a_k,b_k", LAYOUTS)
+@pytest.mark.parametrize("Kd,dtype", [
+    # the last k-tile short: one, two, three, four and six k-tiles
+    (8, torch.bfloat16), (72, torch.float16), (184, torch.bfloat16), (200, torch.bfloat16), (328, torch.float16),
+    # an odd number of whole k-tiles
+    (64, torch.bfloat16), (192, torch.float16),
 ])
-def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd):
+def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd, dtype):
     """128 tiles of 256x256 with ragged edges, every k-tile count the loop
     and its prologue treat apart."""
     M, N = 4088, 2040
-    assert _plan(M, N, Kd, a_k, b_k, torch.float32) == _plan(M, N, Kd, a_k, b_k, torch.bfloat16) == (256, M, N, 0)
+    assert _plan(M, N, Kd, a_k, b_k, torch.float32) == _plan(M, N, Kd, a_k, b_k, dtype) == (256, M, N, 0)
     announce(f"gemm wide {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
-    a, b, ad, bd = _operands(M, N, Kd, a_k, b_k, torch.bfloat16, cuda, Kd)
+    a, b, ad, bd = _operands(M, N, Kd, a_k, b_k, dtype, cuda, Kd)
     ref, mag = a @ b, a.abs() @ b.abs()
     acc = torch.full((M, N), 0.5, device=cuda)
     K.gemm(ad, bd, out=acc, accumulate=True)
     _check(acc, ref + 0.5, mag + 0.5, Kd, torch.float32, "accumulated")
-    _check(K.gemm(ad, bd), ref, mag, Kd, torch.bfloat16, "16-bit")
+    _check(K.gemm(ad, bd), ref, mag, Kd, dtype, "16-bit")
+
+
+@pytest.mark.parametrize("a_k,b_k", LAYOUTS)
+def test_short_k_tile_reads_nothing_past_k(cuda, a_k, b_k):
+    """K columns of operands whose rows go on with NaN: what lies past K in
+    memory is no part of the product."""
+    M, N, Kd = 4088, 2040, 200
+    announce(f"gemm wide views {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
+    a, b, _, _ = _operands(M, N, Kd, a_k, b_k, torch.bfloat16, cuda, 3)
+    wide_a, wide_b = (torch.full((M, Kd + 56) if a_k else (Kd + 56, M), float("nan"), dtype=torch.bfloat16, device=cuda),
+                      torch.full((N, Kd + 56) if b_k else (Kd + 56, N), float("nan"), dtype=torch.bfloat16, device=cuda))
+    ad = wide_a[:, :Kd] if a_k else wide_a[:Kd].t()
+    bd = wide_b[:, :Kd].t() if b_k else wide_b[:Kd]
+    ad.copy_(a)
+    bd.copy_(b)
+    _check(K.gemm(ad, bd), a @ b, a.abs() @ b.abs(), Kd, torch.bfloat16, "views")
 
 
 @pytest.mark.parametrize("a_k,b_k,M,N,Kd,dtype,plan", [
@@ -122,6 +137,7 @@ def test_wide_tiles_any_depth(cuda, a_k, b_k, Kd):
     (True, True, 8192, 2304, 512, torch.bfloat16, (256, 8192, 2048, 64)),
     (True, False, 8184, 2312, 512, torch.float16, (256, 8184, 2048, 128)),
     (False, False, 8184, 2312, 520, torch.float16, (256, 8184, 2048, 128)),
+    (True, True, 8184, 2308, 520, torch.bfloat16, (256, 8184, 2048, 128)),
     (False, True, 8184, 2308, 512, torch.bfloat16, (256, 8184, 2048, 128)),
     # a rest of rows of the same layout
     (False, True, 2552, 7684, 512, torch.float16, (256, 2048, 7684, 128)),
@@ -152,6 +168,11 @@ def test_products_past_whole_rounds(cuda, a_k, b_k, M, N, Kd, dtype, plan):
     (True, False, 1984, 16),  # 31 k-tiles: two each, the last split one
     (False, False, 200, 16),  # fewer k-tiles than splits, the last one short
     (False, True, 512, 2),
+    (True, True, 1000, 5),    # four k-tiles a split, the last split with a short one
+    (True, False, 264, 2),    # the last split two k-tiles, one of them of a single chunk
+    (False, True, 576, 3),    # three k-tiles a split
+    (False, True, 648, 4),    # an odd count and a short k-tile
+    (False, True, 640, 4),    # pairs of k-tiles, the last split an odd one
 ])
 def test_splitk_every_output(cuda, a_k, b_k, Kd, splits):
     M, N = 264, 136
@@ -177,14 +198,13 @@ def test_splitk_every_output(cuda, a_k, b_k, Kd, splits):
 
 def test_deep_product_takes_splits(cuda):
     """A 16-bit output of two wide tiles, 16448 deep: split-K, the same bits
-    every time, and refused where the layout's K does not allow it."""
+    every time, and refused where the plain product is."""
     M, N, Kd = 256, 512, 16448
     announce(f"gemm deep {M}x{N}x{Kd}")
     out = torch.empty(M, N, dtype=torch.bfloat16, device=cuda)
     splits = K._splitk_splits(M, N, Kd, out)
-    assert splits == 16 and K._splitk_pays(M, N, Kd, splits, 1, 0)
-    assert not K._splitk_pays(M, N, Kd + 8, splits, 1, 0) and not K._splitk_pays(M, N, Kd, splits, 0, 1)
-    assert not K._splitk_pays(2048, 2048, 2048, 2, 1, 1)
+    assert splits == 16 and K._splitk_pays(M, N, Kd, splits, 1, 0) and K._splitk_pays(M, N, Kd + 8, splits, 1, 0)
+    assert not K._splitk_pays(M, N, Kd + 4, splits, 1, 0) and not K._splitk_pays(2048, 2048, 2048, 2, 1, 1)
     # half a round of wide tiles splits in two, one tile more does not
     half = torch.empty(2048, 4096, dtype=torch.bfloat16, device=cuda)
     assert K._splitk_splits(2048, 4096, 16384, half) == 2 and K._splitk_pays(2048, 4096, 16384, 2, 1, 1)

@@ -59,7 +59,7 @@ def test_struct_layouts_match_header():
 def test_gemm_plan_covers_the_output():
     """The launches eth_gemm plans: one of three tiles over whole rows or whole
     columns of C, the rest in a second; 256x256 only where that kernel takes
-    the depth and the C rows."""
+    the C rows."""
     import ctypes
     import random
 
@@ -74,13 +74,13 @@ def test_gemm_plan_covers_the_output():
         M, N = (int(2 ** rng.uniform(0, 14)) for _ in range(2))
         K = 8 * int(2 ** rng.uniform(0, 11))
         if rng.random() < 0.5:
-            N, K = -(-N // 8) * 8, -(-K // 128) * 128
+            N = -(-N // 8) * 8
         a_k, b_k, ldc = rng.randrange(2), rng.randrange(2), N + rng.choice((0, 0, 4, 1))
         tile, m, n, rest = plan(M, N, K, a_k, b_k, ldc)
         assert tile in (64, 128, 256) and 0 < m <= M and 0 < n <= N and (m == M or n == N)
         assert (rest == 0) == ((m, n) == (M, N)) and rest in (0, 64, 128, 256)
         if 256 in (tile, rest):
-            assert N % 4 == 0 and ldc % 4 == 0 and K % (64 if a_k else 128 if b_k else 8) == 0
+            assert N % 4 == 0 and ldc % 4 == 0
         if rest:
             assert tile == 256 and m % 256 == 0 or n % 256 == 0
             # whole rounds, but for the last tile row or column of the other side
