@@ -21,9 +21,18 @@ from .distributed import grad_written, main_grad_target, materialize_main_grad
 
 
 # open overlapped_wgrad contexts (of every thread) and the stream that the
-# first of them was entered on
+# first of them was entered on, as (device index, handle)
 _overlap = {"wgrad": 0, "home": None}
 _overlap_lock = threading.Lock()
+
+
+def _here(index):
+    return index, torch._C._cuda_getCurrentRawStream(index)
+
+
+def _stream(here):
+    index, handle = here
+    return torch.cuda.ExternalStream(handle, device=index) if handle else torch.cuda.default_stream(index)
 
 
 class overlapped_wgrad:
@@ -39,8 +48,8 @@ class overlapped_wgrad:
     def __enter__(self):
         self._mark = K.side_mark()
         with _overlap_lock:
-            if _overlap["wgrad"] == 0:
-                _overlap["home"] = torch.cuda.current_stream() if torch.cuda.is_initialized() else None
+            if _overlap["wgrad"] == 0 and torch.cuda.is_initialized():
+                _overlap["home"] = _here(torch._C._cuda_getDevice())
             _overlap["wgrad"] += 1
             self._home = _overlap["home"]
         return self
@@ -50,10 +59,9 @@ class overlapped_wgrad:
             _overlap["wgrad"] -= 1
             if _overlap["wgrad"] == 0:
                 _overlap["home"] = None
-        if self._home is not None:
-            now = torch.cuda.current_stream(self._home.device)
-            if now != self._home:
-                now.wait_stream(self._home)
+        home = self._home
+        if home is not None and _here(home[0]) != home:
+            torch.cuda.current_stream(home[0]).wait_stream(_stream(home))
         K.join_side_streams(since=self._mark)
         return False
 
@@ -108,21 +116,22 @@ def _wgrad(weight, dy2, x2, mg, accumulate):
     if not _overlap["wgrad"] or not dy2.is_cuda:
         K.gemm(dy2.t(), x2, out=mg, accumulate=accumulate)
         return
-    main, home = torch.cuda.current_stream(dy2.device), _overlap["home"]
-    if main == home and 2.0 * dy2.numel() * x2.shape[1] < _SIDE_MIN_FLOPS:
+    device, home = dy2.device, _overlap["home"]
+    here = _here(device.index)
+    if here == home and 2.0 * dy2.numel() * x2.shape[1] < _SIDE_MIN_FLOPS:
         if getattr(weight, "_eth_side_grad", False):
-            main.wait_stream(K.side_stream(dy2.device))
+            torch.cuda.current_stream(device).wait_stream(K.side_stream(device))
         weight._eth_side_grad = False
         K.gemm(dy2.t(), x2, out=mg, accumulate=accumulate)
         return
     # the weight gradient only feeds main_grad: it runs on a side stream,
     # overlapped with the data-gradient chain, and is joined before the
     # gradient sync reads the buffer
-    side = K.side_stream(dy2.device)
+    side = K.side_stream(device)
     K.mark_side_launch()
-    side.wait_stream(main)
-    if main != home and home is not None and not getattr(weight, "_eth_side_grad", True):
-        side.wait_stream(home)
+    side.wait_stream(torch.cuda.current_stream(device))
+    if here != home and home is not None and not getattr(weight, "_eth_side_grad", True):
+        side.wait_stream(_stream(home))
     weight._eth_side_grad = True
     with torch.cuda.stream(side):
         K.gemm(dy2.t(), x2, out=mg, accumulate=accumulate)

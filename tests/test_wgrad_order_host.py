@@ -48,8 +48,15 @@ class Streams:
     def __init__(self, monkeypatch):
         self.main, self.side, self.other, self.third = (Stream(n) for n in ("main", "side", "other", "third"))
         self.now, self.products = self.main, []
+        self.of_handle = dict(enumerate((self.main, self.side, self.other, self.third)))
+        for handle, stream in self.of_handle.items():
+            stream.handle = handle
         monkeypatch.setattr(torch.cuda, "is_initialized", lambda: True)
         monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: self.now)
+        monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: 0, raising=False)
+        monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: self.now.handle, raising=False)
+        monkeypatch.setattr(torch.cuda, "default_stream", lambda device: self.main)
+        monkeypatch.setattr(torch.cuda, "ExternalStream", lambda handle, device: self.of_handle[handle])
         monkeypatch.setattr(torch.cuda, "stream", self.on)
         monkeypatch.setattr(K, "_side", {DEVICE: self.side})
         monkeypatch.setattr(K, "gemm", self.product)
