@@ -130,7 +130,7 @@ VALUE_SIGNATURES = {
     "eth_bias_gelu_bwd_workspace": ([_I64, _I64], _I64),
     "eth_col_sum_workspace": ([_I64, _I64], _I64),
     "eth_gemm_splitk_workspace": ([_I64, _I64, _I32], _I64),
-    "eth_gemm_splitk_pays": ([_I64, _I64, _I64, _I32, _I32, _I32], _I64),
+    "eth_gemm_splitk_pays": ([_I64, _I64, _I64, _I32, _I32, _I32, _I32], _I64),
     "eth_embedding_bwd_workspace": ([_I64, _I64], _I64),
 }
 GEMM_ACCUMULATE, GEMM_BIAS = 1, 2

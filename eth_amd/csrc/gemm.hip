@@ -1069,41 +1069,60 @@ static int launch_ring(const GemmArgs& a, int a_k, int b_k, hipStream_t s) {
   return ETH_OK;
 }
 
-// Microseconds one launch of TILE x TILE tiles takes, fitted to sweeps of
-// transformer-layer products from 256^3 to [3000, 2560] x [10240, 2560] (bf16,
-// all three layouts; within about 15 %): rounds of one workgroup per CU (two
-// for 64x64, whose 64 KB of LDS leaves room for a second) times the k-tiles of
-// 64 at the measured pace plus the prologue and epilogue.  A 256x256 k-tile
-// runs faster when half the CUs idle (more clock and bandwidth for the rest),
-// in a last round too; less so where the rows of both operands start off
-// 128-byte lines (skew: both K-contiguous, K % 64 != 0), which also slows the
-// ring: alone, [2176, 3072] x 1000 forward took 30.3 us on wide tiles and 32.3
-// on 128x128 ones, [768, 7936] x 2016 45.9 and 48.3 on 64x64 ones, and
-// [1008, 6640] x 3928 89.5 on wide tiles (split in two, which is chosen, 69).
-static bool skewed(int64_t K, int a_kcontig, int b_kcontig) { return a_kcontig && b_kcontig && K % 64; }
-static double tile_time(int tile, int64_t M, int64_t N, int64_t K, int splits, bool skew) {
+// What a product's time depends on besides its sizes: an fp32 output (the
+// accumulating epilogue reads C too), and operands whose rows start off
+// 128-byte lines, where every load touches a line more: both K-contiguous
+// (skew_k), or one or two row-contiguous (skew_r).  Sizes stand for strides:
+// rows are rarely padded.
+struct GemmForm {
+  bool f32, skew_k;
+  int skew_r;
+};
+static GemmForm gemm_form(int64_t M, int64_t N, int64_t K, int a_kcontig, int b_kcontig, bool f32) {
+  return GemmForm{f32, a_kcontig && b_kcontig && K % 64 != 0, (!a_kcontig && M % 64 != 0) + (!b_kcontig && N % 64 != 0)};
+}
+
+// Microseconds one launch of TILE x TILE tiles takes, fitted to sweeps (within
+// about 15 %): rounds of one workgroup per CU (two for 64x64, whose 64 KB of
+// LDS leaves room for a second) times the k-tiles of 64 at the measured pace
+// plus the prologue and epilogue.  A 256x256 k-tile runs faster when half the
+// CUs idle (more clock and bandwidth for the rest), in a last round too, and
+// at full pace with a full one.  Past one round deep products on 64x64 tiles
+// lose the L2 (their workgroups drift apart in k), and rows off 128-byte lines
+// cost them most.  Measured where an earlier form of this was wrong (us):
+// weight gradients on wide tiles / two splits, [3328, 2048] x 3584 tokens 74 /
+// 66, [1536, 3200] x 2560 54 / 47; on 64x64 / two splits, [2456, 1544] x 10240
+// 209 / 106; 128x128 / wide, [9216, 832] x 2688 60 / 53, [600, 12816] x 1792
+// 45 / 38; forward with K off a line, wide / 128x128, [2176, 3072] x 1000
+// 30.3 / 32.3, wide / 64x64, [768, 7936] x 2016 45.9 / 48.3, wide / two
+// splits, [1008, 6640] x 3928 89 / 69.
+static double tile_time(int tile, int64_t M, int64_t N, int64_t K, int splits, GemmForm form) {
   const double tiles = (double)((M + tile - 1) / tile) * (double)((N + tile - 1) / tile) * splits;
   const double nk = (double)(((K + splits - 1) / splits + 63) / 64);
+  const double f = form.f32 && splits == 1 ? 1.0 : 0.0, ring = form.skew_k ? 1.1 : 1.0;
   if (tile == 256) {
-    const double rounds = floor(tiles / 256), last = tiles - 256 * rounds;
-    const double full = nk * 1.20 + 9.0;
-    return 3.0 + rounds * full + (last > 128 ? full : last > 0 ? nk * (skew ? 1.08 : 0.93) + 9.0 : 0.0);
+    const double rounds = floor(tiles / 256), last = tiles - 256 * rounds, edge = 9.0 + 4.8 * f;
+    double pace = 0.93 + 0.27 * std::max(0.0, last - 128) / 128;
+    if (form.skew_k) pace = std::max(pace, 1.08);
+    return 3.0 + rounds * (nk * 1.20 + edge) + (last > 0 ? nk * pace + edge : 0.0);
   }
-  const double pace = skew ? 1.1 * nk : nk;
-  if (tile == 128) return 2.0 + ceil(tiles / 256) * (pace * 0.52 + 6.0);
-  return tiles <= 256 ? 2.0 + pace * 0.24 + 1.0 : 1.0 + ceil(tiles / 512) * (pace * 0.36 + 2.7);
+  if (tile == 128) return 2.0 + ceil(tiles / 256) * (nk * 0.52 * ring + 6.0 + 3.3 * f);
+  if (tiles <= 256) return 3.0 + nk * 0.24 * (ring + 0.08 * form.skew_r) + 0.8 * f;
+  const double deep = std::min(1.0, std::max(0.0, (nk - 32.0) / 96.0));
+  const double lines = form.skew_k ? 0.2 : 0.2 * form.skew_r;
+  return 1.0 + ceil(tiles / 512) * (nk * 0.36 * (1.0 + lines + 0.3 * deep) + 2.7 + 1.5 * f);
 }
 
 // The tile that finishes first.  Measured on both sides of the lines (us, 256
 // / 128 / 64): [2048, 2048] x 2048 deep 39 / 24 / 29, [2048, 6144] x 2048 45 /
 // 66 / 76, [1024, 1024] x 4096 69 / 37 / 17, [1024, 4096] x 1024 24 / 16 / 18,
 // [3000, 2560] x 2560 48 / 53 / 66.
-static int plan_tile(int64_t M, int64_t N, int64_t K, bool wide, bool skew) {
+static int plan_tile(int64_t M, int64_t N, int64_t K, bool wide, GemmForm form) {
   int best = 64;
-  double t = tile_time(64, M, N, K, 1, skew);
+  double t = tile_time(64, M, N, K, 1, form);
   for (int tile : {128, 256}) {
     if (tile == 256 && !wide) continue;
-    const double u = tile_time(tile, M, N, K, 1, skew);
+    const double u = tile_time(tile, M, N, K, 1, form);
     if (u <= t) {
       t = u;
       best = tile;
@@ -1151,25 +1170,25 @@ static int launch_256(const GemmArgs& a, int a_k, int b_k, hipStream_t s, int sp
 struct GemmCut {
   int64_t m, n;
 };
-static GemmCut plan_cut(int64_t M, int64_t N, int64_t K, bool wide, bool skew) {
+static GemmCut plan_cut(int64_t M, int64_t N, int64_t K, bool wide, GemmForm form) {
   GemmCut best{M, N};
   if (!wide) return best;
-  const int tile = plan_tile(M, N, K, wide, skew);
+  const int tile = plan_tile(M, N, K, wide, form);
   const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256, rounds = tm * tn / 256;
   if (tile != 256 || rounds < 1 || tm * tn % 256 == 0) return best;
   const int64_t last = tm * tn % 256;
-  double t = (K >= 1024 && last >= 24 && last <= 128 ? 0.98 : 0.93) * tile_time(256, M, N, K, 1, skew);
-  auto rest = [&](int64_t m, int64_t n) { return tile_time(plan_tile(m, n, K, wide, skew), m, n, K, 1, skew); };
+  double t = (K >= 1024 && last >= 24 && last <= 128 ? 0.98 : 0.93) * tile_time(256, M, N, K, 1, form);
+  auto rest = [&](int64_t m, int64_t n) { return tile_time(plan_tile(m, n, K, wide, form), m, n, K, 1, form); };
   const int64_t m1 = rounds * 256 / tn * 256, n1 = rounds * 256 / tm * 256;
   if (m1 > 0 && m1 < M) {
-    const double u = tile_time(256, m1, N, K, 1, skew) + rest(M - m1, N);
+    const double u = tile_time(256, m1, N, K, 1, form) + rest(M - m1, N);
     if (u < t) {
       t = u;
       best = GemmCut{m1, N};
     }
   }
   if (n1 > 0 && n1 < N) {
-    const double u = tile_time(256, M, n1, K, 1, skew) + rest(M, N - n1);
+    const double u = tile_time(256, M, n1, K, 1, form) + rest(M, N - n1);
     if (u < t) best = GemmCut{M, n1};
   }
   return best;
@@ -1181,8 +1200,8 @@ static bool wide_takes(int64_t M, int64_t N, int64_t ldc, int esz, bool c_vec) {
   return c_vec && ((M + 255) * ldc + N) * esz < (1LL << 31);
 }
 
-static int launch_planned(const GemmArgs& a, int a_k, int b_k, bool fp16, bool wide, hipStream_t s) {
-  switch (plan_tile(a.M, a.N, a.K, wide, skewed(a.K, a_k, b_k))) {
+static int launch_planned(const GemmArgs& a, int a_k, int b_k, bool fp16, bool wide, GemmForm form, hipStream_t s) {
+  switch (plan_tile(a.M, a.N, a.K, wide, form)) {
     case 256:
       return fp16 ? launch_256<true>(a, a_k, b_k, s) : launch_256<false>(a, a_k, b_k, s);
     case 128:
@@ -1242,8 +1261,9 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
   const bool wide = wide_takes(M, N, ldc, esz, a.c_vec);
   a.c_bytes = wide ? (uint32_t)(((M - 1) * ldc + N) * esz) : 0;
   const bool fp16 = in_dtype == ETH_F16;
-  const GemmCut cut = plan_cut(M, N, K, wide, skewed(K, a_kcontig, b_kcontig));
-  if (cut.m == M && cut.n == N) return launch_planned(a, a_kcontig, b_kcontig, fp16, wide, s);
+  const GemmForm form = gemm_form(M, N, K, a_kcontig, b_kcontig, c_dtype == ETH_F32);
+  const GemmCut cut = plan_cut(M, N, K, wide, form);
+  if (cut.m == M && cut.n == N) return launch_planned(a, a_kcontig, b_kcontig, fp16, wide, form, s);
   // the part of whole rounds, then the rest (rows or columns of C)
   const int64_t M2 = M - cut.m, N2 = N - cut.n;
   GemmArgs r = a;
@@ -1267,8 +1287,8 @@ extern "C" int eth_gemm(const void* A, int64_t lda, int a_kcontig, const void* B
     if (r.bias) r.bias += cut.n;
     r.c_bytes = (uint32_t)(((M - 1) * ldc + N2) * esz);
   }
-  const int rc = launch_planned(a, a_kcontig, b_kcontig, fp16, wide, s);
-  return rc != ETH_OK ? rc : launch_planned(r, a_kcontig, b_kcontig, fp16, wide, s);
+  const int rc = launch_planned(a, a_kcontig, b_kcontig, fp16, wide, form, s);
+  return rc != ETH_OK ? rc : launch_planned(r, a_kcontig, b_kcontig, fp16, wide, form, s);
 }
 
 extern "C" int eth_gemm_plan(int64_t M, int64_t N, int64_t K, int a_kcontig, int b_kcontig, int64_t ldc, int c_dtype,
@@ -1278,13 +1298,13 @@ extern "C" int eth_gemm_plan(int64_t M, int64_t N, int64_t K, int a_kcontig, int
   ETH_CHECK_ARG(M > 0 && N > 0 && K > 0 && M < (1LL << 31) && N < (1LL << 31) && K < (1LL << 31) && ldc >= N,
                 "eth_gemm_plan: bad shape %lld x %lld x %lld", (long long)M, (long long)N, (long long)K);
   const bool wide = wide_takes(M, N, ldc, c_dtype == ETH_F32 ? 4 : 2, ldc % 4 == 0 && N % 4 == 0);
-  const bool skew = skewed(K, a_kcontig, b_kcontig);
-  const GemmCut cut = plan_cut(M, N, K, wide, skew);
-  plan[0] = plan_tile(cut.m, cut.n, K, wide, skew);
+  const GemmForm form = gemm_form(M, N, K, a_kcontig, b_kcontig, c_dtype == ETH_F32);
+  const GemmCut cut = plan_cut(M, N, K, wide, form);
+  plan[0] = plan_tile(cut.m, cut.n, K, wide, form);
   plan[1] = cut.m;
   plan[2] = cut.n;
   const int64_t m = cut.m < M ? M - cut.m : M, n = cut.n < N ? N - cut.n : N;
-  plan[3] = cut.m == M && cut.n == N ? 0 : plan_tile(m, n, K, wide, skew);
+  plan[3] = cut.m == M && cut.n == N ? 0 : plan_tile(m, n, K, wide, form);
   return ETH_OK;
 }
 
@@ -1350,13 +1370,14 @@ extern "C" int64_t eth_gemm_splitk_workspace(int64_t M, int64_t N, int splits) {
   return splits > 0 && M > 0 && N > 0 ? (int64_t)splits * M * N * 4 : 0;
 }
 
-extern "C" int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits, int a_kcontig, int b_kcontig) {
+extern "C" int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits, int a_kcontig, int b_kcontig,
+                                        int c_dtype) {
   if (M <= 0 || N <= 0 || K <= 0 || splits < 2) return 0;
-  // the second kernel: a launch, and the partials and C at about 4.5 TB/s
-  const double sum = 5.0 + 4.0 * (double)M * (double)N * (splits + 1) / 4.5e6;
-  const bool skew = skewed(K, a_kcontig, b_kcontig);
-  const double one = tile_time(plan_tile(M, N, K, true, skew), M, N, K, 1, skew);
-  return tile_time(256, M, N, K, splits, skew) + sum < one;
+  // the second kernel: a launch, and the partials (and an fp32 C) at 4.3 TB/s
+  const double sum = 4.5 + 4.0 * (double)M * (double)N * (splits + (c_dtype == ETH_F32 ? 1 : 0)) / 4.3e6;
+  const GemmForm form = gemm_form(M, N, K, a_kcontig, b_kcontig, c_dtype == ETH_F32);
+  const double one = tile_time(plan_tile(M, N, K, true, form), M, N, K, 1, form);
+  return tile_time(256, M, N, K, splits, form) + sum < one;
 }
 
 extern "C" int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, const void* B, int64_t ldb,

@@ -89,13 +89,13 @@ def _splitk_splits(M, N, K, out):
 
 
 @functools.lru_cache(maxsize=4096)
-def _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig):
+def _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig, out_code):
     """fp32 elements of workspace if the split-K form takes this product and
-    finishes before the plain one, else 0 (sizes and layout only; the smaller
+    finishes before the plain one, else 0 (by sizes, layout and type; the smaller
     tiles fill the chip without a second pass unless K is deep)."""
     if splits < 2 or K % 8 or 4 * (M + 256) * N >= 2**31:
         return 0
-    if not nat.value("eth_gemm_splitk_pays", M, N, K, splits, a_kcontig, b_kcontig):
+    if not nat.value("eth_gemm_splitk_pays", M, N, K, splits, a_kcontig, b_kcontig, out_code):
         return 0
     return nat.value("eth_gemm_splitk_workspace", M, N, splits) // 4
 
@@ -165,7 +165,8 @@ def gemm(a, b, out=None, bias=None, accumulate=False, out_dtype=None, alpha=1.0)
         flags |= nat.GEMM_BIAS
     _observe("gemm", "begin", 2.0 * M * N * K)
     splits = _splitk_splits(M, N, K, out)
-    partials = _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig)
+    out_code = nat.dtype_code(out.dtype)
+    partials = _splitk_pays(M, N, K, splits, a_kcontig, b_kcontig, out_code)
     if partials:
         # (a fresh buffer per call: two threads may share the stream)
         ws = torch.empty(partials, dtype=torch.float32, device=a.device)
@@ -173,7 +174,7 @@ def gemm(a, b, out=None, bias=None, accumulate=False, out_dtype=None, alpha=1.0)
             "eth_gemm_splitk_out",
             nat.ptr(a), lda, a_kcontig,
             nat.ptr(b), ldb, b_kcontig,
-            nat.ptr(out), out.stride(0), nat.dtype_code(out.dtype),
+            nat.ptr(out), out.stride(0), out_code,
             nat.ptr(bias), M, N, K, code, flags, float(alpha), splits, nat.ptr(ws),
             nat.stream_ptr(a.device),
         )
@@ -183,7 +184,7 @@ def gemm(a, b, out=None, bias=None, accumulate=False, out_dtype=None, alpha=1.0)
         "eth_gemm",
         nat.ptr(a), lda, a_kcontig,
         nat.ptr(b), ldb, b_kcontig,
-        nat.ptr(out), out.stride(0), nat.dtype_code(out.dtype),
+        nat.ptr(out), out.stride(0), out_code,
         nat.ptr(bias), M, N, K, code, flags, float(alpha),
         nat.stream_ptr(a.device),
     )

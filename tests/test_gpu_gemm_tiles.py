@@ -127,8 +127,9 @@ def test_short_k_tile_reads_nothing_past_k(cuda, a_k, b_k):
 
 
 @pytest.mark.parametrize("a_k,b_k,M,N,Kd,dtype,plan", [
-    # 300 wide tiles: 250 and a rest of rows
-    (False, False, 7680, 2552, 520, torch.bfloat16, (256, 6400, 2552, 128)),
+    # 300 wide tiles: 240 and a rest of columns, or of rows
+    (False, False, 7680, 2552, 520, torch.bfloat16, (256, 7680, 2048, 128)),
+    (False, False, 2552, 7680, 520, torch.bfloat16, (256, 2048, 7680, 128)),
     (True, True, 2304, 8192, 512, torch.float16, (256, 2048, 8192, 64)),
     (True, False, 8200, 2048, 512, torch.bfloat16, (256, 8192, 2048, 64)),  # eight rows past a whole round
     # 792: a last round of 24, deep enough for a smaller promise
@@ -203,11 +204,12 @@ def test_deep_product_takes_splits(cuda):
     announce(f"gemm deep {M}x{N}x{Kd}")
     out = torch.empty(M, N, dtype=torch.bfloat16, device=cuda)
     splits = K._splitk_splits(M, N, Kd, out)
-    assert splits == 16 and K._splitk_pays(M, N, Kd, splits, 1, 0) and K._splitk_pays(M, N, Kd + 8, splits, 1, 0)
-    assert not K._splitk_pays(M, N, Kd + 4, splits, 1, 0) and not K._splitk_pays(2048, 2048, 2048, 2, 1, 1)
+    pays = lambda *args: K._splitk_pays(*args, nat.ETH_BF16)  # noqa: E731
+    assert splits == 16 and pays(M, N, Kd, splits, 1, 0) and pays(M, N, Kd + 8, splits, 1, 0)
+    assert not pays(M, N, Kd + 4, splits, 1, 0) and not pays(2048, 2048, 2048, 2, 1, 1)
     # half a round of wide tiles splits in two, one tile more does not
     half = torch.empty(2048, 4096, dtype=torch.bfloat16, device=cuda)
-    assert K._splitk_splits(2048, 4096, 16384, half) == 2 and K._splitk_pays(2048, 4096, 16384, 2, 1, 1)
+    assert K._splitk_splits(2048, 4096, 16384, half) == 2 and pays(2048, 4096, 16384, 2, 1, 1)
     assert K._splitk_splits(2049, 4096, 16384, half) == 1
     a, b, ad, bd = _operands(M, N, Kd, True, False, torch.bfloat16, cuda, 5)
     got = K.gemm(ad, bd)

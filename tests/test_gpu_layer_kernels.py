@@ -147,7 +147,7 @@ def test_gemm_takes_splitk_for_deep_products(cuda, a_k, b_k):
     av, bv = ad if a_k else ad.t(), bd.t() if b_k else bd
     acc = torch.full((M, N), 0.25, dtype=torch.float32, device=cuda)
     splits = K._splitk_splits(M, N, Kd, acc)
-    assert splits > 1 and K._splitk_pays(M, N, Kd, splits, int(a_k), int(b_k)) == splits * M * N
+    assert splits > 1 and K._splitk_pays(M, N, Kd, splits, int(a_k), int(b_k), nat.ETH_F32) == splits * M * N
     K.gemm(av, bv, out=acc, accumulate=True)
     want = torch.full((M, N), 0.25, dtype=torch.float32, device=cuda)
     ws = torch.full((splits * M * N,), float("nan"), device=cuda)
