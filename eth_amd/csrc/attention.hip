@@ -733,13 +733,18 @@ __global__ void __launch_bounds__(2 * kAttnThreads, 1) attn_bwd_dkdv_x128_kernel
 }
 
 // ------------------------------------- backward: dK, dV, head dims to 96 --
-// dK and dV of 32 keys per wave in one wave: both accumulators, the K and V
-// fragments and one 32-query tile of S and dP fit 256 registers up to a head
-// dim of 96, so nothing is handed from wave to wave, a workgroup is four
-// independent waves with one barrier per 64 queries, and two workgroups share
-// a CU, one computing probabilities while the other's MFMAs run.  S = Q K^T
-// and dP = dO V^T are computed with lane = key (query rows swizzled), so P and
-// dS are already the A operands of dV += P^T dO and dK += dS^T Q.
+// dK and dV of 32 keys per wave in one wave, so nothing is handed from wave to
+// wave, a workgroup is four independent waves with one barrier per 64 queries,
+// and two workgroups share a CU, one computing probabilities while the other's
+// MFMAs run.  Both accumulators, the K and V fragments and one 32-query tile
+// of S and dP take 208 to 216 VGPRs at a head dim of 64.  At 96 they need more
+// than the 256 there are: 10 to 12 are spilled with one group of waves and 22
+// to 30 with two, whose reloads between the MFMAs of a step (vector-memory
+// loads complete in order) wait for the rows of the next step, so at 96 that
+// load is only partly hidden.  It still beats pairs of waves that hand P over
+// (backward of 1500 x 2 x 32 heads of 80: 175 us with them, 142 here).  S = Q
+// K^T and dP = dO V^T are computed with lane = key (query rows swizzled), so P
+// and dS are already the A operands of dV += P^T dO and dK += dS^T Q.
 //
 // The Q and dO rows of a step load directly into LDS a step ahead, one image
 // each, double buffered: chunk c (8 columns) of row r at c ^ img_swz(r), which
