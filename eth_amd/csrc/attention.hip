@@ -974,7 +974,8 @@ __global__ void __launch_bounds__(G * kAttnThreads, 2) attn_bwd_dkdv_kernel(Attn
 }
 
 // ------------------------------------------------------------ backward: dQ --
-// G = 2 as in the forward.
+// G = 2 as in the forward (at a head dim of 128 it spills 3 registers, all
+// outside the loop, and with PAD 8).
 template <int D, bool FP16, bool PAD, int G>
 __global__ void __launch_bounds__(G * kAttnThreads, 2) attn_bwd_dq_kernel(AttnArgs a) {
   constexpr int KS = D / 16, DT = D / 32;
