@@ -1079,7 +1079,8 @@ struct GemmForm {
   int skew_r;
 };
 static GemmForm gemm_form(int64_t M, int64_t N, int64_t K, int a_kcontig, int b_kcontig, bool f32) {
-  return GemmForm{f32, a_kcontig && b_kcontig && K % 64 != 0, (!a_kcontig && M % 64 != 0) + (!b_kcontig && N % 64 != 0)};
+  return GemmForm{f32, a_kcontig && b_kcontig && K % 64 != 0,
+                  (!a_kcontig && M % 64 != 0) + (!b_kcontig && N % 64 != 0)};
 }
 
 // Microseconds one launch of TILE x TILE tiles takes, fitted to sweeps (within

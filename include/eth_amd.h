@@ -267,7 +267,8 @@ int eth_gemm_splitk_out(const void* A, int64_t lda, int a_kcontig, const void* B
                         void* C, int64_t ldc, int c_dtype, const void* bias, int64_t M, int64_t N, int64_t K,
                         int in_dtype, int flags, float alpha, int splits, float* workspace, void* stream);
 /* 1 where the split-K form with `splits` is expected to finish before
- * eth_gemm on the same [M, N] x K product, else 0. */
+ * eth_gemm on the same [M, N] x K product of these layouts and output type,
+ * else 0. */
 int64_t eth_gemm_splitk_pays(int64_t M, int64_t N, int64_t K, int splits, int a_kcontig, int b_kcontig, int c_dtype);
 
 /* ------------------------------------------------------------------------

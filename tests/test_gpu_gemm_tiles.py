@@ -117,8 +117,9 @@ def test_short_k_tile_reads_nothing_past_k(cuda, a_k, b_k):
     M, N, Kd = 4088, 2040, 200
     announce(f"gemm wide views {M}x{N}x{Kd} a_k={a_k} b_k={b_k}")
     a, b, _, _ = _operands(M, N, Kd, a_k, b_k, torch.bfloat16, cuda, 3)
-    wide_a, wide_b = (torch.full((M, Kd + 56) if a_k else (Kd + 56, M), float("nan"), dtype=torch.bfloat16, device=cuda),
-                      torch.full((N, Kd + 56) if b_k else (Kd + 56, N), float("nan"), dtype=torch.bfloat16, device=cuda))
+    nan = lambda *shape: torch.full(shape, float("nan"), dtype=torch.bfloat16, device=cuda)  # noqa: E731
+    wide_a = nan(M, Kd + 56) if a_k else nan(Kd + 56, M)
+    wide_b = nan(N, Kd + 56) if b_k else nan(Kd + 56, N)
     ad = wide_a[:, :Kd] if a_k else wide_a[:Kd].t()
     bd = wide_b[:, :Kd].t() if b_k else wide_b[:Kd]
     ad.copy_(a)

@@ -55,12 +55,13 @@ def test_join_waits_only_for_new_side_work(cuda):
     assert K.side_mark() != mark
 
 
+@pytest.mark.parametrize("own_stream", [False, True])
 @pytest.mark.parametrize("tokens", [64, 4096])
-def test_node_of_another_stream_and_nested_contexts(cuda, tokens):
-    """One weight used by a product on the context's stream and one on
-    another stream that is behind; an inner context that launches nothing
-    leaves the wait to the outer one."""
-    announce(f"wgrad streams nested {tokens}")
+def test_node_of_another_stream_and_nested_contexts(cuda, tokens, own_stream):
+    """One weight used by a product on the context's stream (the default one
+    or its own) and one on another stream that is behind; an inner context
+    that launches nothing leaves the wait to the outer one."""
+    announce(f"wgrad streams nested {tokens} own={own_stream}")
     h = 2048
     gen = torch.Generator(device=cuda).manual_seed(tokens)
     xs = [torch.randn(tokens, h, device=cuda, generator=gen).bfloat16() for _ in range(2)]
@@ -70,24 +71,27 @@ def test_node_of_another_stream_and_nested_contexts(cuda, tokens):
         K.gemm(dy.t(), x, out=want, accumulate=True)
     w = torch.nn.Parameter(torch.randn(h, h, device=cuda, generator=gen).bfloat16())
     w.main_grad = torch.zeros(h, h, device=cuda)
+    home = torch.cuda.Stream() if own_stream else torch.cuda.current_stream()
     other = torch.cuda.Stream()
-    for order in (0, 1):
-        w.main_grad.fill_(7.0)
-        w._eth_main_grad_stale = True  # the first contribution stores
-        outs = [Fn.LinearFn.apply(xs[0], w, None)]
-        other.wait_stream(torch.cuda.current_stream())
-        with torch.cuda.stream(other):
-            outs.append(Fn.LinearFn.apply(xs[1], w, None))
-        torch.cuda.synchronize()
-        first, second = (0, 1) if order == 0 else (1, 0)
-        with Fn.overlapped_wgrad():
+    torch.cuda.synchronize()
+    for order in ((0, 1), (1, 0)):
+        with torch.cuda.stream(home):
+            w.main_grad.fill_(7.0)
+            w._eth_main_grad_stale = True  # the first contribution stores
+            outs = [Fn.LinearFn.apply(xs[0], w, None)]
+            other.wait_stream(home)
             with torch.cuda.stream(other):
-                torch.cuda._sleep(DELAY)
-            for i in (first, second):
-                torch.autograd.backward(outs[i], dys[i])
+                outs.append(Fn.LinearFn.apply(xs[1], w, None))
+            torch.cuda.synchronize()
             with Fn.overlapped_wgrad():
-                pass
-        got = w.main_grad.clone()
-        # (the two sums of one pair of products: fp32 addition commutes)
-        assert torch.equal(got, want)
+                # each of the two streams is behind when it is to be waited for
+                with torch.cuda.stream(other if order[0] else home):
+                    torch.cuda._sleep(DELAY)
+                for i in order:
+                    torch.autograd.backward(outs[i], dys[i])
+                with Fn.overlapped_wgrad():
+                    pass
+            got = w.main_grad.clone()
+            # (the two sums of one pair of products: fp32 addition commutes)
+            assert torch.equal(got, want)
         torch.cuda.synchronize()
